@@ -67,66 +67,90 @@ struct StepParams {
 
 constexpr int kScanChunk = 8 * kBlock;  // tiles per block in the two-level tile scan
 
-// Membership of `target` in a group's edge list (known_to_known/const test,
-// core/engine.hpp:179-184,211-216). SORTED lists use an 8-lane 9-ary search:
-// each lane reads one pivot, a ballot counts the pivots below the target and
-// the range shrinks ~9x per round; the last <= 8 entries are compared at once.
-// Unsorted lists are scanned 8 entries at a time with early exit, like the
-// reference's linear scan. Both report the reference's work count: index of
-// the first match + 1, or the degree when absent.
-template <bool SORTED, bool FRAMED>
-__device__ __forceinline__ void group_member(const GraphView &g, uint64_t estart, uint64_t efb, uint32_t off,
-                                             uint32_t deg, uint32_t target, bool valid, bool &found,
-                                             uint32_t &examined) {
+// Membership of `target` in an 8-lane group's edge list (known_to_known/const
+// test, core/engine.hpp:179-184,211-216), for lists that need not be sorted:
+// 8 entries at a time with early exit, like the reference's linear scan. The
+// work count is the reference's: index of the first match + 1, or the
+// degree when absent.
+template <bool FRAMED>
+__device__ __forceinline__ void group_scan(const GraphView &g, uint64_t estart, uint64_t efb, uint32_t off,
+                                           uint32_t deg, uint32_t target, bool valid, bool &found,
+                                           uint32_t &examined) {
   const uint32_t lane = lane_id(), l8 = lane & 7, gbase = lane & ~7u;
-  bool act = valid && deg > 0;
+  const bool act = valid && deg > 0;
   found = false;
-  uint32_t idx = 0;
-  if (SORTED) {
-    uint32_t lo = 0, hi = deg;
-    while (true) {
-      const bool need = act && (hi - lo > 8);
-      if (!wave_ballot(need)) break;
-      bool lt = false;
-      const uint32_t span = hi - lo;
-      if (need) {
-        const uint32_t pos = lo + (uint32_t)(((uint64_t)span * (l8 + 1)) / 9);
-        lt = edge_at<FRAMED>(g, estart, efb, (uint64_t)off + pos) < target;
-      }
-      const uint32_t m = __builtin_popcount((uint32_t)(wave_ballot(need && lt) >> gbase) & 0xffu);
-      if (need) {
-        const uint32_t nlo = m == 0 ? lo : lo + (uint32_t)(((uint64_t)span * m) / 9) + 1;
-        const uint32_t nhi = m == 8 ? hi : lo + (uint32_t)(((uint64_t)span * (m + 1)) / 9) + 1;
-        lo = nlo;
-        hi = nhi;
-      }
-    }
+  uint32_t idx = 0, j = 0;
+  while (true) {
+    const bool go = act && !found && j < deg;
+    if (!wave_ballot(go)) break;
     bool eq = false;
-    if (act && l8 < hi - lo) eq = edge_at<FRAMED>(g, estart, efb, (uint64_t)off + lo + l8) == target;
+    if (go && j + l8 < deg) eq = edge_at<FRAMED>(g, estart, efb, (uint64_t)off + j + l8) == target;
     const uint32_t gb = (uint32_t)(wave_ballot(eq) >> gbase) & 0xffu;
-    if (act && gb) {
-      found = true;
-      idx = lo + (uint32_t)__builtin_ctz(gb);
-    }
-  } else {
-    uint32_t j = 0;
-    while (true) {
-      const bool go = act && !found && j < deg;
-      if (!wave_ballot(go)) break;
-      bool eq = false;
-      if (go && j + l8 < deg) eq = edge_at<FRAMED>(g, estart, efb, (uint64_t)off + j + l8) == target;
-      const uint32_t gb = (uint32_t)(wave_ballot(eq) >> gbase) & 0xffu;
-      if (go) {
-        if (gb) {
-          found = true;
-          idx = j + (uint32_t)__builtin_ctz(gb);
-        } else {
-          j += 8;
-        }
+    if (go) {
+      if (gb) {
+        found = true;
+        idx = j + (uint32_t)__builtin_ctz(gb);
+      } else {
+        j += 8;
       }
     }
   }
   examined = found ? idx + 1 : deg;
+}
+
+// Membership of every lane's own target in its own edge list (one row per
+// lane; the whole wave calls it): found and the reference's work count.
+// Sorted lists: each lane searches by itself, three pivots loaded together
+// per round, so a round quarters the range and the last <= 4 entries are
+// compared at once. What bounds it is the chain of dependent loads, and a
+// wave has 64 of them in flight; an 8-lane 9-ary search,
+// which this replaced, ran a group's 8 rows one after another (8
+// chains in flight, 8 times as long): a known_to_known step over
+// 3M rows, half of them walked edges, 401 -> 210 us; known_to_const over 12M
+// rows of one-entry lists 443 -> 370 us.
+// Unsorted lists: the 8 lanes of a group scan the group's 8 lists in turn.
+template <bool SORTED, bool FRAMED>
+__device__ __forceinline__ void rows_member(const GraphView &g, uint64_t estart, uint64_t efb, uint32_t off,
+                                            uint32_t deg, uint32_t target, bool valid, bool &found,
+                                            uint32_t &examined) {
+  found = false;
+  examined = deg;
+  if constexpr (SORTED) {
+    if (valid && deg) {
+      uint32_t lo = 0, hi = deg - 1;  // the first match, if any, is in [lo, hi]
+      while (hi - lo > 3) {
+        const uint32_t q = (hi - lo) >> 2, p1 = lo + q, p2 = p1 + q, p3 = p2 + q;
+        const uint32_t v1 = edge_at<FRAMED>(g, estart, efb, (uint64_t)off + p1);
+        const uint32_t v2 = edge_at<FRAMED>(g, estart, efb, (uint64_t)off + p2);
+        const uint32_t v3 = edge_at<FRAMED>(g, estart, efb, (uint64_t)off + p3);
+        lo = v3 < target ? p3 + 1 : v2 < target ? p2 + 1 : v1 < target ? p1 + 1 : lo;
+        hi = v3 < target ? hi : v2 < target ? p3 : v1 < target ? p2 : p1;
+      }
+      uint32_t v[4];
+#pragma unroll
+      for (int k = 0; k < 4; k++) v[k] = lo + k <= hi ? edge_at<FRAMED>(g, estart, efb, (uint64_t)off + lo + k) : ~target;
+#pragma unroll
+      for (int k = 3; k >= 0; k--)
+        if (v[k] == target) {
+          found = true;
+          examined = lo + k + 1;
+        }
+    }
+  } else {
+    const uint32_t lane = lane_id(), gbase = lane & ~7u, l8 = lane & 7;
+#pragma unroll 1
+    for (uint32_t u = 0; u < 8; u++) {
+      const uint32_t src = gbase + u;
+      bool f;
+      uint32_t x;
+      group_scan<FRAMED>(g, estart, efb, shfl32(off, src), shfl32(deg, src), shfl32(target, src),
+                         shfl32(valid ? 1u : 0u, src) != 0, f, x);
+      if (l8 == u) {
+        found = f;
+        examined = x;
+      }
+    }
+  }
 }
 
 // Probe pass over one tile (TR rows; `lt` is the tile's index within its
@@ -143,7 +167,7 @@ __device__ __forceinline__ void probe_tile(const GraphView &g, const StepParams 
   __shared__ uint64_t s_tmp[kBlock / kWave];
   __shared__ uint32_t s_probed[kBlock / kWave];
   __shared__ WaveProbeLds s_wp[kBlock / kWave];
-  const uint32_t tid = threadIdx.x, lane = lane_id(), gbase = lane & ~7u, l8 = lane & 7;
+  const uint32_t tid = threadIdx.x, lane = lane_id();
   const uint32_t wave = tid / kWave;
   const uint64_t base = lt * TR;
   const DevMeta m = g.meta[p.pid < g.num_metas ? p.pid : 0];
@@ -176,28 +200,12 @@ __device__ __forceinline__ void probe_tile(const GraphView &g, const StepParams 
       s_cnt[local] = deg;
       s_aux[local] = off;
     } else {
-      // the 8 lanes of a group test the group's 8 rows one after another
-      uint32_t my_found = 0, my_ex = 0;
-#pragma unroll
-      for (int u = 0; u < 8; u++) {
-        const uint32_t src = gbase + u;
-        const uint32_t du = shfl32(deg, src), ou = shfl32(off, src);
-        uint32_t target = p.target;
-        bool valid = p.target_ok != 0;
-        if (p.mode == kModeK2K) {
-          const int32_t ec = (int32_t)shfl32((uint32_t)end_cell, src);
-          target = (uint32_t)ec;
-          valid = ec >= 0;
-        }
-        bool found;
-        uint32_t examined;
-        group_member<SORTED, FRAMED>(g, m.edge_start, m.eframe_base, ou, du, target, valid, found, examined);
-        if (l8 == (uint32_t)u) {
-          my_found = found ? 1u : 0u;
-          my_ex = examined;
-        }
-      }
-      s_cnt[local] = my_found;
+      const bool k2k = p.mode == kModeK2K;
+      bool my_found;
+      uint32_t my_ex;
+      rows_member<SORTED, FRAMED>(g, m.edge_start, m.eframe_base, off, deg, k2k ? (uint32_t)end_cell : p.target,
+                                  k2k ? end_cell >= 0 : p.target_ok != 0, my_found, my_ex);
+      s_cnt[local] = my_found ? 1u : 0u;
       s_aux[local] = my_ex;
     }
   }
@@ -624,7 +632,7 @@ __global__ __launch_bounds__(kBlock) void k_small_step(GraphView g, StepParams p
 //    its list into the table;
 //  - a known-start step: wave w probes rows [64 w r, 64 (w + 1) r) of the
 //    input (r = rounds of 64 rows, at most 4), filters test membership with
-//    the 8-lane group test, then a workgroup scan of the degrees (kept
+//    the probe pass's search, then a workgroup scan of the degrees (kept
 //    flags) gives every row its first output row; known_to_unknown writes
 //    output row k = (the last row whose first output row is <= k, its list
 //    entry k - that first row), filters copy the kept rows in order. Output
@@ -689,7 +697,7 @@ __device__ __forceinline__ uint64_t sq_uniform(uint64_t v) {
 template <bool SORTED, bool FRAMED>
 __device__ __forceinline__ void sq_run(const GraphView &g, SQShared &sh, int32_t *dst, uint64_t (&res)[5]) {
   const SmallQuery &q = sh.q;
-  const uint32_t tid = threadIdx.x, lane = lane_id(), wave = tid / kWave, l8 = lane & 7, gbase = lane & ~7u;
+  const uint32_t tid = threadIdx.x, lane = lane_id(), wave = tid / kWave;
   uint64_t expanded = 0, status = 0;
   uint32_t rows = 0, cols = 0, cur = 0, l = 0;
   const uint32_t nsteps = sq_uniform((uint32_t)q.nsteps);
@@ -776,28 +784,12 @@ __device__ __forceinline__ void sq_run(const GraphView &g, SQShared &sh, int32_t
             sh.off[row] = off;
           }
         } else {
-          // the 8 lanes of a group test the group's 8 rows one after another
-          uint32_t my_found = 0, my_ex = 0;
-#pragma unroll 1
-          for (int u = 0; u < 8; u++) {
-            const uint32_t src = gbase + u;
-            const uint32_t du = shfl32(deg, src), ou = shfl32(off, src);
-            uint32_t target = (uint32_t)d.vid;
-            bool valid = target_ok;
-            if (mode == kModeK2K) {
-              const int32_t e = (int32_t)shfl32((uint32_t)end_cell, src);
-              target = (uint32_t)e;
-              valid = e >= 0;
-            }
-            bool found;
-            uint32_t examined;
-            group_member<SORTED, FRAMED>(g, m.edge_start, m.eframe_base, ou, du, target, valid, found, examined);
-            if (l8 == (uint32_t)u) {
-              my_found = found ? 1u : 0u;
-              my_ex = examined;
-            }
-          }
-          if (row < rows) sh.deg[row] = my_found;
+          bool my_found;
+          uint32_t my_ex;
+          rows_member<SORTED, FRAMED>(g, m.edge_start, m.eframe_base, off, deg,
+                                      mode == kModeK2K ? (uint32_t)end_cell : (uint32_t)d.vid,
+                                      mode == kModeK2K ? end_cell >= 0 : target_ok, my_found, my_ex);
+          if (row < rows) sh.deg[row] = my_found ? 1u : 0u;
           ex += my_ex;
         }
       }
@@ -1281,7 +1273,7 @@ __global__ __launch_bounds__(kBlock) void k_key_degrees(GraphView g, uint32_t pi
 // entry, D entry and target; a list of at most kLaneList entries is scanned
 // by the row's own lane (the reference's early-exit scan, so its work count
 // is the scan's: first match + 1, or the degree). Longer lists go through
-// the probe pass's 8-lane membership test in a second phase, which a block
+// the probe pass's membership test in a second phase, which a block
 // skips when it has none. Kept flags become the tile's bit words; the tile's
 // sums are kept rows and edges examined.
 template <int TR, bool SORTED>
@@ -1294,7 +1286,7 @@ __global__ __launch_bounds__(kBlock) void k_fanout_filter(GraphView g, StepParam
   __shared__ uint64_t s_m[2];
   __shared__ uint32_t s_any;
   const uint64_t lt = p.tile0 + blockIdx.x;
-  const uint32_t tid = threadIdx.x, lane = lane_id(), gbase = lane & ~7u, l8 = lane & 7;
+  const uint32_t tid = threadIdx.x, lane = lane_id();
   const uint64_t base = lt * TR;
   const DevMeta m = g.meta[p.pid < g.num_metas ? p.pid : 0];
   if (tid == 0) {  // the parents this tile's rows lie in: [i0, i1]
@@ -1365,7 +1357,7 @@ __global__ __launch_bounds__(kBlock) void k_fanout_filter(GraphView g, StepParam
     if (big_any) s_any = 1;
   }
   __syncthreads();
-  if (s_any) {  // long lists: the 8-lane membership test, 64 rows per wave per round
+  if (s_any) {  // long lists: the membership test of the probe pass, 64 rows per wave per round
     constexpr uint32_t kWaveRows = TR / (kBlock / kWave);
     const uint32_t wave = tid / kWave;
     for (int rd = 0; rd < TR / kBlock; rd++) {
@@ -1373,18 +1365,12 @@ __global__ __launch_bounds__(kBlock) void k_fanout_filter(GraphView g, StepParam
       const bool big = s_big[local] != 0;
       const uint32_t off = big ? s_off[local] : 0u, deg = big ? s_deg[local] : 0u, tgt = big ? s_tgt[local] : 0u;
       if (!wave_ballot(big)) continue;
-#pragma unroll
-      for (int u = 0; u < 8; u++) {
-        const uint32_t src = gbase + u;
-        const uint32_t du = shfl32(deg, src), ou = shfl32(off, src), tu = shfl32(tgt, src);
-        const bool bu = shfl32(big ? 1u : 0u, src) != 0;
-        bool found;
-        uint32_t examined;
-        group_member<SORTED, false>(g, m.edge_start, m.eframe_base, ou, du, tu, bu, found, examined);
-        if (l8 == (uint32_t)u && big) {
-          s_keep[local] = found ? 1 : 0;
-          ex += examined;
-        }
+      bool found;
+      uint32_t examined;
+      rows_member<SORTED, false>(g, m.edge_start, m.eframe_base, off, deg, tgt, big, found, examined);
+      if (big) {
+        s_keep[local] = found ? 1 : 0;
+        ex += examined;
       }
     }
   }
@@ -1432,7 +1418,7 @@ __global__ __launch_bounds__(kBlock) void k_fanout_units(GraphView g, StepParams
   __shared__ uint8_t s_bigb[kBlock];         // per thread: which of its rows have long lists
   __shared__ __align__(4) uint8_t s_kb[kBlock];  // per thread: its rows' kept bits
   __shared__ uint32_t s_any;
-  const uint32_t tid = threadIdx.x, lane = lane_id(), gbase = lane & ~7u, l8 = lane & 7;
+  const uint32_t tid = threadIdx.x, lane = lane_id();
   const uint64_t e = p.tile0 + blockIdx.x;
   // the unit: list L, j-block, parent
   uint64_t L = 0, hi = u.nl - 1;
@@ -1497,7 +1483,7 @@ __global__ __launch_bounds__(kBlock) void k_fanout_units(GraphView g, StepParams
   s_bigb[tid] = (uint8_t)bigb;
   if (bigb) s_any = 1;
   __syncthreads();
-  if (s_any) {  // long lists: the 8-lane membership test, 64 rows per wave per round
+  if (s_any) {  // long lists: the membership test of the probe pass, 64 rows per wave per round
     constexpr uint32_t kWaveRows = TR / (kBlock / kWave);
     const uint32_t wave = tid / kWave;
     for (int rd = 0; rd < TR / kBlock; rd++) {
@@ -1505,18 +1491,12 @@ __global__ __launch_bounds__(kBlock) void k_fanout_units(GraphView g, StepParams
       const bool big = (s_bigb[local / RPT] >> (local % RPT)) & 1u;
       const uint32_t off = big ? s_off[local] : 0u, deg = big ? s_deg[local] : 0u;
       if (!wave_ballot(big)) continue;
-#pragma unroll
-      for (int q = 0; q < 8; q++) {
-        const uint32_t src = gbase + q;
-        const uint32_t du = shfl32(deg, src), ou = shfl32(off, src);
-        const bool bu = shfl32(big ? 1u : 0u, src) != 0;
-        bool found;
-        uint32_t examined;
-        group_member<SORTED, false>(g, m.edge_start, m.eframe_base, ou, du, tgt, bu, found, examined);
-        if (l8 == (uint32_t)q && big) {
-          s_keep[local] = found ? 1 : 0;
-          ex += examined;
-        }
+      bool found;
+      uint32_t examined;
+      rows_member<SORTED, false>(g, m.edge_start, m.eframe_base, off, deg, tgt, big, found, examined);
+      if (big) {
+        s_keep[local] = found ? 1 : 0;
+        ex += examined;
       }
     }
     __syncthreads();
