@@ -163,7 +163,7 @@ int wkg_table_wrap_device(wkg_ctx *ctx, const int32_t *cells, uint64_t rows, int
  * produced and consumed in chunks of at most this size. */
 int wkg_set_table_limit(wkg_ctx *ctx, uint64_t max_table_bytes);
 /* Rows per probe tile of the per-step calls: 256, 512, 1024 or 2048, or 0
- * (the default) to choose by input size (the largest tile that leaves at
+ * (the default) to choose by input size (512 when that leaves at
  * least four tiles per compute unit). A tuning knob with no counterpart in
  * the reference; results do not depend on it. */
 int wkg_set_probe_tile_rows(wkg_ctx *ctx, int rows);

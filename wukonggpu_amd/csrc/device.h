@@ -65,7 +65,23 @@ struct GraphView {
   const uint64_t *eframes;  // framed: physical first edge of each logical frame
   uint32_t vshift, eshift;  // log2 of buckets / edges per frame
   uint32_t num_metas;
+  const uint2 *tags;  // resident: a tag word per main bucket, or null
 };
+
+// Tag words, one per main bucket: byte i < 7 is the tag of the key in slot i
+// (0: empty slot), and each key in the bucket's chain sets one of the eight
+// bits of byte 7. A probe that finds its key's tag reads that one slot; one
+// that finds neither tag nor chain bit knows the key is absent and reads no
+// bucket (at the builder's load, about 5.25 keys per bucket, one absent key
+// in twenty still does). The words are a sixteenth of the buckets, so a
+// predicate's stay in the L2s where its buckets do not.
+__host__ __device__ __forceinline__ uint32_t key_tag(uint64_t hash) {  // 1..255
+  const uint32_t t = (uint32_t)(hash >> 56);
+  return t ? t : 1u;
+}
+__host__ __device__ __forceinline__ uint32_t key_chain_bit(uint64_t hash) {  // of the word's high half
+  return 1u << (24 + (uint32_t)((hash >> 53) & 7));
+}
 
 __device__ __forceinline__ uint32_t lane_id() {
   return __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
@@ -115,28 +131,40 @@ struct WaveProbeLds {
 
 // Cluster-chaining probe of 64 consecutive rows, one per lane, all under one
 // predicate (get_vertex_local, core/gstore.hpp:389-409; device form
-// core/gpu_hash.cu:181-234).
-//  0. The caller's carry holds the key of the row just before lane 0 (the
-//     previous call's lane 63) and its result: a run of equal keys that
-//     continues from the previous call is not probed again.
-//  1. A run of equal keys in consecutive lanes is probed once: its first lane
-//     (the run leader) hashes the key and parks (key, bucket, its rank among
-//     the leaders) in LDS as a pending walk.
-//  2. Pending walks are taken 8 lanes per walk: group g takes walks g, g+8,
-//     g+16, ...; each lane of the group loads one 16-byte slot of the bucket
-//     (one coalesced 128-byte read; a group's walks are loaded together, so
-//     up to 8 bucket reads are in flight per lane). The lane whose slot
-//     holds the key writes the leader's (degree, offset) to LDS; in a group
-//     with no match, lane 7 (the link slot) either records a miss or appends
-//     the walk, moved to the linked bucket, to the next hop's pending list.
-//     The next hop only walks what is still pending, compacted.
-//  3. Every lane reads its run leader's result.
+// core/gpu_hash.cu:181-234), in three parts. A caller with several rounds of
+// 64 rows plans and picks the next rounds before it finishes this one, so
+// the loads of each part have arrived when the next part wants them.
+// probe_plan: a run of equal keys in consecutive lanes is probed once, by its
+//  first lane (the run leader); `before63` is the key of the row just before
+//  lane 0 (the previous round's lane 63), whose run continues here without a
+//  probe. A leader hashes its key to its main bucket and (TAGS) loads the
+//  bucket's tag word.
+// probe_pick (TAGS): a leader whose tag is in the word loads that slot; one
+//  with only a chain bit will walk; the others' keys are absent.
+// probe_finish: a leader whose slot holds its key is done. Those that must
+//  walk (without tags: every leader; with them: keys in chains and tag
+//  collisions, about one in fifteen) park (key, bucket, lane) in LDS as
+//  pending walks, taken 8 lanes per walk: each lane of a group loads one
+//  16-byte slot of the bucket (one coalesced 128-byte read, up to 8 bucket
+//  reads in flight per lane). The lane whose slot holds the key writes the
+//  leader's (degree, offset) to LDS; in a group with no match, lane 7 (the
+//  link slot) either records a miss or appends the walk, moved to the linked
+//  bucket, to the next hop's pending list. At last every lane takes its run
+//  leader's result.
 // Buckets are addressed with 32 bits (images hold fewer than 2^32 buckets).
-// Every lane of the wave must call this with the wave's own `w`. key == 0
-// means "no key". Gives the lane's degree (0 on a miss) and list offset
-// relative to the predicate's edge_start, moves the carry to lane 63 (it
-// starts as key 0: valid keys are never 0) and returns the number of keys
-// the wave probed (its run leaders).
+// Every lane of the wave must call these with the wave's own `w`. key == 0
+// means "no key". They give the lane's degree (0 on a miss) and list offset
+// relative to the predicate's edge_start, move the carry to lane 63 (it
+// starts as key 0: valid keys are never 0) and return the number of distinct
+// runs (the leaders).
+// What bounds a large probe is cache misses: the L2s miss at 55-63 G lines/s
+// whatever is read from a line (4 B or 128 B), and serve 264 G hits/s. Read
+// through the buckets, every key misses, present or not. 24M random keys, 36%
+// of them present: 512 us through the buckets (47 G keys/s), 300 us through
+// the tags (80 G keys/s); the executor's 512-query mix, mostly absent keys,
+// 730 -> 661 us a batch. Nontemporal slot reads leave the tag words their
+// place in the L2s (16.4M -> 13.2M misses) but measured slower (604 against
+// 517 us a step), as did nontemporal table reads and hit lists.
 struct ProbeCarry {
   uint64_t key = 0;
   uint32_t deg = 0, off = 0;
@@ -165,6 +193,11 @@ __device__ __forceinline__ uint4 gload(const uint4 *p) {
   const gu32x4 v = *(const WKG_GLOBAL gu32x4 *)p;
   return make_uint4(v.x, v.y, v.z, v.w);
 }
+// A read that is not kept in the caches ahead of others (nontemporal).
+__device__ __forceinline__ uint4 gload_once(const uint4 *p) {
+  const gu32x4 v = __builtin_nontemporal_load((const WKG_GLOBAL gu32x4 *)p);
+  return make_uint4(v.x, v.y, v.z, v.w);
+}
 __device__ __forceinline__ void gstore(uint2 *p, uint2 v) { *(WKG_GLOBAL gu32x2 *)p = gu32x2{v.x, v.y}; }
 __device__ __forceinline__ void gstore(uint4 *p, uint4 v) { *(WKG_GLOBAL gu32x4 *)p = gu32x4{v.x, v.y, v.z, v.w}; }
 
@@ -174,90 +207,164 @@ __device__ __forceinline__ uint64_t lanes_below() {
   return lane ? (~0ull >> (64 - lane)) : 0ull;
 }
 
-template <bool FRAMED>
-__device__ __forceinline__ uint32_t wave_probe(const GraphView &g, const DevMeta &m, uint64_t key, WaveProbeLds &w,
-                                               uint32_t &deg_out, uint32_t &off_out, ProbeCarry &carry) {
+struct ProbePlan {
+  uint64_t key;       // 0: none
+  uint64_t leaders;   // run leaders (wave-uniform)
+  uint32_t bucket;    // leaders: main bucket
+  uint32_t tag, cbit; // leaders: the key's tag in every byte, its chain bit
+  uint2 word;         // leaders: the bucket's tag word
+  uint4 slot;         // after probe_pick: the picked slot (key 0: none)
+  bool walk;          // after probe_pick: the buckets must be walked
+};
+
+template <bool FRAMED, bool TAGS>
+__device__ __forceinline__ ProbePlan probe_plan(const GraphView &g, const DevMeta &m, uint64_t key, uint64_t before63) {
+  static_assert(!(FRAMED && TAGS), "framed graphs have no tags");
+  ProbePlan r;
+  r.key = m.psz != 0 ? key : 0;
+  const uint64_t before = wave_shr1_64(r.key);
+  const bool lead = r.key != 0 && r.key != (lane_id() == 0 ? before63 : before);
+  r.leaders = wave_ballot(lead);
+  r.bucket = r.tag = r.cbit = 0;
+  r.word = make_uint2(0, 0);
+  r.slot = make_uint4(0, 0, 0, 0);
+  r.walk = lead;
+  if (lead) {
+    const uint64_t hash = mix64(key), local = fastmod(hash, m.psz, m.magic);
+    r.bucket = (uint32_t)(FRAMED ? bucket_phys<true>(g, m, local) : m.main_start + local);
+    if constexpr (TAGS) {
+      r.tag = key_tag(hash) * 0x01010101u;
+      r.cbit = key_chain_bit(hash);
+      if (g.tags) r.word = g.tags[r.bucket];
+    }
+  }
+  return r;
+}
+
+template <bool TAGS>
+__device__ __forceinline__ void probe_pick(const GraphView &g, ProbePlan &r) {
+  if constexpr (TAGS) {
+    if (!g.tags) return;  // (no tags: every leader walks)
+    const bool lead = (r.leaders >> lane_id()) & 1;
+    // bytes equal to the tag (exact for the lowest, which is the one taken)
+    const uint32_t vx = r.word.x ^ r.tag, vy = r.word.y ^ r.tag;
+    const uint32_t cx = (vx - 0x01010101u) & ~vx & 0x80808080u, cy = (vy - 0x01010101u) & ~vy & 0x00808080u;
+    const bool hit = lead && (cx | cy) != 0;
+    r.walk = lead && !hit && (r.word.y & r.cbit) != 0;
+    if (hit) {
+      const uint32_t i = cx ? (uint32_t)__builtin_ctz(cx) >> 3 : 4 + ((uint32_t)__builtin_ctz(cy) >> 3);
+      r.slot = g.slots[(uint64_t)r.bucket * kAssoc + i];
+    }
+    r.tag = hit ? 1u : 0u;
+  }
+}
+
+template <bool FRAMED, bool TAGS>
+__device__ __forceinline__ uint32_t probe_finish(const GraphView &g, const DevMeta &m, const ProbePlan &pl,
+                                                 WaveProbeLds &w, uint32_t &deg_out, uint32_t &off_out,
+                                                 ProbeCarry &carry) {
+  constexpr int U = TAGS ? 2 : 8;  // bucket reads in flight per lane
   const uint32_t lane = lane_id(), l8 = lane & 7, grp = lane >> 3, gbase = lane & ~7u;
-  const bool valid = key != 0 && m.psz != 0;
-  const uint64_t before = wave_shr1_64(key);
-  const uint64_t prev = lane == 0 ? carry.key : before;
-  const bool lead = valid && key != prev;
-  const uint64_t leaders = wave_ballot(lead);
-  const uint32_t L = (uint32_t)__builtin_popcountll(leaders);
-  if (L == 0) {  // every valid lane continues the carried run (wave-uniform)
+  const bool valid = pl.key != 0;
+  const uint64_t leaders = pl.leaders;
+  if (leaders == 0) {  // every valid lane continues the carried run (wave-uniform)
     deg_out = valid ? carry.deg : 0u;
     off_out = valid ? carry.off : 0u;
-    if (lane63_64(key) != carry.key) carry = ProbeCarry{};  // lane 63 has no key
+    if (lane63_64(pl.key) != carry.key) carry = ProbeCarry{};  // lane 63 has no key
     return 0;
   }
   const uint64_t below = lanes_below();
-  if (lead) {
-    const uint32_t j = (uint32_t)__builtin_popcountll(leaders & below);
-    const uint64_t local = fastmod(mix64(key), m.psz, m.magic);
-    const uint64_t b = FRAMED ? bucket_phys<true>(g, m, local) : m.main_start + local;
-    w.kb[j] = make_uint4((uint32_t)key, (uint32_t)(key >> 32), (uint32_t)b, j);
+  const uint32_t klo = (uint32_t)pl.key, khi = (uint32_t)(pl.key >> 32);
+  uint32_t deg = 0, off = 0;
+  bool walk = pl.walk;
+  if constexpr (TAGS) {
+    if (g.tags && pl.tag) {
+      if (pl.slot.x == klo && pl.slot.y == khi) {
+        const uint64_t v = ((uint64_t)pl.slot.w << 32) | pl.slot.z;
+        deg = (uint32_t)ptr_size(v);
+        off = (uint32_t)(ptr_off(v) - m.edge_start);
+      } else {
+        walk = true;  // another key with this tag
+      }
+    }
   }
-  __builtin_amdgcn_wave_barrier();
-  uint32_t n = L;  // pending walks (wave-uniform)
-  for (uint32_t hop = 0; n; hop++) {
-    const uint32_t umax = (n + 7) >> 3;
-    uint4 e[8], sl[8];
-#pragma unroll
-    for (int u = 0; u < 8; u++) {
-      e[u] = make_uint4(0, 0, 0, 0);
-      sl[u] = make_uint4(0, 0, 0, 0);
-      if ((uint32_t)u < umax && grp + 8u * u < n) {
-        e[u] = w.kb[grp + 8u * u];
-        sl[u] = g.slots[(uint64_t)e[u].z * kAssoc + l8];
-      }
-    }
-    // (every pending entry is read above before any is rewritten below: a
-    // wave's LDS operations complete in order)
-    uint32_t nn = 0;
-#pragma unroll
-    for (int u = 0; u < 8; u++) {
-      if ((uint32_t)u >= umax) break;  // wave-uniform
-      const bool in = grp + 8u * u < n;
-      const bool hit = in && l8 < 7 && sl[u].x == e[u].x && sl[u].y == e[u].y;
-      if (hit) {
-        const uint64_t v = ((uint64_t)sl[u].w << 32) | sl[u].z;
-        w.res[e[u].w] = make_uint2((uint32_t)ptr_size(v), (uint32_t)(ptr_off(v) - m.edge_start));
-      }
-      const uint32_t gb = (uint32_t)(wave_ballot(hit) >> gbase) & 0x7fu;
-      const uint64_t link = ((uint64_t)sl[u].y << 32) | sl[u].x;
-      const bool tail = in && l8 == 7 && gb == 0;  // lane 7 of a group without a match
-      const bool follow = tail && link != 0 && hop + 1 < kMaxHops;
-      if (tail && !follow) w.res[e[u].w] = make_uint2(0u, 0u);
-      const uint64_t fb = wave_ballot(follow);
-      if (follow) {
-        const uint64_t nb = key_vid(link);
-        const uint64_t bkt = FRAMED ? bucket_phys<true>(g, m, nb - m.indrct_start + m.psz) : nb;
-        w.kb[nn + (uint32_t)__builtin_popcountll(fb & below)] = make_uint4(e[u].x, e[u].y, (uint32_t)bkt, e[u].w);
-      }
-      nn += (uint32_t)__builtin_popcountll(fb);
-    }
+  const uint64_t walkers = wave_ballot(walk);
+  if (walkers) {
+    if (walk) w.kb[__builtin_popcountll(walkers & below)] = make_uint4(klo, khi, pl.bucket, lane);
     __builtin_amdgcn_wave_barrier();
-    n = nn;
-  }
-  deg_out = 0;
-  off_out = 0;
-  if (valid) {
-    // leaders at or below this lane; none: the lane continues the carried run
-    const uint32_t nl = (uint32_t)__builtin_popcountll(leaders & (below | (1ull << lane)));
-    if (nl) {
-      const uint2 r = w.res[nl - 1];
-      deg_out = r.x;
-      off_out = r.y;
-    } else {
-      deg_out = carry.deg;
-      off_out = carry.off;
+    uint32_t n = (uint32_t)__builtin_popcountll(walkers);  // pending walks (wave-uniform)
+    for (uint32_t hop = 0; n; hop++) {
+      uint32_t nn = 0;
+      for (uint32_t k0 = 0; k0 < n; k0 += 8 * U) {
+        uint4 e[U], sl[U];
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+          e[u] = make_uint4(0, 0, 0, 0);
+          sl[u] = make_uint4(0, 0, 0, 0);
+          if (k0 + grp + 8u * u < n) {
+            e[u] = w.kb[k0 + grp + 8u * u];
+            sl[u] = g.slots[(uint64_t)e[u].z * kAssoc + l8];
+          }
+        }
+        // (these pending entries are read above before any is rewritten
+        // below -- at most as many are appended as were read, and a wave's
+        // LDS operations complete in order)
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+          if (k0 + 8u * u >= n) break;  // wave-uniform
+          const bool in = k0 + grp + 8u * u < n;
+          const bool hit = in && l8 < 7 && sl[u].x == e[u].x && sl[u].y == e[u].y;
+          if (hit) {
+            const uint64_t v = ((uint64_t)sl[u].w << 32) | sl[u].z;
+            w.res[e[u].w] = make_uint2((uint32_t)ptr_size(v), (uint32_t)(ptr_off(v) - m.edge_start));
+          }
+          const uint32_t gb = (uint32_t)(wave_ballot(hit) >> gbase) & 0x7fu;
+          const uint64_t link = ((uint64_t)sl[u].y << 32) | sl[u].x;
+          const bool tail = in && l8 == 7 && gb == 0;  // lane 7 of a group without a match
+          const bool follow = tail && link != 0 && hop + 1 < kMaxHops;
+          if (tail && !follow) w.res[e[u].w] = make_uint2(0u, 0u);
+          const uint64_t fb = wave_ballot(follow);
+          if (follow) {
+            const uint64_t nb = key_vid(link);
+            const uint64_t bkt = FRAMED ? bucket_phys<true>(g, m, nb - m.indrct_start + m.psz) : nb;
+            w.kb[nn + (uint32_t)__builtin_popcountll(fb & below)] =
+                make_uint4(e[u].x, e[u].y, (uint32_t)bkt, e[u].w);
+          }
+          nn += (uint32_t)__builtin_popcountll(fb);
+        }
+      }
+      __builtin_amdgcn_wave_barrier();
+      n = nn;
     }
+    if (walk) {
+      const uint2 r = w.res[lane];
+      deg = r.x;
+      off = r.y;
+    }
+    __builtin_amdgcn_wave_barrier();  // w is reused by the wave's next call
   }
-  __builtin_amdgcn_wave_barrier();  // w is reused by the wave's next call
-  carry.key = lane63_64(key);
+  if (wave_ballot(valid) != leaders) {  // lanes that follow a leader take its result
+    const uint64_t mine = leaders & (below | (1ull << lane));
+    const uint32_t src = mine ? 63u - (uint32_t)__builtin_clzll(mine) : lane;
+    const uint32_t d = shfl32(deg, src), o = shfl32(off, src);
+    deg = mine ? d : carry.deg;  // (no leader: the lane continues the carried run)
+    off = mine ? o : carry.off;
+  }
+  deg_out = valid ? deg : 0u;
+  off_out = valid ? off : 0u;
+  carry.key = lane63_64(pl.key);
   carry.deg = lane63(deg_out);
   carry.off = lane63(off_out);
-  return L;
+  return (uint32_t)__builtin_popcountll(leaders);
+}
+
+// All parts at once, through the buckets alone: for a single key, and where
+// so few rows are probed that the tag word's latency costs more than it saves.
+template <bool FRAMED>
+__device__ __forceinline__ uint32_t wave_probe(const GraphView &g, const DevMeta &m, uint64_t key, WaveProbeLds &w,
+                                               uint32_t &deg_out, uint32_t &off_out, ProbeCarry &carry) {
+  return probe_finish<FRAMED, false>(g, m, probe_plan<FRAMED, false>(g, m, key, carry.key), w, deg_out, off_out,
+                                     carry);
 }
 
 // Inclusive wave scan of u64 values.

@@ -1154,7 +1154,8 @@ int wkg_batch_launch(wkg_batch *b, int nq, const wkg_plan_step *steps, const int
   {  // the captured sequences hold the graph view; a reloaded graph invalidates them
     const GraphView v = ctx->view(), &o = b->args.g;
     if (v.slots != o.slots || v.edges != o.edges || v.meta != o.meta || v.vframes != o.vframes ||
-        v.eframes != o.eframes || v.vshift != o.vshift || v.eshift != o.eshift || v.num_metas != o.num_metas) {
+        v.eframes != o.eframes || v.vshift != o.vshift || v.eshift != o.eshift || v.num_metas != o.num_metas ||
+        v.tags != o.tags) {
       b->clear_graphs();
       b->args.g = v;
     }

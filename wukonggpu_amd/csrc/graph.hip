@@ -61,6 +61,30 @@ __global__ void k_validate(const uint4 *slots, uint64_t num_buckets_total, uint6
   }
 }
 
+// The tag word of every main bucket (device.h), from its slots and its chain
+// (a checked image's chains end).
+__global__ __launch_bounds__(256) void k_make_tags(const uint4 *slots, uint64_t num_main, uint2 *tags) {
+  for (uint64_t b = blockIdx.x * 256ull + threadIdx.x; b < num_main; b += (uint64_t)gridDim.x * 256) {
+    uint64_t word = 0, link = 0;
+    for (int i = 0; i < kAssoc; i++) {
+      const uint4 v = slots[b * kAssoc + i];
+      const uint64_t k = ((uint64_t)v.y << 32) | v.x;
+      if (i == kAssoc - 1) link = k;
+      else if (k) word |= (uint64_t)key_tag(mix64(k)) << (8 * i);
+    }
+    for (uint32_t hop = 0; link && hop < kMaxHops; hop++) {
+      const uint4 *s = slots + key_vid(link) * kAssoc;
+      for (int i = 0; i < kAssoc; i++) {
+        const uint4 v = s[i];
+        const uint64_t k = ((uint64_t)v.y << 32) | v.x;
+        if (i == kAssoc - 1) link = k;
+        else if (k) word |= (uint64_t)key_chain_bit(mix64(k)) << 32;
+      }
+    }
+    tags[b] = make_uint2((uint32_t)word, (uint32_t)(word >> 32));
+  }
+}
+
 int log2_floor(uint64_t x) {
   int r = 0;
   while ((x >> (r + 1)) != 0) r++;
@@ -78,6 +102,7 @@ void wkg_ctx::free_graph() {
   if (d_slots) (void)hipFree(d_slots);
   if (d_edges) (void)hipFree(d_edges);
   if (d_meta) (void)hipFree(d_meta);
+  if (d_tags) (void)hipFree(d_tags);
   if (d_vframes) (void)hipFree(d_vframes);
   if (d_eframes) (void)hipFree(d_eframes);
   if (res) {
@@ -93,6 +118,7 @@ void wkg_ctx::free_graph() {
   d_slots = nullptr;
   d_edges = nullptr;
   d_meta = nullptr;
+  d_tags = nullptr;
   d_vframes = d_eframes = nullptr;
   res = nullptr;
   loaded = framed = sorted = false;
@@ -352,7 +378,7 @@ int wkg_ctx::set_image_metas(uint64_t nslots, uint64_t nedges, const wkg_pred_me
 
 // Second half of a resident load, with d_slots and d_edges in place: device
 // metas, the image checks on the device, and the table budget.
-int wkg_ctx::finish_resident(uint32_t flags, hipStream_t s) {
+int wkg_ctx::finish_resident(uint32_t flags, hipStream_t s, uint64_t tag_bytes) {
   if (hipMalloc(&d_meta, sizeof(DevMeta) * num_metas) != hipSuccess) {
     (void)hipGetLastError();
     free_graph();
@@ -388,6 +414,22 @@ int wkg_ctx::finish_resident(uint32_t flags, hipStream_t s) {
     return fail(WKG_EINVAL, "corrupt image (%s)", (vflags & 1u) ? "list outside its segment" : "bad chain link");
   }
   sorted = (flags & WKG_LOAD_SORTED_LISTS) || !(vflags & 4u);
+  // the probe's tag words, where memory (and the graph budget) allow
+  if (num_main && num_main * sizeof(uint2) <= tag_bytes) {
+    if (hipMalloc(&d_tags, num_main * sizeof(uint2)) == hipSuccess) {
+      k_make_tags<<<(unsigned)std::min<uint64_t>((num_main + 255) / 256, 1u << 16), 256, 0, s>>>(d_slots, num_main,
+                                                                                                  d_tags);
+      e = hipGetLastError();
+      if (e == hipSuccess) e = hipStreamSynchronize(s);
+      if (e != hipSuccess) {
+        free_graph();
+        return fail(WKG_EDEVICE, "tag words: %s", hipGetErrorString(e));
+      }
+    } else {
+      (void)hipGetLastError();
+      d_tags = nullptr;
+    }
+  }
   resident_bytes = num_slots * 16 + std::max<uint64_t>(num_edges, 1) * 4;
   loaded = true;
   if (!budget_request) {  // default table budget: 75% of what is left
@@ -424,7 +466,9 @@ int wkg_load_graph(wkg_ctx *ctx, const uint64_t *slots, uint64_t num_slots, cons
       ctx->free_graph();
       return ctx->fail(WKG_EDEVICE, "image upload failed: %s", hipGetErrorString(e));
     }
-    return ctx->finish_resident(flags, s);
+    // (a graph budget bounds the tag words too)
+    return ctx->finish_resident(flags, s,
+                                graph_budget_bytes ? graph_budget_bytes - slot_bytes - edge_bytes : ~uint64_t(0));
   } else {
     bool srt = true;
     int rc = validate_host(ctx, slots, edges, !(flags & WKG_LOAD_SORTED_LISTS), &srt);

@@ -161,6 +161,7 @@ template <int TR, bool SORTED, bool FRAMED>
 __device__ __forceinline__ void probe_tile(const GraphView &g, const StepParams &p, uint64_t lt) {
   constexpr int kRounds = TR / kBlock;  // one row per lane per round
   constexpr int kRowsPerThread = TR / kBlock;
+  constexpr bool kTags = !FRAMED;
   static_assert(TR % kBlock == 0, "tile rows must be a multiple of the block");
   __shared__ uint32_t s_cnt[TR];  // degree, or kept flag
   __shared__ uint32_t s_aux[TR];  // segment offset, or edges examined
@@ -183,19 +184,31 @@ __device__ __forceinline__ void probe_tile(const GraphView &g, const StepParams 
     cells[rd] = in ? T[row * p.c + p.sc] : -1;
     ends[rd] = in && p.mode == kModeK2K ? T[row * p.c + p.ec] : 0;
   }
-  ProbeCarry carry;
-  uint32_t probed = 0;
-  for (int rd = 0; rd < kRounds; rd++) {
-    const uint32_t local = wave * kWaveRows + rd * kWave + lane;
-    const uint64_t row = base + local;
+  auto plan = [&](int rd, uint64_t before63) {
+    const uint64_t row = base + wave * kWaveRows + rd * kWave + lane;
     uint64_t key = 0;
-    const int32_t end_cell = ends[rd];
     if (row < p.R) {
       if (p.key) key = p.key;
       else if (cells[rd] >= 0) key = make_key((uint32_t)cells[rd], p.pid, p.dir);
     }
+    return probe_plan<FRAMED, kTags>(g, m, key, before63);
+  };
+  ProbeCarry carry;
+  uint32_t probed = 0;
+  // round rd is finished while round rd + 1's slots and round rd + 2's tag
+  // words are on their way
+  ProbePlan pl[3];
+  pl[0] = plan(0, 0);
+  if (kRounds > 1) pl[1] = plan(1, lane63_64(pl[0].key));
+  probe_pick<kTags>(g, pl[0]);
+#pragma unroll
+  for (int rd = 0; rd < kRounds; rd++) {
+    const uint32_t local = wave * kWaveRows + rd * kWave + lane;
+    const int32_t end_cell = ends[rd];
+    if (rd + 2 < kRounds) pl[(rd + 2) % 3] = plan(rd + 2, lane63_64(pl[(rd + 1) % 3].key));
+    if (rd + 1 < kRounds) probe_pick<kTags>(g, pl[(rd + 1) % 3]);
     uint32_t deg, off;
-    probed += wave_probe<FRAMED>(g, m, key, s_wp[wave], deg, off, carry);
+    probed += probe_finish<FRAMED, kTags>(g, m, pl[rd % 3], s_wp[wave], deg, off, carry);
     if (p.mode == kModeK2U) {
       s_cnt[local] = deg;
       s_aux[local] = off;

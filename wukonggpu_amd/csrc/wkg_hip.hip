@@ -177,6 +177,7 @@ GraphView wkg_ctx::view() const {
   g.vshift = vshift;
   g.eshift = eshift;
   g.num_metas = num_metas;
+  g.tags = d_tags;
   return g;
 }
 
@@ -324,15 +325,13 @@ int wkg_ctx::step_single_list(uint64_t key, int pid, hipStream_t s, wkg_table **
   return WKG_OK;
 }
 
-// Probe tile rows for an R-row input: the largest tile that still gives
-// every CU at least four tiles, down to one 64-row round per wave. Small
-// inputs otherwise run on a few blocks whose rounds' bucket walks are one
-// long chain of load latencies each.
-static int probe_tile_rows(uint64_t R, int ncu) {
-  for (int tr = kTileRows; tr > kBlock; tr /= 2)
-    if (R >= (uint64_t)tr * 4 * (uint64_t)ncu) return tr;
-  return kBlock;
-}
+// Probe tile rows for an R-row input: 512 when that gives every CU at least
+// four tiles, else 256. Small inputs otherwise run on a few blocks whose
+// rounds' bucket walks are one long chain of load latencies each; larger
+// tiles, on large inputs, only make the compaction's units longer (the probe
+// itself is bound by cache misses: 24M random keys 320 us at 2048 rows and
+// 299 us at 512; the compaction of 1.5M kept rows of 3 cells 40 and 19 us).
+static int probe_tile_rows(uint64_t R, int ncu) { return R >= 512ull * 4 * (uint64_t)ncu ? 512 : kBlock; }
 
 // The per-step path splits its probe, finalize and expand passes into
 // launches of thread_launch_rows() input rows (expand: that / 64 tiles of

@@ -187,6 +187,7 @@ struct wkg_ctx {
   uint4 *d_slots = nullptr;
   uint32_t *d_edges = nullptr;
   wkg::DevMeta *d_meta = nullptr;
+  uint2 *d_tags = nullptr;  // tag words of a resident graph (null: none)
   uint64_t *d_vframes = nullptr, *d_eframes = nullptr;
   uint32_t vshift = 0, eshift = 0;
   uint32_t num_metas = 0;
@@ -265,7 +266,7 @@ struct wkg_ctx {
                          wkg_table **out, uint64_t *expanded);
   // residency
   int set_image_metas(uint64_t nslots, uint64_t nedges, const wkg_pred_meta_abi *m_in, int nmetas);
-  int finish_resident(uint32_t flags, hipStream_t s);
+  int finish_resident(uint32_t flags, hipStream_t s, uint64_t tag_bytes = ~uint64_t(0));
   int ensure_pred(int pid, hipStream_t s, const std::vector<int> *keep = nullptr);
   int load_pred(int pid, hipStream_t s, const std::vector<int> *keep, bool prefetch);
   void free_graph();
