@@ -101,7 +101,7 @@ def _kernel_table(dev, names, n):
 
 
 STEP_KERNELS = ("probe", "probe_filter", "fanout_filter", "scan_tiles", "finalize", "compact", "partition", "expand",
-                "probe_one", "copy_list", "small_step", "lineage")
+                "probe_one", "copy_list", "follow", "lineage")
 
 
 def _expand_roofline(dev, n_queries, traffic_file, extra=None):

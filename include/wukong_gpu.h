@@ -197,10 +197,12 @@ int wkg_set_fanout_blocks(wkg_ctx *ctx, int on, uint64_t kept_cap);
  * _end. No counterpart in the reference (one engine thread per GPU). */
 int wkg_thread_context_begin(wkg_ctx *ctx);
 int wkg_thread_context_end(wkg_ctx *ctx);
-/* A known-start step over at most 512 input rows runs its probe, scan,
- * compaction and (up to 2048 output rows) expand in one launch instead of
- * five; its output is the same, row for row. On by default; 0 turns it off.
- * A launch-count optimisation with no counterpart in the reference. */
+/* A known-start step over at most 2^20 input rows (2048 probe tiles) runs as
+ * two launches, the probe and one that scans, compacts and expands, while
+ * its output fits a table guessed for it (twice the input's rows, at most 8 MB
+ * and a 256th of the table budget), instead of three to five; its output is
+ * the same, row for row. On by default; 0 turns it off. A launch-count
+ * optimisation with no counterpart in the reference. */
 int wkg_set_small_steps(wkg_ctx *ctx, int on);
 /* Input rows per launch of the calling thread's per-step probe and
  * compaction passes (the expand: rows / 64 tiles of 512 items per launch);
@@ -476,7 +478,7 @@ int wkg_batch_autotune(wkg_batch *b, int nq, const wkg_plan_step *steps, const i
  * (core/rcache.hpp:300-385, BREAK_DOWN). Here each kernel launch can be
  * bracketed by HIP events on its own stream. Kernel names: "probe",
  * "probe_filter", "scan_tiles", "finalize", "compact", "partition", "expand",
- * "probe_one", "copy_list", "batch_probe", "batch_scan", "batch_finalize",
+ * "probe_one", "copy_list", "follow", "batch_probe", "batch_scan", "batch_finalize",
  * "batch_partition", "batch_expand", "copy_calibrate".
  * alg_bytes sums each launch's algorithmic byte count. */
 int wkg_profile_enable(wkg_ctx *ctx, int on);

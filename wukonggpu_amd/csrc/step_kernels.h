@@ -4,11 +4,14 @@
 //
 // One known_to_unknown step (RCache::known_to_unknown, core/rcache.hpp:
 // 232-414) runs as
-//   k_probe -> k_scan_tiles -> k_finalize -> [totals read back] -> k_partition -> k_expand
+//   k_probe -> k_follow (up to kScanChunk probe tiles and an output that fits), or
+//   k_probe -> tile scan -> [totals read back] -> k_hit_splits -> k_expand_hits, or
+//   k_probe -> tile scan -> k_finalize -> [totals] -> k_partition -> k_expand (large fan-outs)
 // replacing the reference's keygen, probe, edge-list fetch, Thrust scan and
 // one-thread-per-row update (core/gpu_hash.cu:145-316, 527-610, 685-694).
 // known_to_known / known_to_const (core/gpu_hash.cu:320-466, 613-682) run as
-//   k_probe -> k_scan_tiles -> k_finalize (stable compaction of kept rows)
+//   k_probe -> k_follow, or
+//   k_probe -> tile scan -> k_finalize (stable compaction of kept rows)
 // index_to_unknown / const_to_unknown are k_probe_copy (+ k_copy_list for a
 // list above kListCap entries).
 //
@@ -43,7 +46,8 @@ struct StepParams {
   uint32_t target_ok;  // K2C constant fits u32 (otherwise nothing matches)
   int mode;            // kMode*
   uint64_t key;        // != 0: single-key step (index / const start), R == 1
-  uint4 *hits;         // per tile, one entry per tile row: (row, offset, degree, 0) of rows with output
+  uint4 *hits;         // per tile, one entry per tile row: (row, offset, degree, K2U: the tile's output rows
+                       // before this one (mod 2^32)) of rows with output
   uint2 *cinfo;        // K2U, compacted rows: (row, offset)
   uint64_t *cexcl;     // K2U, compacted rows: exclusive output-row offset
   int32_t *O;          // filters: compacted output, capacity R x c
@@ -241,14 +245,15 @@ __device__ __forceinline__ void probe_tile(const GraphView &g, const StepParams 
   }
   uint64_t nz_total, sum_total, ex_total = 0;
   uint32_t pos = (uint32_t)block_excl_scan(nz, s_tmp, nz_total);
-  (void)block_excl_scan(sum, s_tmp, sum_total);
+  uint32_t before = (uint32_t)block_excl_scan(sum, s_tmp, sum_total);
   if (p.mode != kModeK2U) (void)block_excl_scan(ex, s_tmp, ex_total);
   uint4 *hits = p.hits + lt * TR;
 #pragma unroll
   for (int k = 0; k < kRowsPerThread; k++) {
     const uint32_t local = tid * kRowsPerThread + k;
     const uint32_t c = s_cnt[local];
-    if (c) gstore(hits + pos++, make_uint4((uint32_t)(base + local), p.mode == kModeK2U ? s_aux[local] : 0u, c, 0u));
+    if (c) gstore(hits + pos++, make_uint4((uint32_t)(base + local), p.mode == kModeK2U ? s_aux[local] : 0u, c, before));
+    before += c;
   }
   if (tid == 0) {
     gmem(p.tile_sum)[lt] = sum_total;
@@ -598,42 +603,342 @@ __global__ __launch_bounds__(kBlock) void k_expand(GraphView g, ExpandParams a) 
   expand_tile<kExpandVT, FRAMED>(g, a, a.tile0 + blockIdx.x);
 }
 
-// ---- a small step in one launch --------------------------------------------
-// A known-start step over at most kSmallRows input rows runs in one
-// workgroup: the probe tiles (kBlock rows each), the tile scan, the
-// finalize and, for known_to_unknown with at most `cap` output rows, the
-// merge-path split points and the expand into x.O (cap rows reserved) --
-// the multi-launch path's own tile bodies, separated by workgroup barriers
-// (after which the block sees its own global writes), so the tables are the
-// same. A bigger output leaves the compacted rows for the multi-launch
-// expand. Saves four launches on the per-step path's small steps, whose
-// time is launch latency.
-constexpr uint64_t kSmallRows = 2 * kBlock;
-constexpr uint64_t kSmallCap = 4 * kExpandNV;  // output rows expanded in the same launch
+// ---- expand and compaction straight from the probe's lists ----
+// A workgroup takes NV consecutive output rows and finds their hits (the
+// probe's per-tile lists) itself: the tile and the hit of its first and last
+// row by 64-ary searches over the tiles' prefixes and the tile's running
+// counts, so neither a compaction of the hits nor split points are needed
+// (two launches and 32 B moved per hit less than k_finalize, k_partition and
+// k_expand). Every hit has output, so NV rows need at most that many
+// hits. What bounds it: the output rows' stores and one random edge read per
+// row; the searches are a chain of dependent reads, hidden by the other
+// workgroups of the CU on large outputs.
+constexpr int kHitNV = kBlock * 4;     // output rows per block, large outputs
+constexpr int kFollowNV = kBlock * 2;  // and in k_follow: its outputs are small, their blocks few
+// (18M rows of 4 cells with 2048 / 1024 / 512 rows a block: 115 / 94 / 120 us;
+// 16 interactive queries, 2048 / 1024 / 512 in k_follow: 577 / 584 / 560 us.)
+struct HitExpand {
+  uint32_t pid;
+  const int32_t *T;  // input table
+  uint32_t c, tr;    // input columns; probe tile rows
+  const uint4 *hits;
+  uint64_t ntiles;
+  int32_t *O;        // known_to_unknown: rows x (c + 1); filters: rows x c
+  // known_to_unknown: where the compacted rows go (null: nowhere)
+  uint2 *cinfo;
+  uint64_t *cexcl;
+};
 
-template <bool SORTED, bool FRAMED>
-__global__ __launch_bounds__(kBlock) void k_small_step(GraphView g, StepParams p, ExpandParams x, uint64_t cap,
-                                                       uint64_t *part, Signal sg) {
-  for (uint64_t lt = 0; lt < p.ntiles; lt++) {
-    probe_tile<kBlock, SORTED, FRAMED>(g, p, lt);
-    __syncthreads();  // the tile's LDS is reused by the next
+// Largest i in [0, n) with f(i) <= x, by the whole wave (f ascends, f(0) <= x).
+template <class F>
+__device__ __forceinline__ uint64_t wave_last_le(uint64_t n, uint64_t x, F f) {
+  uint64_t lo = 0, hi = n;
+  while (hi - lo > 1) {
+    const uint64_t step = (hi - lo + kWave - 1) / kWave, i = lo + lane_id() * step;
+    const uint32_t k = (uint32_t)__builtin_popcountll(wave_ballot(i < hi && f(i) <= x));
+    lo += (k - 1) * step;
+    hi = lo + step < hi ? lo + step : hi;
   }
-  scan_chunk(p, 0, 1);
+  return lo;
+}
+
+typedef int32_t v4i32 __attribute__((ext_vector_type(4)));
+// The block's nrows x nc output cells, cell(row, column), to out (16-byte
+// aligned) as whole quads.
+template <class F>
+__device__ __forceinline__ void store_rows(int32_t *out, uint32_t nrows, uint32_t nc, F cell) {
+  const uint32_t tid = threadIdx.x, nint = nrows * nc;
+  for (uint32_t q = tid; q < nint / 4; q += kBlock) {
+    uint32_t r = 4 * q / nc, col = 4 * q - r * nc;
+    v4i32 v;
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+      v[k] = cell(r, col);
+      if (++col == nc) {
+        col = 0;
+        r++;
+      }
+    }
+    __builtin_nontemporal_store(v, (v4i32 *)out + q);
+  }
+  if (tid < (nint & 3)) {
+    const uint32_t e = (nint & ~3u) + tid;
+    out[e] = cell(e / nc, e % nc);
+  }
+}
+
+// The tile (from t0, of nt tiles) of hit n0 + r: the last whose first hit is
+// at most it (an empty tile shares its with the next). s_first: the tiles'
+// first hits from n0, or null: then nzp is read.
+template <class F>
+__device__ __forceinline__ uint64_t hit_tile(uint64_t t0, uint32_t nt, uint64_t n0, uint32_t r, const uint32_t *s_first,
+                                             F nzp) {
+  uint32_t lo = 0, hi = nt - 1;
+  while (lo < hi) {
+    const uint32_t mid = (lo + hi + 1) >> 1;
+    if (s_first ? s_first[mid] <= r : nzp(t0 + mid) <= n0 + r) lo = mid;
+    else hi = mid - 1;
+  }
+  return t0 + lo;
+}
+
+// The tile and the hit (counted over all tiles) of output row o, by the whole wave.
+template <class FP, class FN>
+__device__ __forceinline__ void find_hit(const HitExpand &a, uint64_t o, FP pre, FN nzp, uint64_t &tile, uint64_t &hit) {
+  tile = wave_last_le(a.ntiles, o, pre);
+  const uint64_t n = nzp(tile), cnt = nzp(tile + 1) - n, local = o - pre(tile);
+  hit = n + wave_last_le(cnt, local, [&](uint64_t k) -> uint64_t { return a.hits[tile * a.tr + k].w; });
+}
+
+// Output rows [o0, o0 + nout), nout <= NV, of a known_to_unknown step. pre(t)
+// and nzp(t): output rows and hits before tile t (nzp(ntiles): all hits). split:
+// (tile, hit) of the block's first row and of the next block's (the last
+// block's: of the last row), or null: then they are searched here. With
+// compact, the hits that start in the block also go to cinfo / cexcl.
+template <int NV, bool FRAMED, class FP, class FN>
+__device__ __forceinline__ void expand_hits_block(const GraphView &g, const HitExpand &a, uint64_t o0, uint32_t nout,
+                                                  bool compact, const uint2 *split, FP pre, FN nzp) {
+  constexpr int PER = NV / kBlock;
+  __shared__ int32_t s_start[NV + 1];    // per hit: its first output row, from the block's first
+  __shared__ uint32_t s_off[NV + 1], s_row[NV + 1];
+  __shared__ uint32_t s_edge[NV];        // per tile of the block (first), per output row (then)
+  __shared__ __align__(4) uint16_t s_map[NV];  // the hit that starts at an output row; then every row's hit
+  __shared__ uint64_t s_t[2], s_n[2];    // tile and hit of the block's first row and of its end
+  __shared__ uint32_t s_wmax[kBlock / kWave];
+  const uint32_t tid = threadIdx.x, lane = lane_id(), wave = tid / kWave;
+  for (uint32_t i = tid; i < NV / 2; i += kBlock) ((uint32_t *)s_map)[i] = 0;
+  if (split) {
+    if (tid < 2) {
+      const uint2 v = gload(split + tid);
+      s_t[tid] = v.x;
+      s_n[tid] = v.y;
+    }
+  } else if (wave < 2) {
+    uint64_t t, n;
+    find_hit(a, wave ? o0 + nout - 1 : o0, pre, nzp, t, n);
+    if (lane == 0) {
+      s_t[wave] = t;
+      s_n[wave] = n;
+    }
+  }
   __syncthreads();
-  for (uint64_t lt = threadIdx.x / kWave; lt < p.ntiles; lt += kBlock / kWave) finalize_tile<kBlock>(p, lt);
-  __syncthreads();
-  const uint64_t E = p.totals[0], nz = p.totals[2];
-  if (p.mode == kModeK2U && E != 0 && E <= cap) {
-    const uint64_t nx = (nz + E + kExpandNV - 1) / kExpandNV;
-    for (uint64_t k = threadIdx.x; k <= nx; k += kBlock) part[k] = merge_split<kExpandNV>(p.cexcl, nz, E, k);
+  const uint64_t t0 = s_t[0], n0 = s_n[0];
+  const uint32_t nt = (uint32_t)(s_t[1] - t0 + 1), nr = (uint32_t)(s_n[1] - n0 + 1);
+  const bool staged = nt <= (uint32_t)NV;  // the tiles' first hits, from n0, fit s_edge
+  if (staged && nt > 1) {
+    for (uint32_t i = tid; i < nt; i += kBlock) {
+      const uint64_t n = nzp(t0 + i);
+      s_edge[i] = n > n0 ? (uint32_t)(n - n0) : 0u;
+    }
     __syncthreads();
-    ExpandParams xx = x;
-    xx.R = nz;
-    xx.E = E;
-    xx.part = part;
-    for (uint64_t t = 0; t < nx; t++) expand_tile<kExpandVT, FRAMED>(g, xx, t);
   }
-  if (threadIdx.x == 0) publish(sg, p.totals, 3);  // (thread 0 wrote the totals)
+  for (uint32_t r = tid; r < nr; r += kBlock) {
+    const uint64_t t = hit_tile(t0, nt, n0, r, staged ? s_edge : nullptr, nzp);
+    const uint4 h = gload(a.hits + t * a.tr + (n0 + r - nzp(t)));
+    const int64_t start = (int64_t)(pre(t) + h.w) - (int64_t)o0;
+    s_start[r] = (int32_t)start;
+    s_row[r] = h.x;
+    s_off[r] = h.y;
+    // (hit 0 starts at or before the block's first row; the next block's hit may start at its first)
+    const bool inside = start < (int64_t)nout;
+    if (r && inside) s_map[start] = (uint16_t)r;
+    if (compact && start >= 0 && inside) {
+      gstore(a.cinfo + n0 + r, make_uint2(h.x, h.y));
+      gmem(a.cexcl)[n0 + r] = o0 + (uint64_t)start;
+    }
+  }
+  __syncthreads();
+  // every output row's hit: the last that starts at or before it
+  uint32_t hit[PER], m = 0;
+#pragma unroll
+  for (int k = 0; k < PER; k++) {
+    const uint32_t v = s_map[tid * PER + k];
+    m = v > m ? v : m;
+    hit[k] = m;
+  }
+  uint32_t run = m;
+#pragma unroll
+  for (int d = 1; d < kWave; d <<= 1) {
+    const uint32_t y = shfl32(run, (lane - d) & 63);
+    if (lane >= (uint32_t)d && y > run) run = y;
+  }
+  if (lane == kWave - 1) s_wmax[wave] = run;
+  uint32_t base = shfl32(run, (lane - 1) & 63);  // (by every lane: a masked lane's value cannot be read)
+  if (lane == 0) base = 0;
+  __syncthreads();
+#pragma unroll
+  for (int w = 0; w < kBlock / kWave - 1; w++)
+    if (w < (int)wave && s_wmax[w] > base) base = s_wmax[w];
+  const DevMeta mt = g.meta[a.pid];
+  uint32_t ev[PER];
+#pragma unroll
+  for (int k = 0; k < PER; k++) {
+    hit[k] = hit[k] > base ? hit[k] : base;
+    const uint32_t o = tid * PER + k;
+    ev[k] = o < nout ? edge_at<FRAMED>(g, mt.edge_start, mt.eframe_base,
+                                       s_off[hit[k]] + (uint32_t)((int32_t)o - s_start[hit[k]]))
+                     : 0u;
+  }
+#pragma unroll
+  for (int k = 0; k < PER; k++) {
+    s_map[tid * PER + k] = (uint16_t)hit[k];
+    s_edge[tid * PER + k] = ev[k];
+  }
+  __syncthreads();
+  // the block's output is contiguous and (NV being a multiple of 4) 16-byte aligned
+  const uint32_t c = a.c, nc = c + 1;
+  store_rows(a.O + o0 * nc, nout, nc, [&](uint32_t r, uint32_t col) -> int32_t {
+    return col < c ? gmem(a.T)[(uint64_t)s_row[s_map[r]] * c + col] : (int32_t)s_edge[r];
+  });
+}
+
+// Kept rows [o0, o0 + nout) of a filter step (a hit each).
+template <int NV, class FN>
+__device__ __forceinline__ void compact_hits_block(const HitExpand &a, uint64_t o0, uint32_t nout, FN nzp) {
+  __shared__ uint32_t s_row[NV];
+  __shared__ uint64_t s_t[2];  // tile of the block's first and last row
+  const uint32_t tid = threadIdx.x, wave = tid / kWave;
+  if (wave < 2) {
+    const uint64_t t = wave_last_le(a.ntiles, wave ? o0 + nout - 1 : o0, nzp);
+    if (lane_id() == 0) s_t[wave] = t;
+  }
+  __syncthreads();
+  const uint64_t t0 = s_t[0];
+  const uint32_t nt = (uint32_t)(s_t[1] - t0 + 1);
+  for (uint32_t r = tid; r < nout; r += kBlock) {
+    const uint64_t t = hit_tile(t0, nt, o0, r, nullptr, nzp);
+    s_row[r] = gload(a.hits + t * a.tr + (o0 + r - nzp(t))).x;
+  }
+  __syncthreads();
+  const uint32_t c = a.c;
+  store_rows(a.O + o0 * c, nout, c, [&](uint32_t r, uint32_t col) -> int32_t {
+    return gmem(a.T)[(uint64_t)s_row[r] * c + col];
+  });
+}
+
+// Large known_to_unknown outputs, after the tile scan (E < 2^32): the
+// blocks' first hits by one wave each, then the blocks. (Searched in the
+// blocks themselves the five dependent reads were half of a block's chain:
+// 2M rows to 18M of 4 cells 152 us a step, 146 with the splits.)
+struct ScannedTiles {
+  const uint64_t *tile_sum, *tile_nz, *chunk_sum, *chunk_nz;
+  uint64_t nz, E;
+  uint64_t block0;  // the launch's first block of kHitNV rows
+  uint2 *split;     // per block (+1): (tile, hit) of its first row
+  __device__ __forceinline__ uint64_t pre(uint64_t i) const { return tile_sum[i] + chunk_sum[i / kScanChunk]; }
+  __device__ __forceinline__ uint64_t nzp(uint64_t i, uint64_t ntiles) const {
+    return i >= ntiles ? nz : tile_nz[i] + chunk_nz[i / kScanChunk];
+  }
+};
+__global__ __launch_bounds__(kBlock) void k_hit_splits(HitExpand a, ScannedTiles t, uint64_t nblocks) {
+  const uint64_t b = blockIdx.x * (uint64_t)(kBlock / kWave) + threadIdx.x / kWave;
+  if (b > nblocks) return;
+  uint64_t tile, hit;
+  find_hit(a, b < nblocks ? b * kHitNV : t.E - 1, [&](uint64_t i) -> uint64_t { return t.pre(i); },
+           [&](uint64_t i) -> uint64_t { return t.nzp(i, a.ntiles); }, tile, hit);
+  if (lane_id() == 0) t.split[b] = make_uint2((uint32_t)tile, (uint32_t)hit);
+}
+template <bool FRAMED>
+__global__ __launch_bounds__(kBlock) void k_expand_hits(GraphView g, HitExpand a, ScannedTiles t) {
+  const uint64_t b = t.block0 + blockIdx.x, o0 = b * (uint64_t)kHitNV;
+  const uint32_t nout = (uint32_t)(t.E - o0 < (uint64_t)kHitNV ? t.E - o0 : (uint64_t)kHitNV);
+  expand_hits_block<kHitNV, FRAMED>(
+      g, a, o0, nout, a.cinfo != nullptr, t.split + b, [&](uint64_t i) -> uint64_t { return t.pre(i); },
+      [&](uint64_t i) -> uint64_t { return t.nzp(i, a.ntiles); });
+}
+
+// ---- the second launch of a step of at most kScanChunk tiles ----
+// Every workgroup scans the tile sums itself (a read of 16 B per tile and one
+// block scan), so no scan kernel runs between the probe and this one, and
+// the first workgroup publishes the step's counts. It is queued right behind
+// the probe, before the host knows the counts, into a table of `cap` rows:
+//  - filters (cap: the input's rows) copy their kept rows;
+//  - a known_to_unknown whose E rows fit cap expands them, and keeps the
+//    compacted rows when it fans out (E >= 4 hits);
+//  - one whose output does not fit compacts its hits (cinfo / cexcl, with
+//    64-bit offsets) for the expand that the host launches into a table of
+//    E rows.
+// @@M4@@
+struct FollowStep {
+  int mode;
+  uint64_t cap;
+  const uint64_t *tile_sum, *tile_nz, *tile_ex;  // the probe's, not scanned
+  uint64_t *totals;
+  Signal sg;
+};
+template <bool FRAMED>
+__global__ __launch_bounds__(kBlock) void k_follow(GraphView g, HitExpand a, FollowStep f) {
+  constexpr int PT = kScanChunk / kBlock;
+  __shared__ uint64_t s_pre[kScanChunk];
+  __shared__ uint32_t s_nzp[kScanChunk + 1];
+  __shared__ uint64_t s_tmp[2 * (kBlock / kWave)];
+  const uint32_t tid = threadIdx.x, lane = lane_id(), n = (uint32_t)a.ntiles;
+  const uint32_t lo = tid * PT;
+  uint64_t vs[PT], vn[PT], v[2] = {0, 0}, tot[2];
+#pragma unroll
+  for (int k = 0; k < PT; k++) {
+    vs[k] = lo + k < n ? f.tile_sum[lo + k] : 0;
+    vn[k] = lo + k < n ? f.tile_nz[lo + k] : 0;
+  }
+#pragma unroll
+  for (int k = 0; k < PT; k++) {
+    v[0] += vs[k];
+    v[1] += vn[k];
+  }
+  block_excl_scan_n<2>(v, s_tmp, tot);
+  const uint64_t E = tot[0], nz = tot[1];
+  if (blockIdx.x == 0) {
+    uint64_t e = 0, ex;
+    for (uint32_t i = tid; i < n; i += kBlock) e += f.tile_ex[i];
+    (void)block_excl_scan(e, s_tmp, ex);
+    if (tid == 0) {
+      const uint64_t w[3] = {E, ex, nz};
+      f.totals[0] = E;
+      f.totals[1] = ex;
+      f.totals[2] = nz;
+      publish(f.sg, w, 3);
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < PT; k++) {
+    if (lo + k < n) {
+      s_pre[lo + k] = v[0];
+      s_nzp[lo + k] = (uint32_t)v[1];
+    }
+    v[0] += vs[k];
+    v[1] += vn[k];
+  }
+  if (tid == 0) s_nzp[n] = (uint32_t)nz;
+  __syncthreads();
+  auto pre = [&](uint64_t t) -> uint64_t { return s_pre[t]; };
+  auto nzp = [&](uint64_t t) -> uint64_t { return s_nzp[t]; };
+  if (E > f.cap) {  // (known_to_unknown) one wave per tile
+    for (uint32_t t = blockIdx.x * (kBlock / kWave) + tid / kWave; t < n; t += gridDim.x * (kBlock / kWave)) {
+      const uint64_t n0 = s_nzp[t], out0 = s_pre[t];
+      const uint32_t cnt = (uint32_t)(s_nzp[t + 1] - n0);
+      uint64_t carry = 0;
+      for (uint32_t k0 = 0; k0 < cnt; k0 += kWave) {
+        const uint32_t j = k0 + lane;
+        const uint4 h = j < cnt ? gload(a.hits + (uint64_t)t * a.tr + j) : make_uint4(0, 0, 0, 0);
+        const uint64_t inc = wave_incl_scan(h.z);
+        if (j < cnt) {
+          gstore(a.cinfo + n0 + j, make_uint2(h.x, h.y));
+          gmem(a.cexcl)[n0 + j] = out0 + carry + inc - h.z;
+        }
+        carry += shfl64(inc, kWave - 1);
+      }
+    }
+    return;
+  }
+  constexpr uint64_t NV = kFollowNV;
+  for (uint64_t o0 = blockIdx.x * NV; o0 < E; o0 += gridDim.x * NV) {
+    const uint32_t nout = (uint32_t)(E - o0 < NV ? E - o0 : NV);
+    if (f.mode == kModeK2U)
+      expand_hits_block<kFollowNV, FRAMED>(g, a, o0, nout, a.cinfo && E >= 4 * nz, nullptr, pre, nzp);
+    else
+      compact_hits_block<kFollowNV>(a, o0, nout, nzp);
+    __syncthreads();  // the block's LDS is reused
+  }
 }
 
 // ---- a whole small query in one workgroup ----

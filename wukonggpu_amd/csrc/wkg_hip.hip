@@ -331,7 +331,11 @@ int wkg_ctx::step_single_list(uint64_t key, int pid, hipStream_t s, wkg_table **
 // tiles, on large inputs, only make the compaction's units longer (the probe
 // itself is bound by cache misses: 24M random keys 320 us at 2048 rows and
 // 299 us at 512; the compaction of 1.5M kept rows of 3 cells 40 and 19 us).
-static int probe_tile_rows(uint64_t R, int ncu) { return R >= 512ull * 4 * (uint64_t)ncu ? 512 : kBlock; }
+static int probe_tile_rows(uint64_t R, int ncu, int most = 512) {
+  for (int tr = most; tr > kBlock; tr /= 2)
+    if (R >= (uint64_t)tr * 4 * (uint64_t)ncu) return tr;
+  return kBlock;
+}
 
 // The per-step path splits its probe, finalize and expand passes into
 // launches of thread_launch_rows() input rows (expand: that / 64 tiles of
@@ -397,7 +401,7 @@ static uint64_t pass_scratch_words(uint64_t R, int TR) {
 // nothing is allocated.
 static int pass_setup(wkg_ctx *ctx, int mode, const wkg_table *in, int sc, int pid, int dir, int ec, int64_t cval,
                       int32_t *O, hipStream_t s, int TR, uint64_t extra, ProbePass &pp, StepParams &p,
-                      uint64_t *ext_scr = nullptr, void *ext_lin = nullptr) {
+                      uint64_t *ext_scr = nullptr, void *ext_lin = nullptr, bool compact = true) {
   const uint64_t R = in->rows;
   const int c = in->cols;
   const uint64_t ntiles = (R + TR - 1) / TR;
@@ -409,7 +413,7 @@ static int pass_setup(wkg_ctx *ctx, int mode, const wkg_table *in, int sc, int p
     pp.scr = (uint64_t *)ctx->pool->alloc((pass_scratch_words(R, TR) + extra) * 8, s, wkg_ctx::err_slot());
     if (!pp.scr) return WKG_ENOMEM;
   }
-  if (mode == kModeK2U) {  // cinfo[R] (8 B) | cexcl[R]: may outlive the step as the output's lineage
+  if (mode == kModeK2U && compact) {  // cinfo[R] (8 B) | cexcl[R]: may outlive the step as the output's lineage
     pp.lin = ext_scr ? ext_lin : ctx->pool->alloc(R * 16, s, wkg_ctx::err_slot());
     if (!pp.lin) {
       ctx->release_pass(pp, s);
@@ -452,20 +456,25 @@ static int pass_setup(wkg_ctx *ctx, int mode, const wkg_table *in, int sc, int p
 // every known-start step): for K2U the compacted rows with edges (cinfo) and
 // their output offsets (cexcl) in pp.lin; the filters compact into O.
 int wkg_ctx::probe_pass(int mode, const wkg_table *in, int sc, int pid, int dir, int ec, int64_t cval, int32_t *O,
-                        hipStream_t s, ProbePass &pp, int wcol, uint64_t *ext_scr, void *ext_lin, int tile_rows) {
+                        hipStream_t s, ProbePass &pp, int wcol, uint64_t *ext_scr, void *ext_lin, int tile_rows,
+                        bool compact) {
   const uint64_t R = in->rows;
   const int c = in->cols;
   const int TR = tile_rows ? tile_rows : probe_tile ? probe_tile : probe_tile_rows(R, ncu);
   StepParams p{};
-  int rc = pass_setup(this, mode, in, sc, pid, dir, ec, cval, O, s, TR, 0, pp, p, ext_scr, ext_lin);
+  int rc = pass_setup(this, mode, in, sc, pid, dir, ec, cval, O, s, TR, 0, pp, p, ext_scr, ext_lin,
+                      compact);
   if (rc) return rc;
   if (wcol >= 0) {
     p.weighted = 1;
     p.wc = (uint32_t)wcol;
   }
   pp.hits = p.hits;
+  pp.tile_sum = p.tile_sum;
   pp.tile_nz = p.tile_nz;
+  pp.chunk_sum = p.chunk_sum;
   pp.chunk_nz = p.chunk_nz;
+  pp.totals = p.totals;
   pp.ntiles = p.ntiles;
   pp.tr = TR;
   const uint64_t ntiles = p.ntiles, nchunks = (ntiles + kScanChunk - 1) / kScanChunk;
@@ -486,7 +495,8 @@ int wkg_ctx::probe_pass(int mode, const wkg_table *in, int sc, int pid, int dir,
     k_scan_chunks<<<(unsigned)nchunks, kBlock, 0, s>>>(p);
     if (nchunks > 1) k_scan_top<<<1, kBlock, 0, s>>>(p, nchunks);
   }
-  if (mode == kModeK2U || O) {  // (a filter without O leaves its kept rows in pp.hits)
+  // (a filter without O, or a known_to_unknown not to be compacted, leaves its rows in pp.hits)
+  if (mode == kModeK2U ? compact : O != nullptr) {
     ProfScope ps(this, s, mode == kModeK2U ? "finalize" : "compact", 0.0);
     launch_finalize(TR, p, s);
   }
@@ -498,13 +508,48 @@ int wkg_ctx::probe_pass(int mode, const wkg_table *in, int sc, int pid, int dir,
   }
   memcpy(pp.cnt, rb_host(), 3 * sizeof(uint64_t));
   if (mode == kModeK2U) {
-    prof_add_bytes("finalize", 32.0 * pp.cnt[2]);
+    if (compact) prof_add_bytes("finalize", 32.0 * pp.cnt[2]);
     prof_add_bytes("probe", 128.0 * (double)pp.cnt[1] + 16.0 * (double)pp.cnt[2]);
     prof_add_bytes("probe_keys", (double)pp.cnt[1]);  // counts, not bytes: keys probed (run leaders)
     prof_add_bytes("probe_rows", (double)R);           // and rows looked up
   } else if (O) {
     prof_add_bytes("compact", 16.0 * pp.cnt[2] + 8.0 * pp.cnt[2] * c);
   }
+  return WKG_OK;
+}
+
+// Room for the compacted rows of a known_to_unknown pass that was run
+// without them: its rows with edges (cinfo) and their output offsets
+// (cexcl), as many as it counted.
+int wkg_ctx::lineage_rows(ProbePass &pp, hipStream_t s) {
+  const uint64_t nz = pp.cnt[2];
+  if (!(pp.lin = pool->alloc(nz * 16, s, err_slot()))) return WKG_ENOMEM;
+  pp.cinfo = (uint2 *)pp.lin;
+  pp.cexcl = (uint64_t *)((char *)pp.lin + nz * 8);
+  return WKG_OK;
+}
+
+// Compacts such a pass.
+int wkg_ctx::compact_pass(ProbePass &pp, hipStream_t s) {
+  const uint64_t nz = pp.cnt[2];
+  if (pp.lin || !nz) return WKG_OK;
+  if (int rc = lineage_rows(pp, s)) return rc;
+  StepParams p{};
+  p.mode = kModeK2U;
+  p.hits = pp.hits;
+  p.cinfo = pp.cinfo;
+  p.cexcl = pp.cexcl;
+  p.tile_sum = pp.tile_sum;
+  p.tile_nz = pp.tile_nz;
+  p.chunk_sum = pp.chunk_sum;
+  p.chunk_nz = pp.chunk_nz;
+  p.totals = pp.totals;
+  p.ntiles = pp.ntiles;
+  {
+    ProfScope ps(this, s, "finalize", 32.0 * (double)nz);
+    launch_finalize(pp.tr, p, s);
+  }
+  LAUNCHCHK(this);
   return WKG_OK;
 }
 
@@ -561,15 +606,197 @@ int wkg_ctx::expand_pass(const wkg_table *in, int pid, const uint2 *cinfo, const
   return WKG_OK;
 }
 
+// Expand straight from the probe's lists (k_expand_hits) into t (pp.cnt[0]
+// rows); with room for them (lineage_rows) the compacted rows are written too.
+int wkg_ctx::expand_hits(const wkg_table *in, int pid, const ProbePass &pp, hipStream_t s, wkg_table *t) {
+  const uint64_t E = pp.cnt[0], nz = pp.cnt[2];
+  if (!E) return WKG_OK;
+  HitExpand x{};
+  x.pid = (uint32_t)pid;
+  x.T = in->d;
+  x.c = (uint32_t)in->cols;
+  x.tr = (uint32_t)pp.tr;
+  x.hits = pp.hits;
+  x.ntiles = pp.ntiles;
+  x.O = t->d;
+  x.cinfo = pp.cinfo;
+  x.cexcl = pp.cexcl;
+  const uint64_t nb = (E + kHitNV - 1) / kHitNV;
+  uint2 *split = (uint2 *)pool->alloc((nb + 1) * sizeof(uint2), s, err_slot());
+  if (!split) return WKG_ENOMEM;
+  ScannedTiles st{pp.tile_sum, pp.tile_nz, pp.chunk_sum, pp.chunk_nz, nz, E, 0, split};
+  {
+    ProfScope ps(this, s, "partition", 8.0 * (double)(nb + 1));
+    k_hit_splits<<<(unsigned)((nb + 1 + kBlock / kWave - 1) / (kBlock / kWave)), kBlock, 0, s>>>(x, st, nb);
+  }
+  {
+    // as the merge-path expand's, the hits 16 B each
+    ProfScope ps(this, s, "expand", 4.0 * E + 4.0 * E * (in->cols + 1) + 4.0 * nz * in->cols + 16.0 * nz);
+    const GraphView g = view();
+    const uint64_t per = std::max<uint64_t>(thread_launch_rows() / 128, 1);  // split launches, as the probe's
+    for (uint64_t b0 = 0; b0 < nb; b0 += per) {
+      st.block0 = b0;
+      const unsigned grid = (unsigned)std::min<uint64_t>(per, nb - b0);
+      if (framed) k_expand_hits<true><<<grid, kBlock, 0, s>>>(g, x, st);
+      else k_expand_hits<false><<<grid, kBlock, 0, s>>>(g, x, st);
+    }
+  }
+  pool->release(split, s);
+  LAUNCHCHK(this);
+  return WKG_OK;
+}
+
+// The rest of a known_to_unknown step after its probe pass: t is its output
+// if follow_pass already expanded it; else the output table is made here and
+// expanded from the probe's lists or, for fan-outs, from the compacted rows by
+// merge path. Compacted rows stay as the output's lineage when it fans out.
+// The line between the two: compacting costs about 8 ns per row with edges
+// and the split points 0.5 ns per output row, the hits' searches 0.7 ns per
+// output row (2M rows to 18M of 4 cells: 81 + 13 + 10 us by merge path, 77 + 14
+// from the lists), so the merge path is ahead above some 50 output rows per
+// row with edges; 24M keys to 9.3M rows of 2 cells: 127 + 54 + 15 and 128 + 14 us.
+int wkg_ctx::finish_k2u(const wkg_table *in, int pid, ProbePass &pp, hipStream_t s, wkg_table *t, wkg_table **out) {
+  const uint64_t E = pp.cnt[0], nz = pp.cnt[2];
+  const int out_cols = in->cols + 1;
+  int rc = WKG_OK;
+  if (table_limit && in->rows >= 2 && E * (uint64_t)out_cols * 4 > table_limit) {  // (one row cannot be split)
+    rc = fail(WKG_ENOMEM, "a %llu-row output is above the table limit", (unsigned long long)E);
+  } else if (!t && !(rc = new_table(E, out_cols, s, &t))) {
+    if (!pp.lin && E < (1ull << 32) && E < 32 * nz) {
+      if (wants_lineage(in, nz, E)) rc = lineage_rows(pp, s);
+      if (!rc) rc = expand_hits(in, pid, pp, s, t);
+    } else if (!(rc = compact_pass(pp, s))) {
+      rc = expand_pass(in, pid, pp.cinfo, pp.cexcl, nz, E, s, t);
+    }
+  }
+  if (rc) {
+    release_pass(pp, s);
+    drop_table(t);
+    return rc;
+  }
+  keep_lineage(in, pp, nz, t, pid);
+  release_pass(pp, s);
+  *out = t;
+  return WKG_OK;
+}
+
+// A step whose probe pass has at most kScanChunk tiles runs as two launches,
+// the probe and k_follow (small_steps; the rule's other side is the probe,
+// scan and compaction or expand passes). *tr: its probe tile rows.
+bool wkg_ctx::follows(uint64_t R, int *tr) const {
+  *tr = probe_tile ? probe_tile : probe_tile_rows(R, ncu);
+  return small_steps && (R + *tr - 1) / *tr <= (uint64_t)kScanChunk;
+}
+
+// The two launches. Filters: *t is the output. known_to_unknown: *t is the
+// output if it fitted the table that was guessed for it (else null, and
+// pp.lin holds the compacted rows, as it does when the output fans out).
+int wkg_ctx::follow_pass(int mode, const wkg_table *in, int sc, int pid, int dir, int ec, int64_t cval, int tr,
+                         hipStream_t s, ProbePass &pp, wkg_table **out) {
+  const uint64_t R = in->rows;
+  const int c = in->cols, out_cols = mode == kModeK2U ? c + 1 : c;
+  // the guess: twice the input's rows, within 8 MB and a 256th of the table
+  // budget (a table keeps its memory when it turns out shorter)
+  uint64_t cap = R;
+  if (mode == kModeK2U) {
+    uint64_t most = std::min<uint64_t>(8ull << 20, pool->budget / 256);
+    if (table_limit) most = std::min(most, table_limit);
+    cap = std::min(std::max<uint64_t>(2 * R, 8192), most / (4 * (uint64_t)out_cols));
+  }
+  wkg_table *t = nullptr;
+  int rc;
+  if (cap && (rc = new_table(cap, out_cols, s, &t))) {
+    if (mode != kModeK2U) return rc;
+    t = nullptr;
+    cap = 0;
+  }
+  StepParams p{};
+  if ((rc = pass_setup(this, mode, in, sc, pid, dir, ec, cval, t ? t->d : nullptr, s, tr, 0, pp, p))) {
+    drop_table(t);
+    return rc;
+  }
+  pp.hits = p.hits;
+  pp.tr = tr;
+  pp.ntiles = p.ntiles;
+  const GraphView g = view();
+  {
+    const double b = 4.0 * (double)R * c + (mode == kModeK2U ? 0.0 : 128.0 * (double)R);
+    ProfScope ps(this, s, mode == kModeK2U ? "probe" : "probe_filter", b);
+    launch_probe(tr, framed, sorted || mode == kModeK2U, g, p, s);
+  }
+  HitExpand x{};
+  x.pid = (uint32_t)pid;
+  x.T = in->d;
+  x.c = (uint32_t)c;
+  x.tr = (uint32_t)tr;
+  x.hits = p.hits;
+  x.ntiles = p.ntiles;
+  x.O = t ? t->d : nullptr;
+  x.cinfo = pp.cinfo;
+  x.cexcl = pp.cexcl;
+  FollowStep f{};
+  f.mode = mode;
+  f.cap = cap;
+  f.tile_sum = p.tile_sum;
+  f.tile_nz = p.tile_nz;
+  f.tile_ex = p.tile_ex;
+  f.totals = p.totals;
+  f.sg = next_signal();
+  {
+    ProfScope ps(this, s, "follow", 24.0 * (double)p.ntiles);
+    // blocks for the guessed rows, and for compacting the tiles (one wave each)
+    const uint64_t nb = std::max<uint64_t>((cap + kFollowNV - 1) / kFollowNV,
+                                           std::min<uint64_t>((p.ntiles + 3) / 4, (uint64_t)ncu));
+    if (framed) k_follow<true><<<(unsigned)nb, kBlock, 0, s>>>(g, x, f);
+    else k_follow<false><<<(unsigned)nb, kBlock, 0, s>>>(g, x, f);
+  }
+  hipError_t le = hipGetLastError();
+  rc = le == hipSuccess ? wait_signal(f.sg, s) : fail(WKG_EDEVICE, "step launch failed: %s", hipGetErrorString(le));
+  if (rc) {
+    release_pass(pp, s);
+    drop_table(t);
+    return rc;
+  }
+  memcpy(pp.cnt, rb_host(), 3 * sizeof(uint64_t));
+  const uint64_t rows = pp.cnt[0], nz = pp.cnt[2];
+  if (mode == kModeK2U) {
+    prof_add_bytes("probe", 128.0 * (double)pp.cnt[1] + 16.0 * (double)nz);
+    prof_add_bytes("probe_keys", (double)pp.cnt[1]);  // counts, not bytes: keys probed (run leaders)
+    prof_add_bytes("probe_rows", (double)R);           // and rows looked up
+  }
+  if (rows > cap) {
+    drop_table(t);
+    t = nullptr;
+  } else {
+    prof_add_bytes("follow", mode == kModeK2U ? 4.0 * rows * (out_cols + 1) + 4.0 * nz * c + 16.0 * nz
+                                              : 16.0 * rows + 8.0 * rows * c);
+    if (mode == kModeK2U && rows < 4 * nz) {  // (not compacted)
+      if (pp.lin) pool->release(pp.lin, s);
+      pp.lin = nullptr;
+    }
+    if (!t && (rc = new_table(0, out_cols, s, &t))) {
+      release_pass(pp, s);
+      return rc;
+    }
+    t->rows = rows;
+    t->bytes = rows * (uint64_t)out_cols * 4;
+  }
+  *out = t;
+  return WKG_OK;
+}
+
 // Keeps (cinfo, cexcl) of a known_to_unknown step with its output `t` when
 // the step fanned out (at least 4 output rows per input row with edges) and
 // both the input and the arrays are small next to the budget: a later
 // known_to_unknown step on one of the input's columns then probes once per
 // compacted input row (step_k2u_lineage).
+bool wkg_ctx::wants_lineage(const wkg_table *in, uint64_t nz, uint64_t E) const {
+  return lineage && nz != 0 && E >= 4 * nz &&
+         (in->owned || in->slice_of) &&  // not a caller's buffer (no-alloc step): nothing keeps it alive
+         in->bytes + in->rows * 16 <= pool->budget / 16;
+}
 void wkg_ctx::keep_lineage(const wkg_table *in, ProbePass &pp, uint64_t nz, wkg_table *t, int pid) {
-  if (!lineage || !pp.lin || nz == 0 || t->rows < 4 * nz) return;
-  if (!in->owned && !in->slice_of) return;  // a caller's buffer (no-alloc step): nothing keeps it alive
-  if (in->bytes + in->rows * 16 > pool->budget / 16) return;
+  if (!pp.lin || !wants_lineage(in, nz, t->rows)) return;
   wkg_table *par = const_cast<wkg_table *>(in);
   par->refs++;
   t->lin_parent = par;
@@ -1106,7 +1333,7 @@ int wkg_ctx::step_k2u_filter(const wkg_table *in, int sc, int pid, int dir, int 
                              uint64_t *ex_f) {
   *fused = 0;
   *ex_f = 0;
-  const bool fits = lineage && !framed && in && in->rows > kSmallRows && in->cols >= 1 && sc >= 0 && sc < in->cols &&
+  const bool fits = lineage && !framed && in && in->rows > 512 && in->cols >= 1 && sc >= 0 && sc < in->cols &&
                     !(in->lin_parent && sc < in->lin_parent->cols) && in->cols + 1 <= kBlock &&
                     in->rows < (1ull << 32) && (in->owned || in->slice_of);
   if (!fits || check_pattern(fpid, fdir) != WKG_OK || (fmode == kModeK2K && (ec < 0 || ec >= in->cols)))
@@ -1116,11 +1343,20 @@ int wkg_ctx::step_k2u_filter(const wkg_table *in, int sc, int pid, int dir, int 
   if ((rc = ensure_pred(pid, s))) return rc;
   const int c = in->cols;
   ProbePass pp;
-  if ((rc = probe_pass(kModeK2U, in, sc, pid, dir, -1, -1, nullptr, s, pp))) return rc;
+  wkg_table *t = nullptr;
+  int tr;
+  if (follows(in->rows, &tr)) rc = follow_pass(kModeK2U, in, sc, pid, dir, -1, -1, tr, s, pp, &t);
+  else rc = probe_pass(kModeK2U, in, sc, pid, dir, -1, -1, nullptr, s, pp, -1, nullptr, nullptr, 0, false);
+  if (rc) return rc;
   const uint64_t E = pp.cnt[0], nz = pp.cnt[2];
   *ex_u = E;
   if (E >= group_filter_rows && E < (1ull << 32) && nz > 0 && E >= 4 * nz && in->bytes + in->rows * 16 <= pool->budget / 16) {
     // the fan-out as lineage only
+    drop_table(t);
+    if ((rc = compact_pass(pp, s))) {
+      release_pass(pp, s);
+      return rc;
+    }
     wkg_table *v = new (std::nothrow) wkg_table;
     if (!v) {
       release_pass(pp, s);
@@ -1154,21 +1390,7 @@ int wkg_ctx::step_k2u_filter(const wkg_table *in, int sc, int pid, int dir, int 
     prof_add_bytes("fused_fanouts", -1.0);
     return step_known(kModeK2U, in, sc, pid, dir, -1, -1, s, out, ex_u);
   }
-  const int out_cols = c + 1;
-  if (table_limit && in->rows >= 2 && E * (uint64_t)out_cols * 4 > table_limit) {
-    release_pass(pp, s);
-    return fail(WKG_ENOMEM, "a %llu-row output is above the table limit", (unsigned long long)E);
-  }
-  wkg_table *t = nullptr;
-  if ((rc = new_table(E, out_cols, s, &t)) || (rc = expand_pass(in, pid, pp.cinfo, pp.cexcl, nz, E, s, t))) {
-    release_pass(pp, s);
-    drop_table(t);
-    return rc;
-  }
-  keep_lineage(in, pp, nz, t, pid);
-  release_pass(pp, s);
-  *out = t;
-  return WKG_OK;
+  return finish_k2u(in, pid, pp, s, t, out);
 }
 
 int wkg_ctx::step_known(int mode, const wkg_table *in, int sc, int pid, int dir, int ec, int64_t cval,
@@ -1191,129 +1413,43 @@ int wkg_ctx::step_known(int mode, const wkg_table *in, int sc, int pid, int dir,
   }
   if (mode == kModeK2U && lineage && in->lin_parent && sc < in->lin_parent->cols)
     return step_k2u_lineage(in, sc, pid, dir, s, out, expanded);
-  if (small_steps && R <= kSmallRows) return step_small(mode, in, sc, pid, dir, ec, cval, s, out, expanded);
-  if (mode != kModeK2U && lineage && !framed && in->glin_parent && sc == c - 1 &&
+  const bool tiny = small_steps && R <= 512;  // (too few rows for the filters below to pay)
+  if (mode != kModeK2U && !tiny && lineage && !framed && in->glin_parent && sc == c - 1 &&
       (mode == kModeK2C || ec < in->glin_parent->cols) && R >= group_filter_rows && R >= 4 * in->glin_dtot)
     return step_filter_groups(mode, in, pid, dir, ec, cval, s, out, expanded);
-  if (mode != kModeK2U && lineage && !framed && in->lin_parent && sc == c - 1 &&
+  if (mode != kModeK2U && !tiny && lineage && !framed && in->lin_parent && sc == c - 1 &&
       (mode == kModeK2C || ec < in->lin_parent->cols) && R >= group_filter_rows) {
     rc = step_filter_fanout(mode, in, pid, dir, ec, cval, s, out, expanded);
     if (rc != kNotTaken) return rc;
   }
 
   wkg_table *t = nullptr;
-  if (mode != kModeK2U && (rc = new_table(R, c, s, &t))) return rc;
   ProbePass pp;
-  if ((rc = probe_pass(mode, in, sc, pid, dir, ec, cval, t ? t->d : nullptr, s, pp))) {
-    drop_table(t);
-    return rc;
-  }
-  if (mode != kModeK2U) {  // filters: kept rows compacted in place
-    t->rows = pp.cnt[0];
-    t->bytes = t->rows * (uint64_t)c * 4;
-    if (expanded) *expanded = pp.cnt[1];
-    release_pass(pp, s);
-    *out = t;
-    return WKG_OK;
-  }
-  const uint64_t E = pp.cnt[0], nz = pp.cnt[2];
-  if (table_limit && R >= 2 && E * (uint64_t)out_cols * 4 > table_limit) {  // (one row cannot be split)
-    release_pass(pp, s);
-    return fail(WKG_ENOMEM, "a %llu-row output is above the table limit", (unsigned long long)E);
-  }
-  if (expanded) *expanded = E;
-  if ((rc = new_table(E, out_cols, s, &t)) || (rc = expand_pass(in, pid, pp.cinfo, pp.cexcl, nz, E, s, t))) {
-    release_pass(pp, s);
-    drop_table(t);
-    return rc;
-  }
-  keep_lineage(in, pp, nz, t, pid);
-  release_pass(pp, s);
-  *out = t;
-  return WKG_OK;
-}
-
-// A known-start step over at most kSmallRows rows in one launch
-// (k_small_step) and one read-back of its totals. A known_to_unknown output
-// of more than kSmallCap rows is expanded by the multi-launch expand from
-// the compacted rows the launch left.
-int wkg_ctx::step_small(int mode, const wkg_table *in, int sc, int pid, int dir, int ec, int64_t cval,
-                        hipStream_t s, wkg_table **out, uint64_t *expanded) {
-  const uint64_t R = in->rows;
-  const int c = in->cols;
-  const int out_cols = mode == kModeK2U ? c + 1 : c;
-  wkg_table *t = nullptr;
-  int rc = new_table(mode == kModeK2U ? kSmallCap : R, out_cols, s, &t);
-  if (rc) return rc;
-  ProbePass pp;
-  StepParams p{};
-  const uint64_t part_words = kSmallCap / kExpandNV + 2;  // split points of the in-launch expand
-  if ((rc = pass_setup(this, mode, in, sc, pid, dir, ec, cval, mode == kModeK2U ? nullptr : t->d, s, kBlock,
-                       part_words, pp, p))) {
-    drop_table(t);
-    return rc;
-  }
-  uint64_t *part = (uint64_t *)(p.hits + p.ntiles * kBlock);
-  ExpandParams x{};
-  x.pid = (uint32_t)pid;
-  x.T = in->d;
-  x.c = (uint32_t)c;
-  x.cinfo = p.cinfo;
-  x.cexcl = p.cexcl;
-  x.O = t->d;
-  const GraphView g = view();
-  const bool srt = sorted || mode == kModeK2U;
-  const Signal sg = next_signal();
-  {
-    ProfScope ps(this, s, "small_step", 4.0 * (double)R * c + 128.0 * (double)R);
-    if (framed) {
-      if (srt) k_small_step<true, true><<<1, kBlock, 0, s>>>(g, p, x, kSmallCap, part, sg);
-      else k_small_step<false, true><<<1, kBlock, 0, s>>>(g, p, x, kSmallCap, part, sg);
-    } else {
-      if (srt) k_small_step<true, false><<<1, kBlock, 0, s>>>(g, p, x, kSmallCap, part, sg);
-      else k_small_step<false, false><<<1, kBlock, 0, s>>>(g, p, x, kSmallCap, part, sg);
-    }
-  }
-  hipError_t le = hipGetLastError();
-  rc = le == hipSuccess ? wait_signal(sg, s) : fail(WKG_EDEVICE, "small step launch failed: %s", hipGetErrorString(le));
-  if (rc) {
-    release_pass(pp, s);
-    drop_table(t);
-    return rc;
-  }
-  memcpy(pp.cnt, rb_host(), 3 * sizeof(uint64_t));
-  if (mode != kModeK2U) {  // filters: kept rows compacted in place
-    t->rows = pp.cnt[0];
-    t->bytes = t->rows * (uint64_t)c * 4;
-    if (expanded) *expanded = pp.cnt[1];
-    release_pass(pp, s);
-    *out = t;
-    return WKG_OK;
-  }
-  const uint64_t E = pp.cnt[0], nz = pp.cnt[2];
-  if (table_limit && R >= 2 && E * (uint64_t)out_cols * 4 > table_limit) {  // (one row cannot be split)
-    release_pass(pp, s);
-    drop_table(t);
-    return fail(WKG_ENOMEM, "a %llu-row output is above the table limit", (unsigned long long)E);
-  }
-  if (E <= kSmallCap) {  // expanded in the launch
-    t->rows = E;
-    t->bytes = E * (uint64_t)out_cols * 4;
+  int tr;
+  if (follows(R, &tr)) {
+    if ((rc = follow_pass(mode, in, sc, pid, dir, ec, cval, tr, s, pp, &t))) return rc;
   } else {
-    drop_table(t);
-    t = nullptr;
-    if ((rc = new_table(E, out_cols, s, &t)) || (rc = expand_pass(in, pid, pp.cinfo, pp.cexcl, nz, E, s, t))) {
-      release_pass(pp, s);
+    if (mode != kModeK2U && (rc = new_table(R, c, s, &t))) return rc;
+    if ((rc = probe_pass(mode, in, sc, pid, dir, ec, cval, t ? t->d : nullptr, s, pp, -1, nullptr, nullptr, 0,
+                         false))) {
       drop_table(t);
       return rc;
     }
   }
+  if (mode != kModeK2U) {  // filters: kept rows compacted in place
+    t->rows = pp.cnt[0];
+    t->bytes = t->rows * (uint64_t)c * 4;
+    if (expanded) *expanded = pp.cnt[1];
+    release_pass(pp, s);
+    *out = t;
+    return WKG_OK;
+  }
+  const uint64_t E = pp.cnt[0];
+  if ((rc = finish_k2u(in, pid, pp, s, t, out))) return rc;
   if (expanded) *expanded = E;
-  keep_lineage(in, pp, nz, t, pid);
-  release_pass(pp, s);
-  *out = t;
   return WKG_OK;
 }
+
 
 int wkg_thread_launch_rows(wkg_ctx *ctx, uint64_t rows) {
   if (!ctx) return WKG_EINVAL;
@@ -1822,7 +1958,8 @@ int wkg_step_k2u_noalloc(wkg_ctx *ctx, const int32_t *in, uint64_t rows, int col
   hipStream_t s = ctx->pick(stream);
   // scratch: the probe passes' words | compacted rows (16 B per row) | the expand's split points
   auto up = [](uint64_t b) { return (b + 255) & ~uint64_t(255); };
-  const int TR = ctx->probe_tile ? ctx->probe_tile : probe_tile_rows(rows, ctx->ncu);
+  // (large tiles: fewer scratch words, so the largest input fits)
+  const int TR = ctx->probe_tile ? ctx->probe_tile : probe_tile_rows(rows, ctx->ncu, kTileRows);
   const uint64_t pass_b = up(pass_scratch_words(rows, TR) * 8), lin_b = up(rows * 16);
   if (pass_b + lin_b + 256 > WKG_NOALLOC_SCRATCH_BYTES)
     return ctx->fail(WKG_ERANGE, "a %llu-row input needs %llu bytes of step scratch, above the %llu of the no-alloc step",

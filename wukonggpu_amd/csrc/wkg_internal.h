@@ -100,13 +100,13 @@ constexpr int kNotTaken = 1;
 // One step's probe, tile scan and compaction (wkg_ctx::probe_pass).
 struct ProbePass {
   uint64_t *scr = nullptr;    // step scratch
-  void *lin = nullptr;        // known_to_unknown: cinfo | cexcl (may become the output's lineage)
+  void *lin = nullptr;        // known_to_unknown, compacted: cinfo | cexcl (may become the output's lineage)
   uint2 *cinfo = nullptr;     // compacted rows with edges: (row, list offset)
   uint64_t *cexcl = nullptr;  // their first output row
   uint64_t cnt[3] = {0, 0, 0};  // output rows, edges examined or keys probed, rows with output
   // the probe's kept-row lists and their tile prefixes (valid until release)
-  const uint4 *hits = nullptr;
-  const uint64_t *tile_nz = nullptr, *chunk_nz = nullptr;
+  uint4 *hits = nullptr;
+  uint64_t *tile_sum = nullptr, *tile_nz = nullptr, *chunk_sum = nullptr, *chunk_nz = nullptr, *totals = nullptr;
   uint64_t ntiles = 0;
   int tr = 0;
   bool external = false;  // scr / lin are the caller's memory, not the pool's
@@ -163,7 +163,7 @@ struct wkg_ctx {
   uint64_t group_filter_rows = 1ull << 22;  // smallest input a filter decides per lineage group
   bool fanout_blocks = true;  // long shared lists: k_fanout_blocks (else k_fanout_units)
   uint64_t fanout_kept_cap = 1ull << 22;  // k_fanout_blocks' kept-row list (more: rerun on k_fanout_units)
-  bool small_steps = true;   // steps over at most kSmallRows rows in one launch
+  bool small_steps = true;   // steps of at most kScanChunk probe tiles in two launches
   uint64_t *noalloc_scratch = nullptr;  // this device's no-alloc step scratch (wkg_step_k2u_noalloc)
   SQServer *sqs = nullptr;   // the persistent small-query server (created on first use)
   int sq_workgroups = 4;     // its workgroups (0: one launch per small query)
@@ -251,12 +251,18 @@ struct wkg_ctx {
                       int64_t cval, hipStream_t s, wkg_table **out, int *fused, uint64_t *ex_u, uint64_t *ex_f);
   int probe_pass(int mode, const wkg_table *in, int sc, int pid, int dir, int ec, int64_t cval, int32_t *O,
                  hipStream_t s, ProbePass &pp, int wcol = -1, uint64_t *ext_scr = nullptr, void *ext_lin = nullptr,
-                 int tile_rows = 0);
-  int step_small(int mode, const wkg_table *in, int sc, int pid, int dir, int ec, int64_t cval, hipStream_t s,
-                 wkg_table **out, uint64_t *expanded);
+                 int tile_rows = 0, bool compact = true);
+  int lineage_rows(ProbePass &pp, hipStream_t s);
+  int compact_pass(ProbePass &pp, hipStream_t s);
+  int expand_hits(const wkg_table *in, int pid, const ProbePass &pp, hipStream_t s, wkg_table *t);
+  int finish_k2u(const wkg_table *in, int pid, ProbePass &pp, hipStream_t s, wkg_table *t, wkg_table **out);
+  bool follows(uint64_t R, int *tr) const;
+  int follow_pass(int mode, const wkg_table *in, int sc, int pid, int dir, int ec, int64_t cval, int tr, hipStream_t s,
+                  ProbePass &pp, wkg_table **t);
   void release_pass(ProbePass &pp, hipStream_t s);
   int expand_pass(const wkg_table *in, int pid, const uint2 *cinfo, const uint64_t *cexcl, uint64_t nz, uint64_t E,
                   hipStream_t s, wkg_table *t, const char *tag = "expand", uint64_t *ext_part = nullptr);
+  bool wants_lineage(const wkg_table *in, uint64_t nz, uint64_t E) const;
   void keep_lineage(const wkg_table *in, ProbePass &pp, uint64_t nz, wkg_table *t, int pid);
   int step_filter_fanout(int mode, const wkg_table *in, int pid, int dir, int ec, int64_t cval, hipStream_t s,
                          wkg_table **out, uint64_t *expanded);

@@ -144,7 +144,7 @@ class Device:
         self._check(N.hip_lib().wkg_thread_launch_rows(self._h, int(rows)))
 
     def set_small_steps(self, on):
-        """Known-start steps over at most 512 rows in one launch (on by default)."""
+        """Known-start steps over at most 2^20 rows in two launches (on by default)."""
         self._check(N.hip_lib().wkg_set_small_steps(self._h, 1 if on else 0))
 
     def set_lineage(self, on):
