@@ -282,29 +282,24 @@ def run_config5(args, quick=False, nested=False):
     nf, msf, bf = dev.profile_read("fanout_filter")
     dev.profile(False)
     log(f"fan-out filter per query: {fanout}")
-    # the dominant kernel: the fan-out filter (k_fanout_blocks) when the
+    # the dominant kernel: the fan-out filter (k_list_filter) when the
     # fan-out is fused with its filter (the longest launch of the query; the
     # four probe launches together take about as long), else the expand
     roof = None
     if msf > 0:
         ach = bf / (msf * 1e-3) / 1e9
         pairs = r.expanded  # (the fan-out's rows dominate the work count)
-        tp = os.path.join(ROOT, "profiles", "fanout_cycle_2b.traffic.json")
         traffic, tsrc = None, None
-        if os.path.exists(tp):
-            with open(tp) as fh:
-                tj = json.load(fh)
-            traffic, tsrc = tj["hbm_bytes_per_launch"], tj["source"]
         roof = {"bound": "hbm", "achieved": ach, "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": ach / HBM_PEAK_GBS,
                 "traffic": traffic, "traffic_source": tsrc,
-                "kernel": "fanout_filter (k_fanout_blocks, with its 1-word counter reset)",
+                "kernel": "fanout_filter (k_list_filter and k_list_long)",
                 "launches_per_query": nf / n_prof, "avg_launch_ms": msf / nf, "alg_bytes_per_launch": bf / nf,
                 "pair_tests_per_s": pairs / (msf / n_prof * 1e-3),
-                "note": "the fused fan-out's filter tests each of the ~1.36G (parent row, list entry) pairs with a "
-                        "register compare (64 rows per compare mask); its HBM bytes are each D entry once per "
-                        "group of 64 parents and three counters per unit, so it is bound by each workgroup's "
-                        "chain of dependent loads (list, parents, targets, entries), not HBM: pair_tests_per_s "
-                        "against 39.3 T compare lanes/s (256 CUs x 4 SIMD16 x 2.4 GHz)"}
+                "note": "the fused fan-out's filter decides ~1.36G (parent row, list entry) pairs by probing each "
+                        "distinct list entry once (a tag word, the slot of a present key, its list) and looking "
+                        "its neighbours up among the hashed targets of the list's parents; 140 B per distinct "
+                        "entry are counted; it is bound by the probes' cache misses. pair_tests_per_s counts the "
+                        "pairs decided"}
     else:
         roof = _expand_roofline(dev, n_prof, "expand_cycle_2b.traffic.json")
     log(f"{roof['kernel']}: {roof['launches_per_query']:.0f} launches/query, {roof['avg_launch_ms']:.3f} ms avg, "

@@ -1841,8 +1841,8 @@ __global__ __launch_bounds__(kBlock) void k_fanout_units(GraphView g, StepParams
   }
 }
 
-// The fan-out filter for long shared lists, a block of list entries at a
-// time: a workgroup takes kFBRows entries of one distinct list and up to
+// The fan-out filter for long shared lists of many kept rows (or unsorted
+// filter lists), a block of list entries at a time: a workgroup takes kFBRows entries of one distinct list and up to
 // kFBGroup (= 64) of the parents sharing that list, and tests every parent
 // against every entry's list, holding the block in registers:
 //  - thread t takes entries t, t + 256, ...: their D entries are read once;
@@ -2073,6 +2073,265 @@ __global__ __launch_bounds__(kBlock) void k_fanout_blocks(GraphView g, StepParam
     p.tile_nz[rank] = s_kcnt[tid];
     p.tile_ex[rank] = xt;
   }
+}
+
+// ---- the fan-out filter through its lists (sorted images, few kept rows) ----
+// The pairs (parent, list entry) of a fan-out need not be tested one by one:
+// row (i, j) is kept iff parent i's target is in the filter list of entry j
+// of i's list, so the targets of the parents sharing a list are hashed once
+// (k_list_parents), and every element of every entry's filter list is looked
+// up among them (k_list_filter; elements of long filter lists in
+// k_list_long). The work is one probe per distinct list entry and one lookup
+// per element of the lists it finds, whatever the number of parents; the work
+// count is, per list, its parents times its entries' degrees, less what the
+// reference's early exit spares each kept row. Kept rows are listed
+// unordered and ranked by their row (k_list_rows).
+// What bounds it: the probe of the distinct entries (cache misses); nearly
+// all lookups end at a bit of a filter in L1. The cycle's closing filter over
+// 1.9G pairs of 1.6M distinct entries: its query 618 -> 285 us (pair by pair in
+// k_fanout_blocks 256 us, on top of the probe's 46 us, its passes' 40 us, and
+// 150 us of lists gathered on the host).
+struct ListFilter {
+  // the fan-out's parents
+  const uint2 *info;     // (parent row, list offset)
+  const uint64_t *excl;  // first child row
+  uint64_t np, R;
+  const int32_t *P;
+  uint32_t pc;
+  int32_t ec;            // known_to_known end column (a parent column); -1: known_to_const
+  uint32_t target, target_ok;
+  uint32_t lpid, pid, dir;  // the fan-out's predicate; the filter's pattern
+  // distinct lists, in first-come order: offset, entries before, length, parents
+  uint32_t *l_off, *l_base, *l_len, *l_np;
+  uint32_t *seen, *seen_list, mask1;  // offset -> list (open addressing)
+  uint32_t *p_list, *p_tgt, *next;    // per parent: list, target, next parent of the same two (+1)
+  uint32_t *head, *count, log2;       // (list, target) -> first parent (+1), parents (open addressing, 2^log2)
+  uint32_t *bits, blog2;              // two bits of a word per (list, target), 2^blog2 words
+  unsigned long long *ctr;            // kList*
+  uint4 *kept;                        // (row, parent, entry, 0)
+  uint64_t cap;
+  uint4 *longs;                       // (entry, offset, degree, first element)
+  uint64_t long_cap;
+};
+enum { kListSums = 0, kListUnits, kListKept, kListEx, kListSpared, kListLongs, kListCtrs };
+constexpr uint32_t kNoList = 0xffffffffu;  // (segments hold fewer than 2^32 edges)
+constexpr uint32_t kListInline = 16;       // longer filter lists go to k_list_long,
+constexpr uint32_t kListChunk = 1024;      // this many elements an item
+constexpr int kListTile = 1024;            // list entries per workgroup
+constexpr uint64_t kListKeptCap = 32768;   // ranking compares all kept rows with each other
+
+__device__ __forceinline__ uint32_t pair_hash(uint32_t l, uint32_t t) {
+  uint32_t h = (l * 0x9E3779B1u + t) * 0x85EBCA6Bu;
+  h ^= h >> 15;
+  return h * 0xC2B2AE35u;
+}
+__device__ __forceinline__ uint32_t pair_slot(const ListFilter &f, uint32_t h) { return (h * 0x27D4EB2Fu) >> (32 - f.log2); }
+__device__ __forceinline__ uint32_t pair_bits(uint32_t h) { return (1u << (h & 31)) | (1u << ((h >> 5) & 31)); }
+
+// The distinct lists and the parents' targets, by one workgroup (its phases
+// are separated by barriers; words changed by atomics are read as atomics).
+__global__ __launch_bounds__(1024) void k_list_parents(ListFilter f, Signal sg) {
+  const uint32_t tid = threadIdx.x, np = (uint32_t)f.np;
+  for (uint32_t i = tid; i <= f.mask1; i += 1024) f.seen[i] = kNoList;
+  for (uint32_t i = tid; i < 1u << f.log2; i += 1024) f.head[i] = f.count[i] = 0;
+  for (uint32_t i = tid; i < 1u << f.blog2; i += 1024) f.bits[i] = 0;
+  for (uint32_t i = tid; i < np; i += 1024) f.l_np[i] = 0;
+  if (tid < kListCtrs) f.ctr[tid] = 0;
+  __threadfence();
+  __syncthreads();
+  uint64_t units = 0;
+  for (uint32_t i = tid; i < np; i += 1024) {
+    const uint32_t off = f.info[i].y;
+    const uint64_t n = (i + 1 < np ? f.excl[i + 1] : f.R) - f.excl[i];
+    units += (n + kFBRows - 1) / kFBRows;
+    uint32_t s = (off * 0x9E3779B1u) & f.mask1;
+    for (;; s = (s + 1) & f.mask1) {
+      uint32_t old = __hip_atomic_load(&f.seen[s], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (old == kNoList) old = atomicCAS(&f.seen[s], kNoList, off);
+      if (old == kNoList) {  // the first parent of this list
+        const unsigned long long v = atomicAdd(&f.ctr[kListSums], (1ull << 40) | n);
+        const uint32_t l = (uint32_t)(v >> 40);
+        f.l_off[l] = off;
+        f.l_base[l] = (uint32_t)v;
+        f.l_len[l] = (uint32_t)n;
+        f.seen_list[s] = l;
+        break;
+      }
+      if (old == off) break;
+    }
+    f.next[i] = s;  // (the list's slot, for now)
+  }
+  if (units) atomicAdd(&f.ctr[kListUnits], (unsigned long long)units);
+  __threadfence();
+  __syncthreads();
+  for (uint32_t i = tid; i < np; i += 1024) {
+    const uint32_t l = f.seen_list[f.next[i]];
+    f.p_list[i] = l;
+    f.p_tgt[i] = f.ec >= 0 ? (uint32_t)f.P[(uint64_t)f.info[i].x * f.pc + (uint32_t)f.ec] : f.target;
+    atomicAdd(&f.l_np[l], 1u);
+  }
+  __threadfence();
+  __syncthreads();
+  for (uint32_t i = tid; i < np; i += 1024) {
+    const uint32_t l = f.p_list[i], t = f.p_tgt[i];
+    if (f.ec >= 0 ? (int32_t)t < 0 : !f.target_ok) continue;
+    const uint32_t h = pair_hash(l, t);
+    atomicOr(&f.bits[h >> (32 - f.blog2)], pair_bits(h));
+    for (uint32_t s = pair_slot(f, h);; s = (s + 1) & ((1u << f.log2) - 1)) {
+      const uint32_t old = atomicCAS(&f.head[s], 0u, i + 1);
+      if (old != 0 && (f.p_list[old - 1] != l || f.p_tgt[old - 1] != t)) continue;
+      f.next[i] = old ? atomicExch(&f.head[s], i + 1) : 0u;
+      atomicAdd(&f.count[s], 1u);
+      break;
+    }
+  }
+  __threadfence();
+  __syncthreads();
+  if (tid == 0) {
+    const uint64_t sums = __hip_atomic_load(&f.ctr[kListSums], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const uint64_t v[3] = {sums & ((1ull << 40) - 1), sums >> 40,
+                           __hip_atomic_load(&f.ctr[kListUnits], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)};
+    publish(sg, v, 3);
+  }
+}
+
+// Element idx (x) of the filter list of list l's entry j (e): the parents of
+// l with target x keep row (parent, j).
+__device__ __forceinline__ void list_element(const GraphView &g, uint64_t estart, const ListFilter &f, uint32_t l,
+                                             uint32_t j, uint32_t e, uint32_t off, uint32_t deg, uint32_t idx,
+                                             uint32_t x) {
+  const uint32_t h = pair_hash(l, x), b = pair_bits(h);
+  if ((f.bits[h >> (32 - f.blog2)] & b) != b) return;
+  for (uint32_t s = pair_slot(f, h);; s = (s + 1) & ((1u << f.log2) - 1)) {
+    const uint32_t hd = f.head[s];
+    if (!hd) return;
+    if (f.p_list[hd - 1] != l || f.p_tgt[hd - 1] != x) continue;
+    if (idx && g.edges[estart + off + idx - 1] == x) return;  // (only the first match counts)
+    const uint32_t n = f.count[s];
+    uint64_t k = atomicAdd(&f.ctr[kListKept], (unsigned long long)n);
+    atomicAdd(&f.ctr[kListSpared], (unsigned long long)n * (deg - (idx + 1)));
+    if (k + n <= f.cap)
+      for (uint32_t p = hd; p; p = f.next[p - 1])
+        f.kept[k++] = make_uint4((uint32_t)(f.excl[p - 1] + j), p - 1, e, 0u);
+    return;
+  }
+}
+
+__global__ __launch_bounds__(kBlock) void k_list_filter(GraphView g, ListFilter f, uint32_t total, uint32_t nl) {
+  constexpr int RD = kListTile / kBlock;
+  __shared__ WaveProbeLds s_wp[kBlock / kWave];
+  __shared__ uint64_t s_tmp[kBlock / kWave];
+  const uint32_t tid = threadIdx.x, lane = lane_id(), wave = tid / kWave;
+  const DevMeta ml = g.meta[f.lpid], m = g.meta[f.pid];
+  uint32_t l[RD], j[RD], e[RD], deg[RD], off[RD];
+  bool in[RD];
+#pragma unroll
+  for (int r = 0; r < RD; r++) {  // the entries and their lists
+    const uint32_t k0 = blockIdx.x * (uint32_t)kListTile + (wave * RD + r) * kWave, k = k0 + lane;
+    in[r] = k < total;
+    l[r] = j[r] = e[r] = 0;
+    if (k0 < total) {  // (wave-uniform)
+      const uint32_t l0 = (uint32_t)wave_last_le(nl, k0, [&](uint64_t i) -> uint64_t { return f.l_base[i]; });
+      uint32_t lo = l0, hi = nl - 1 < l0 + kWave ? nl - 1 : l0 + kWave;  // (every list has an entry)
+      if (l0 + 1 >= nl || f.l_base[l0 + 1] > k0 + kWave - 1) hi = l0;
+      while (lo < hi) {
+        const uint32_t mid = (lo + hi + 1) >> 1;
+        if (f.l_base[mid] <= k) lo = mid;
+        else hi = mid - 1;
+      }
+      l[r] = lo;
+      j[r] = k - f.l_base[lo];
+      if (in[r]) e[r] = g.edges[ml.edge_start + f.l_off[lo] + j[r]];
+    }
+  }
+  auto plan = [&](int r, uint64_t before63) {
+    return probe_plan<false, true>(g, m, in[r] && (int32_t)e[r] >= 0 ? make_key(e[r], f.pid, f.dir) : 0, before63);
+  };
+  ProbeCarry carry;
+  ProbePlan pl[3];
+  pl[0] = plan(0, 0);
+  if (RD > 1) pl[1] = plan(1, lane63_64(pl[0].key));
+  probe_pick<true>(g, pl[0]);
+#pragma unroll
+  for (int r = 0; r < RD; r++) {
+    if (r + 2 < RD) pl[(r + 2) % 3] = plan(r + 2, lane63_64(pl[(r + 1) % 3].key));
+    if (r + 1 < RD) probe_pick<true>(g, pl[(r + 1) % 3]);
+    (void)probe_finish<false, true>(g, m, pl[r % 3], s_wp[wave], deg[r], off[r], carry);
+  }
+  uint64_t ex = 0;
+  uint32_t x[RD];
+#pragma unroll
+  for (int r = 0; r < RD; r++) {
+    ex += deg[r] ? (uint64_t)deg[r] * f.l_np[l[r]] : 0;
+    x[r] = deg[r] && deg[r] <= kListInline ? g.edges[m.edge_start + off[r]] : 0u;
+  }
+#pragma unroll
+  for (int r = 0; r < RD; r++) {
+    if (deg[r] && deg[r] <= kListInline) list_element(g, m.edge_start, f, l[r], j[r], e[r], off[r], deg[r], 0, x[r]);
+    for (uint32_t q = 1; deg[r] <= kListInline && q < deg[r]; q += 3) {
+      uint32_t y[3];
+#pragma unroll
+      for (int u = 0; u < 3; u++) y[u] = q + u < deg[r] ? g.edges[m.edge_start + off[r] + q + u] : 0u;
+#pragma unroll
+      for (int u = 0; u < 3; u++)
+        if (q + u < deg[r]) list_element(g, m.edge_start, f, l[r], j[r], e[r], off[r], deg[r], q + u, y[u]);
+    }
+    if (deg[r] > kListInline) {
+      const uint32_t n = (deg[r] + kListChunk - 1) / kListChunk;
+      const uint64_t b = atomicAdd(&f.ctr[kListLongs], (unsigned long long)n);
+      for (uint32_t c = 0; c < n && b + c < f.long_cap; c++)
+        f.longs[b + c] = make_uint4(f.l_base[l[r]] + j[r], off[r], deg[r], c * kListChunk);
+    }
+  }
+  uint64_t sum;
+  (void)block_excl_scan(ex, s_tmp, sum);
+  if (tid == 0 && sum) atomicAdd(&f.ctr[kListEx], (unsigned long long)sum);
+}
+
+// The long filter lists, a chunk per workgroup at a time.
+__global__ __launch_bounds__(kBlock) void k_list_long(GraphView g, ListFilter f, uint32_t nl) {
+  const uint64_t all = f.ctr[kListLongs], n = all < f.long_cap ? all : f.long_cap;
+  const DevMeta ml = g.meta[f.lpid], m = g.meta[f.pid];
+  for (uint64_t i = blockIdx.x; i < n; i += gridDim.x) {
+    const uint4 it = f.longs[i];
+    const uint32_t l = (uint32_t)wave_last_le(nl, it.x, [&](uint64_t q) -> uint64_t { return f.l_base[q]; });
+    const uint32_t j = it.x - f.l_base[l], e = g.edges[ml.edge_start + f.l_off[l] + j];
+    uint32_t v[kListChunk / kBlock];
+#pragma unroll
+    for (int u = 0; u < (int)(kListChunk / kBlock); u++) {
+      const uint32_t q = it.w + threadIdx.x + u * kBlock;
+      v[u] = q < it.z ? g.edges[m.edge_start + it.y + q] : 0u;
+    }
+#pragma unroll
+    for (int u = 0; u < (int)(kListChunk / kBlock); u++) {
+      const uint32_t q = it.w + threadIdx.x + u * kBlock;
+      if (q < it.z) list_element(g, m.edge_start, f, l, j, e, it.y, it.z, q, v[u]);
+    }
+  }
+}
+
+// The n kept rows in row order: a thread counts the rows before its own, then
+// writes it (the parent's cells and the list entry).
+__global__ __launch_bounds__(kBlock) void k_list_rows(ListFilter f, uint32_t n, int32_t *O) {
+  __shared__ __align__(16) uint32_t s_row[kBlock * 4];
+  const uint32_t k = blockIdx.x * (uint32_t)kBlock + threadIdx.x;
+  const uint4 mine = k < n ? f.kept[k] : make_uint4(0, 0, 0, 0);
+  uint32_t rank = 0;
+  for (uint32_t b = 0; b < n; b += kBlock * 4) {
+    __syncthreads();
+    for (uint32_t i = threadIdx.x; i < kBlock * 4; i += kBlock) s_row[i] = b + i < n ? f.kept[b + i].x : 0xffffffffu;
+    __syncthreads();
+    if (k < n)
+      for (uint32_t i = 0; i < kBlock * 4; i += 4) {
+        const uint4 q = *(const uint4 *)&s_row[i];
+        rank += (q.x < mine.x) + (q.y < mine.x) + (q.z < mine.x) + (q.w < mine.x);
+      }
+  }
+  if (k >= n) return;
+  const int32_t *prow = f.P + (uint64_t)f.info[mine.y].x * f.pc;
+  int32_t *o = O + (uint64_t)rank * (f.pc + 1);
+  for (uint32_t c = 0; c < f.pc; c++) o[c] = prow[c];
+  o[f.pc] = (int32_t)mine.z;
 }
 
 // Compaction of the kept rows k_fanout_blocks listed: one thread per kept

@@ -1056,6 +1056,10 @@ int wkg_ctx::step_filter_fanout(int mode, const wkg_table *in, int pid, int dir,
   const uint64_t np = in->lin_n, R = in->rows;
   const int c = in->cols;
   if (np == 0 || np > kMaxParents) return kNotTaken;
+  if (sorted && fanout_blocks) {
+    const int lrc = step_filter_lists(mode, in, pid, dir, ec, cval, s, out, expanded);
+    if (lrc != kOtherForm) return lrc;
+  }
   // the compacted parents' lists: (offset, first child row) per parent
   std::vector<uint64_t> h((size_t)np * 2);
   {
@@ -1317,6 +1321,117 @@ int wkg_ctx::step_filter_fanout(int mode, const wkg_table *in, int pid, int dir,
   if (expanded) *expanded = examined;
   *out = t;
   t = nullptr;
+  return done(WKG_OK);
+}
+
+// step_filter_fanout's form for long shared lists of a sorted image with at
+// most kListKeptCap kept rows (kOtherForm: not so; kNotTaken: no form is
+// worth it): every distinct list entry is probed once and the elements of its
+// filter list are looked up among the targets of the list's parents. The
+// lists are deduplicated and the targets hashed on the device.
+int wkg_ctx::step_filter_lists(int mode, const wkg_table *in, int pid, int dir, int ec, int64_t cval, hipStream_t s,
+                               wkg_table **out, uint64_t *expanded) {
+  const uint64_t np = in->lin_n, R = in->rows;
+  int rc = ensure_pred(in->lin_pid, s);
+  if (rc) return rc;
+  auto log2_up = [](uint64_t n) {
+    uint32_t l = 1;
+    while ((1ull << l) < n) l++;
+    return l;
+  };
+  ListFilter f{};
+  f.info = in->lin_info;
+  f.excl = in->lin_excl;
+  f.np = np;
+  f.R = R;
+  f.P = in->lin_parent->d;
+  f.pc = (uint32_t)in->lin_parent->cols;
+  f.ec = mode == kModeK2K ? ec : -1;
+  f.target = (uint32_t)cval;
+  f.target_ok = (cval >= 0 && cval <= 0xffffffffLL) ? 1u : 0u;
+  f.lpid = (uint32_t)in->lin_pid;
+  f.pid = (uint32_t)pid;
+  f.dir = (uint32_t)dir;
+  f.log2 = log2_up(2 * np);
+  f.mask1 = (1u << f.log2) - 1;
+  f.blog2 = std::max(log2_up(np), 8u);  // 32 bits per parent
+  f.cap = std::min<uint64_t>(std::min<uint64_t>(R, fanout_kept_cap), kListKeptCap);
+  // counters | lists x 4, parents x 3 | two hash tables of two words a slot | bits
+  const uint64_t slots = 1ull << f.log2, words = 2 * kListCtrs + 7 * np + 4 * slots + (1ull << f.blog2);
+  uint32_t *buf = (uint32_t *)pool->alloc(words * 4, s, err_slot());
+  if (!buf) return WKG_ENOMEM;
+  uint32_t *w = buf;
+  auto take = [&](uint64_t n) {
+    uint32_t *r = w;
+    w += n;
+    return r;
+  };
+  f.ctr = (unsigned long long *)take(2 * kListCtrs);
+  f.l_off = take(np);
+  f.l_base = take(np);
+  f.l_len = take(np);
+  f.l_np = take(np);
+  f.p_list = take(np);
+  f.p_tgt = take(np);
+  f.next = take(np);
+  f.seen = take(slots);
+  f.seen_list = take(slots);
+  f.head = take(slots);
+  f.count = take(slots);
+  f.bits = take(1ull << f.blog2);
+  char *rows = nullptr;  // kept rows | long lists
+  auto done = [&](int r) {
+    if (rows) pool->release(rows, s);
+    pool->release(buf, s);
+    return r;
+  };
+  const Signal sg = next_signal();
+  {
+    ProfScope ps(this, s, "lineage", 40.0 * (double)np);
+    k_list_parents<<<1, 1024, 0, s>>>(f, sg);
+  }
+  hipError_t le = hipGetLastError();
+  if (le != hipSuccess) return done(fail(WKG_EDEVICE, "fan-out filter launch failed: %s", hipGetErrorString(le)));
+  if ((rc = wait_signal(sg, s))) return done(rc);
+  const uint64_t total = rb_host()[0], nl = rb_host()[1], units = rb_host()[2];
+  if (R < 4 * total) return done(kNotTaken);
+  if (units * 256 > R) return done(kOtherForm);  // short lists: their rows, tile by tile
+  f.long_cap = total / 16 + 65536;
+  rows = (char *)pool->alloc((f.cap + f.long_cap) * 16, s, err_slot());
+  if (!rows) return done(WKG_ENOMEM);
+  f.kept = (uint4 *)rows;
+  f.longs = f.kept + f.cap;
+  const GraphView g = view();
+  {
+    // per distinct entry: itself, its tag word and its bucket's line
+    ProfScope ps(this, s, "fanout_filter", 140.0 * (double)total);
+    k_list_filter<<<(unsigned)((total + kListTile - 1) / kListTile), kBlock, 0, s>>>(g, f, (uint32_t)total,
+                                                                                     (uint32_t)nl);
+    k_list_long<<<(unsigned)(4 * ncu), kBlock, 0, s>>>(g, f, (uint32_t)nl);
+  }
+  if ((le = hipGetLastError()) != hipSuccess)
+    return done(fail(WKG_EDEVICE, "fan-out filter launch failed: %s", hipGetErrorString(le)));
+  uint64_t c[kListCtrs];
+  if ((rc = read_words((const uint64_t *)f.ctr, kListCtrs, s, c))) return done(rc);
+  const uint64_t kept = c[kListKept];
+  if (kept > f.cap || c[kListLongs] > f.long_cap) return done(kOtherForm);
+  wkg_table *t = nullptr;
+  if ((rc = new_table(kept, in->cols, s, &t))) return done(rc);
+  if (kept) {
+    ProfScope ps(this, s, "compact", 8.0 * (double)kept * in->cols);
+    k_list_rows<<<(unsigned)((kept + kBlock - 1) / kBlock), kBlock, 0, s>>>(f, (uint32_t)kept, t->d);
+  }
+  if ((le = hipGetLastError()) != hipSuccess) {
+    drop_table(t);
+    return done(fail(WKG_EDEVICE, "fan-out compaction launch failed: %s", hipGetErrorString(le)));
+  }
+  prof_add_bytes("fanout_filters", 1.0);  // counts
+  prof_add_bytes("fanout_units", 1.0);
+  prof_add_bytes("fanout_parents", (double)np);  // sizes, summed over the filters
+  prof_add_bytes("fanout_lists", (double)nl);
+  prof_add_bytes("fanout_list_entries", (double)total);
+  if (expanded) *expanded = c[kListEx] - c[kListSpared];
+  *out = t;
   return done(WKG_OK);
 }
 

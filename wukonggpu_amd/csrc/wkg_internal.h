@@ -96,6 +96,7 @@ struct wkg_table {
 // Returned by a specialised step path that declined the step (nothing was
 // done; the general path runs it). Positive, so never a WKG_* status.
 constexpr int kNotTaken = 1;
+constexpr int kOtherForm = 2;  // ... declined by one form of it: another form may take it
 
 // One step's probe, tile scan and compaction (wkg_ctx::probe_pass).
 struct ProbePass {
@@ -266,6 +267,8 @@ struct wkg_ctx {
   void keep_lineage(const wkg_table *in, ProbePass &pp, uint64_t nz, wkg_table *t, int pid);
   int step_filter_fanout(int mode, const wkg_table *in, int pid, int dir, int ec, int64_t cval, hipStream_t s,
                          wkg_table **out, uint64_t *expanded);
+  int step_filter_lists(int mode, const wkg_table *in, int pid, int dir, int ec, int64_t cval, hipStream_t s,
+                        wkg_table **out, uint64_t *expanded);
   int step_k2u_lineage(const wkg_table *in, int sc, int pid, int dir, hipStream_t s, wkg_table **out,
                        uint64_t *expanded);
   int step_filter_groups(int mode, const wkg_table *in, int pid, int dir, int ec, int64_t cval, hipStream_t s,
