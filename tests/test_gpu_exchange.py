@@ -81,6 +81,16 @@ def test_concat_edges(dev_small):
         dev_small.table_concat([dev_small.table(a), dev_small.table(_table(rng, 2, 3))])
 
 
+@pytest.mark.parametrize("cols", [1, 3, 4, 5])
+def test_concat_part_sizes(dev_small, cols):
+    # parts of no whole quad, one, several workgroups, at every alignment; more than one launch's parts
+    rng = np.random.default_rng(cols)
+    sizes = [1, 0, 2, 3, 4, 5, 8191, 8192, 1, 8193, 30001] + [int(x) for x in rng.integers(0, 9, 150)]
+    parts = [_table(rng, n, cols) for n in sizes]
+    got = dev_small.table_concat([dev_small.table(p) for p in parts]).to_host()
+    assert np.array_equal(got, np.vstack(parts))
+
+
 def test_split_bad_arguments(dev_small):
     d = dev_small.table(np.ones((4, 2), dtype=np.int32))
     for col, n in ((2, 4), (-1, 4), (0, 0), (0, 1025)):

@@ -2088,7 +2088,7 @@ __global__ __launch_bounds__(kBlock) void k_fanout_blocks(GraphView g, StepParam
 // unordered and ranked by their row (k_list_rows).
 // What bounds it: the probe of the distinct entries (cache misses); nearly
 // all lookups end at a bit of a filter in L1. The cycle's closing filter over
-// 1.9G pairs of 1.6M distinct entries: its query 618 -> 285 us (pair by pair in
+// 1.9G pairs of 1.6M distinct entries: its query 618 -> 205 us (pair by pair in
 // k_fanout_blocks 256 us, on top of the probe's 46 us, its passes' 40 us, and
 // 150 us of lists gathered on the host).
 struct ListFilter {
@@ -2110,14 +2110,20 @@ struct ListFilter {
   unsigned long long *ctr;            // kList*
   uint4 *kept;                        // (row, parent, entry, 0)
   uint64_t cap;
-  uint4 *longs;                       // (entry, offset, degree, first element)
+  uint64_t *ex;                       // per wave of k_list_filter: its share of the work count
+  // long filter lists in kListQueues queues of long_cap items (a workgroup
+  // appends to one of them: thousands of workgroups adding to one word take
+  // 17 ns each): (entry, offset, degree, first element)
+  uint4 *longs;
+  unsigned long long *long_n;         // per queue, kListPad words apart
   uint64_t long_cap;
 };
-enum { kListSums = 0, kListUnits, kListKept, kListEx, kListSpared, kListLongs, kListCtrs };
+enum { kListSums = 0, kListUnits, kListKept, kListEx, kListSpared, kListLost, kListCtrs };
+constexpr uint32_t kListQueues = 64, kListPad = 16;
 constexpr uint32_t kNoList = 0xffffffffu;  // (segments hold fewer than 2^32 edges)
 constexpr uint32_t kListInline = 16;       // longer filter lists go to k_list_long,
 constexpr uint32_t kListChunk = 1024;      // this many elements an item
-constexpr int kListTile = 1024;            // list entries per workgroup
+constexpr int kListTile = 512;             // list entries per workgroup
 constexpr uint64_t kListKeptCap = 32768;   // ranking compares all kept rows with each other
 
 __device__ __forceinline__ uint32_t pair_hash(uint32_t l, uint32_t t) {
@@ -2130,13 +2136,31 @@ __device__ __forceinline__ uint32_t pair_bits(uint32_t h) { return (1u << (h & 3
 
 // The distinct lists and the parents' targets, by one workgroup (its phases
 // are separated by barriers; words changed by atomics are read as atomics).
-__global__ __launch_bounds__(1024) void k_list_parents(ListFilter f, Signal sg) {
-  const uint32_t tid = threadIdx.x, np = (uint32_t)f.np;
+// Up to kListLds parents the hash tables are built in LDS and copied out: the
+// parents of a popular list all meet at its words, which serialises in memory
+// (800 parents: 54 us, in LDS 31 us).
+constexpr uint32_t kListLds = 2048;
+__global__ __launch_bounds__(1024) void k_list_parents(ListFilter fg, Signal sg) {
+  __shared__ uint32_t s_tab[(4 * 2 + 2) * kListLds];  // seen, seen_list, head, count: two slots a parent; l_np, bits
+  __shared__ unsigned long long s_ctr[kListCtrs];
+  const uint32_t tid = threadIdx.x, np = (uint32_t)fg.np;
+  ListFilter f = fg;
+  const bool lds = np <= kListLds;
+  if (lds) {
+    f.seen = s_tab;
+    f.seen_list = s_tab + 2 * kListLds;
+    f.head = s_tab + 4 * kListLds;
+    f.count = s_tab + 6 * kListLds;
+    f.l_np = s_tab + 8 * kListLds;
+    f.bits = s_tab + 9 * kListLds;
+    f.ctr = s_ctr;
+  }
   for (uint32_t i = tid; i <= f.mask1; i += 1024) f.seen[i] = kNoList;
   for (uint32_t i = tid; i < 1u << f.log2; i += 1024) f.head[i] = f.count[i] = 0;
   for (uint32_t i = tid; i < 1u << f.blog2; i += 1024) f.bits[i] = 0;
   for (uint32_t i = tid; i < np; i += 1024) f.l_np[i] = 0;
   if (tid < kListCtrs) f.ctr[tid] = 0;
+  if (tid < kListQueues) f.long_n[tid * kListPad] = 0;
   __threadfence();
   __syncthreads();
   uint64_t units = 0;
@@ -2187,6 +2211,15 @@ __global__ __launch_bounds__(1024) void k_list_parents(ListFilter f, Signal sg) 
   }
   __threadfence();
   __syncthreads();
+  if (lds) {
+    for (uint32_t i = tid; i < 1u << f.log2; i += 1024) {
+      fg.head[i] = f.head[i];
+      fg.count[i] = f.count[i];
+    }
+    for (uint32_t i = tid; i < 1u << f.blog2; i += 1024) fg.bits[i] = f.bits[i];
+    for (uint32_t i = tid; i < np; i += 1024) fg.l_np[i] = f.l_np[i];
+    if (tid < kListCtrs) fg.ctr[tid] = f.ctr[tid];
+  }
   if (tid == 0) {
     const uint64_t sums = __hip_atomic_load(&f.ctr[kListSums], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     const uint64_t v[3] = {sums & ((1ull << 40) - 1), sums >> 40,
@@ -2220,28 +2253,39 @@ __device__ __forceinline__ void list_element(const GraphView &g, uint64_t estart
 __global__ __launch_bounds__(kBlock) void k_list_filter(GraphView g, ListFilter f, uint32_t total, uint32_t nl) {
   constexpr int RD = kListTile / kBlock;
   __shared__ WaveProbeLds s_wp[kBlock / kWave];
-  __shared__ uint64_t s_tmp[kBlock / kWave];
-  const uint32_t tid = threadIdx.x, lane = lane_id(), wave = tid / kWave;
+  const uint32_t lane = lane_id(), wave = threadIdx.x / kWave;
   const DevMeta ml = g.meta[f.lpid], m = g.meta[f.pid];
   uint32_t l[RD], j[RD], e[RD], deg[RD], off[RD];
   bool in[RD];
+  {
+    const uint32_t w0 = blockIdx.x * (uint32_t)kListTile + wave * RD * kWave;
+    if (w0 >= total) {  // (waves are independent: no barrier below)
+      if (lane == 0) f.ex[blockIdx.x * (kBlock / kWave) + wave] = 0;
+      return;
+    }
+    // the wave's first list, and whether all its rows are in it
+    const uint32_t l0 = (uint32_t)wave_last_le(nl, w0, [&](uint64_t i) -> uint64_t { return f.l_base[i]; });
+    const uint32_t b0 = f.l_base[l0], o0 = f.l_off[l0];
+    const bool one = l0 + 1 >= nl || f.l_base[l0 + 1] >= w0 + RD * kWave;
+    const uint32_t most = nl - 1 < l0 + RD * kWave ? nl - 1 : l0 + RD * kWave;  // (every list has an entry)
 #pragma unroll
-  for (int r = 0; r < RD; r++) {  // the entries and their lists
-    const uint32_t k0 = blockIdx.x * (uint32_t)kListTile + (wave * RD + r) * kWave, k = k0 + lane;
-    in[r] = k < total;
-    l[r] = j[r] = e[r] = 0;
-    if (k0 < total) {  // (wave-uniform)
-      const uint32_t l0 = (uint32_t)wave_last_le(nl, k0, [&](uint64_t i) -> uint64_t { return f.l_base[i]; });
-      uint32_t lo = l0, hi = nl - 1 < l0 + kWave ? nl - 1 : l0 + kWave;  // (every list has an entry)
-      if (l0 + 1 >= nl || f.l_base[l0 + 1] > k0 + kWave - 1) hi = l0;
-      while (lo < hi) {
-        const uint32_t mid = (lo + hi + 1) >> 1;
-        if (f.l_base[mid] <= k) lo = mid;
-        else hi = mid - 1;
+    for (int r = 0; r < RD; r++) {
+      const uint32_t k = w0 + r * kWave + lane;
+      in[r] = k < total;
+      uint32_t lo = l0, base = b0, o = o0;
+      if (!one) {
+        uint32_t hi = most;
+        while (lo < hi) {
+          const uint32_t mid = (lo + hi + 1) >> 1;
+          if (f.l_base[mid] <= k) lo = mid;
+          else hi = mid - 1;
+        }
+        base = f.l_base[lo];
+        o = f.l_off[lo];
       }
       l[r] = lo;
-      j[r] = k - f.l_base[lo];
-      if (in[r]) e[r] = g.edges[ml.edge_start + f.l_off[lo] + j[r]];
+      j[r] = k - base;
+      e[r] = in[r] ? g.edges[ml.edge_start + o + j[r]] : 0u;
     }
   }
   auto plan = [&](int r, uint64_t before63) {
@@ -2268,32 +2312,56 @@ __global__ __launch_bounds__(kBlock) void k_list_filter(GraphView g, ListFilter 
 #pragma unroll
   for (int r = 0; r < RD; r++) {
     if (deg[r] && deg[r] <= kListInline) list_element(g, m.edge_start, f, l[r], j[r], e[r], off[r], deg[r], 0, x[r]);
-    for (uint32_t q = 1; deg[r] <= kListInline && q < deg[r]; q += 3) {
-      uint32_t y[3];
+    // the further elements of all lanes' lists as one sequence, a lane each
+    const uint32_t more = deg[r] > 1 && deg[r] <= kListInline ? deg[r] - 1 : 0u;
+    if (wave_ballot(more != 0)) {
+      uint32_t inc = more;
 #pragma unroll
-      for (int u = 0; u < 3; u++) y[u] = q + u < deg[r] ? g.edges[m.edge_start + off[r] + q + u] : 0u;
+      for (int d = 1; d < kWave; d <<= 1) {
+        const uint32_t y = shfl32(inc, (lane - d) & 63);
+        if (lane >= (uint32_t)d) inc += y;
+      }
+      const uint32_t all = lane63(inc), before = inc - more;
+      for (uint32_t t0 = 0; t0 < all; t0 += kWave) {  // (wave-uniform)
+        const uint32_t t = t0 + lane;
+        uint32_t src = 0;  // the last lane whose elements start at or before t (lanes without any share their next's)
 #pragma unroll
-      for (int u = 0; u < 3; u++)
-        if (q + u < deg[r]) list_element(g, m.edge_start, f, l[r], j[r], e[r], off[r], deg[r], q + u, y[u]);
+        for (uint32_t step = kWave / 2; step; step >>= 1)
+          if (shfl32(before, src + step) <= t) src += step;
+        const uint32_t q = t - shfl32(before, src) + 1, ol = shfl32(l[r], src), oo = shfl32(off[r], src);
+        const uint32_t od = shfl32(deg[r], src), oj = shfl32(j[r], src), oe = shfl32(e[r], src);
+        if (t < all) list_element(g, m.edge_start, f, ol, oj, oe, oo, od, q, g.edges[m.edge_start + oo + q]);
+      }
     }
     if (deg[r] > kListInline) {
       const uint32_t n = (deg[r] + kListChunk - 1) / kListChunk;
-      const uint64_t b = atomicAdd(&f.ctr[kListLongs], (unsigned long long)n);
+      const uint32_t q = blockIdx.x % kListQueues;
+      const uint64_t b = atomicAdd(&f.long_n[q * kListPad], (unsigned long long)n);
       for (uint32_t c = 0; c < n && b + c < f.long_cap; c++)
-        f.longs[b + c] = make_uint4(f.l_base[l[r]] + j[r], off[r], deg[r], c * kListChunk);
+        f.longs[q * f.long_cap + b + c] = make_uint4(f.l_base[l[r]] + j[r], off[r], deg[r], c * kListChunk);
     }
   }
-  uint64_t sum;
-  (void)block_excl_scan(ex, s_tmp, sum);
-  if (tid == 0 && sum) atomicAdd(&f.ctr[kListEx], (unsigned long long)sum);
+  ex = lane63_64(wave_incl_scan(ex));
+  if (lane == 0) f.ex[blockIdx.x * (kBlock / kWave) + wave] = ex;
 }
 
-// The long filter lists, a chunk per workgroup at a time.
-__global__ __launch_bounds__(kBlock) void k_list_long(GraphView g, ListFilter f, uint32_t nl) {
-  const uint64_t all = f.ctr[kListLongs], n = all < f.long_cap ? all : f.long_cap;
+// The long filter lists, a chunk per workgroup at a time; the first workgroup
+// also adds up the work count.
+__global__ __launch_bounds__(kBlock) void k_list_long(GraphView g, ListFilter f, uint32_t nl, uint32_t nex) {
+  const uint32_t queue = blockIdx.x % kListQueues;
+  const uint64_t all = f.long_n[queue * kListPad], n = all < f.long_cap ? all : f.long_cap;
+  if (all > n && threadIdx.x == 0) f.ctr[kListLost] = 1;
+  if (blockIdx.x == 0) {
+    __shared__ uint64_t s_tmp[kBlock / kWave];
+    uint64_t v = 0, sum;
+#pragma unroll 8
+    for (uint32_t i = threadIdx.x; i < nex; i += kBlock) v += f.ex[i];
+    (void)block_excl_scan(v, s_tmp, sum);
+    if (threadIdx.x == 0) f.ctr[kListEx] = sum;
+  }
   const DevMeta ml = g.meta[f.lpid], m = g.meta[f.pid];
-  for (uint64_t i = blockIdx.x; i < n; i += gridDim.x) {
-    const uint4 it = f.longs[i];
+  for (uint64_t i = blockIdx.x / kListQueues; i < n; i += gridDim.x / kListQueues) {
+    const uint4 it = f.longs[queue * f.long_cap + i];
     const uint32_t l = (uint32_t)wave_last_le(nl, it.x, [&](uint64_t q) -> uint64_t { return f.l_base[q]; });
     const uint32_t j = it.x - f.l_base[l], e = g.edges[ml.edge_start + f.l_off[l] + j];
     uint32_t v[kListChunk / kBlock];
@@ -2310,28 +2378,31 @@ __global__ __launch_bounds__(kBlock) void k_list_long(GraphView g, ListFilter f,
   }
 }
 
-// The n kept rows in row order: a thread counts the rows before its own, then
-// writes it (the parent's cells and the list entry).
+// The n kept rows in row order: the 16 lanes of a group count the rows before
+// their own, then write it (the parent's cells and the list entry).
+constexpr uint32_t kRankLanes = 16;
 __global__ __launch_bounds__(kBlock) void k_list_rows(ListFilter f, uint32_t n, int32_t *O) {
-  __shared__ __align__(16) uint32_t s_row[kBlock * 4];
-  const uint32_t k = blockIdx.x * (uint32_t)kBlock + threadIdx.x;
+  constexpr uint32_t kTile = kBlock * 4;
+  __shared__ __align__(16) uint32_t s_row[kTile];
+  const uint32_t k = blockIdx.x * (kBlock / kRankLanes) + threadIdx.x / kRankLanes, g16 = threadIdx.x % kRankLanes;
   const uint4 mine = k < n ? f.kept[k] : make_uint4(0, 0, 0, 0);
   uint32_t rank = 0;
-  for (uint32_t b = 0; b < n; b += kBlock * 4) {
+  for (uint32_t b = 0; b < n; b += kTile) {
     __syncthreads();
-    for (uint32_t i = threadIdx.x; i < kBlock * 4; i += kBlock) s_row[i] = b + i < n ? f.kept[b + i].x : 0xffffffffu;
+    for (uint32_t i = threadIdx.x; i < kTile; i += kBlock) s_row[i] = b + i < n ? f.kept[b + i].x : 0xffffffffu;
     __syncthreads();
-    if (k < n)
-      for (uint32_t i = 0; i < kBlock * 4; i += 4) {
-        const uint4 q = *(const uint4 *)&s_row[i];
-        rank += (q.x < mine.x) + (q.y < mine.x) + (q.z < mine.x) + (q.w < mine.x);
-      }
+    for (uint32_t i = g16 * 4; i < kTile; i += kRankLanes * 4) {
+      const uint4 q = *(const uint4 *)&s_row[i];
+      rank += (q.x < mine.x) + (q.y < mine.x) + (q.z < mine.x) + (q.w < mine.x);
+    }
   }
+#pragma unroll
+  for (uint32_t d = kRankLanes / 2; d; d >>= 1) rank += shfl32(rank, lane_id() ^ d);
   if (k >= n) return;
   const int32_t *prow = f.P + (uint64_t)f.info[mine.y].x * f.pc;
   int32_t *o = O + (uint64_t)rank * (f.pc + 1);
-  for (uint32_t c = 0; c < f.pc; c++) o[c] = prow[c];
-  o[f.pc] = (int32_t)mine.z;
+  for (uint32_t c = g16; c < f.pc; c += kRankLanes) o[c] = prow[c];
+  if (g16 == 0) o[f.pc] = (int32_t)mine.z;
 }
 
 // Compaction of the kept rows k_fanout_blocks listed: one thread per kept

@@ -1357,7 +1357,8 @@ int wkg_ctx::step_filter_lists(int mode, const wkg_table *in, int pid, int dir, 
   f.blog2 = std::max(log2_up(np), 8u);  // 32 bits per parent
   f.cap = std::min<uint64_t>(std::min<uint64_t>(R, fanout_kept_cap), kListKeptCap);
   // counters | lists x 4, parents x 3 | two hash tables of two words a slot | bits
-  const uint64_t slots = 1ull << f.log2, words = 2 * kListCtrs + 7 * np + 4 * slots + (1ull << f.blog2);
+  const uint64_t slots = 1ull << f.log2;
+  const uint64_t words = 2 * kListCtrs + 2 * kListQueues * kListPad + 7 * np + 4 * slots + (1ull << f.blog2);
   uint32_t *buf = (uint32_t *)pool->alloc(words * 4, s, err_slot());
   if (!buf) return WKG_ENOMEM;
   uint32_t *w = buf;
@@ -1367,6 +1368,7 @@ int wkg_ctx::step_filter_lists(int mode, const wkg_table *in, int pid, int dir, 
     return r;
   };
   f.ctr = (unsigned long long *)take(2 * kListCtrs);
+  f.long_n = (unsigned long long *)take(2 * kListQueues * kListPad);
   f.l_off = take(np);
   f.l_base = take(np);
   f.l_len = take(np);
@@ -1396,30 +1398,32 @@ int wkg_ctx::step_filter_lists(int mode, const wkg_table *in, int pid, int dir, 
   const uint64_t total = rb_host()[0], nl = rb_host()[1], units = rb_host()[2];
   if (R < 4 * total) return done(kNotTaken);
   if (units * 256 > R) return done(kOtherForm);  // short lists: their rows, tile by tile
-  f.long_cap = total / 16 + 65536;
-  rows = (char *)pool->alloc((f.cap + f.long_cap) * 16, s, err_slot());
+  f.long_cap = (total / 16 + 65536) / kListQueues;
+  const uint64_t nwg = (total + kListTile - 1) / kListTile, nex = nwg * (kBlock / kWave);
+  rows = (char *)pool->alloc((f.cap + kListQueues * f.long_cap) * 16 + nex * 8, s, err_slot());
   if (!rows) return done(WKG_ENOMEM);
   f.kept = (uint4 *)rows;
   f.longs = f.kept + f.cap;
+  f.ex = (uint64_t *)(f.longs + kListQueues * f.long_cap);
   const GraphView g = view();
   {
     // per distinct entry: itself, its tag word and its bucket's line
     ProfScope ps(this, s, "fanout_filter", 140.0 * (double)total);
-    k_list_filter<<<(unsigned)((total + kListTile - 1) / kListTile), kBlock, 0, s>>>(g, f, (uint32_t)total,
-                                                                                     (uint32_t)nl);
-    k_list_long<<<(unsigned)(4 * ncu), kBlock, 0, s>>>(g, f, (uint32_t)nl);
+    k_list_filter<<<(unsigned)nwg, kBlock, 0, s>>>(g, f, (uint32_t)total, (uint32_t)nl);
+    k_list_long<<<16 * kListQueues, kBlock, 0, s>>>(g, f, (uint32_t)nl, (uint32_t)nex);
   }
   if ((le = hipGetLastError()) != hipSuccess)
     return done(fail(WKG_EDEVICE, "fan-out filter launch failed: %s", hipGetErrorString(le)));
   uint64_t c[kListCtrs];
   if ((rc = read_words((const uint64_t *)f.ctr, kListCtrs, s, c))) return done(rc);
   const uint64_t kept = c[kListKept];
-  if (kept > f.cap || c[kListLongs] > f.long_cap) return done(kOtherForm);
+  if (kept > f.cap || c[kListLost]) return done(kOtherForm);
   wkg_table *t = nullptr;
   if ((rc = new_table(kept, in->cols, s, &t))) return done(rc);
   if (kept) {
     ProfScope ps(this, s, "compact", 8.0 * (double)kept * in->cols);
-    k_list_rows<<<(unsigned)((kept + kBlock - 1) / kBlock), kBlock, 0, s>>>(f, (uint32_t)kept, t->d);
+    constexpr uint64_t per = kBlock / kRankLanes;
+    k_list_rows<<<(unsigned)((kept + per - 1) / per), kBlock, 0, s>>>(f, (uint32_t)kept, t->d);
   }
   if ((le = hipGetLastError()) != hipSuccess) {
     drop_table(t);
