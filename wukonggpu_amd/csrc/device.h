@@ -259,12 +259,76 @@ __device__ __forceinline__ void probe_pick(const GraphView &g, ProbePlan &r) {
   }
 }
 
+// A leader's (degree, offset) from its picked slot; false: it must walk.
+template <bool TAGS>
+__device__ __forceinline__ bool probe_slot(const GraphView &g, const DevMeta &m, const ProbePlan &pl, uint32_t &deg,
+                                           uint32_t &off) {
+  deg = off = 0;
+  if (TAGS && g.tags && pl.tag) {
+    if (pl.slot.x != (uint32_t)pl.key || pl.slot.y != (uint32_t)(pl.key >> 32)) return false;  // another key's tag
+    const uint64_t v = ((uint64_t)pl.slot.w << 32) | pl.slot.z;
+    deg = (uint32_t)ptr_size(v);
+    off = (uint32_t)(ptr_off(v) - m.edge_start);
+  }
+  return !pl.walk;
+}
+
+// Walks the n (at most 64) pending entries kb -- (key low, key high, bucket,
+// id) -- with U bucket reads in flight per lane; put(id, degree, offset) gets
+// each one's result. kb is rewritten.
+template <bool FRAMED, int U, class F>
+__device__ __forceinline__ void walk_pending(const GraphView &g, const DevMeta &m, uint4 *kb, uint32_t n, F put) {
+  const uint32_t lane = lane_id(), l8 = lane & 7, grp = lane >> 3, gbase = lane & ~7u;
+  const uint64_t below = lanes_below();
+  for (uint32_t hop = 0; n; hop++) {
+    uint32_t nn = 0;
+    for (uint32_t k0 = 0; k0 < n; k0 += 8 * U) {
+      uint4 e[U], sl[U];
+#pragma unroll
+      for (int u = 0; u < U; u++) {
+        e[u] = make_uint4(0, 0, 0, 0);
+        sl[u] = make_uint4(0, 0, 0, 0);
+        if (k0 + grp + 8u * u < n) {
+          e[u] = kb[k0 + grp + 8u * u];
+          sl[u] = g.slots[(uint64_t)e[u].z * kAssoc + l8];
+        }
+      }
+      // (these pending entries are read above before any is rewritten
+      // below -- at most as many are appended as were read, and a wave's
+      // LDS operations complete in order)
+#pragma unroll
+      for (int u = 0; u < U; u++) {
+        if (k0 + 8u * u >= n) break;  // wave-uniform
+        const bool in = k0 + grp + 8u * u < n;
+        const bool hit = in && l8 < 7 && sl[u].x == e[u].x && sl[u].y == e[u].y;
+        if (hit) {
+          const uint64_t v = ((uint64_t)sl[u].w << 32) | sl[u].z;
+          put(e[u].w, (uint32_t)ptr_size(v), (uint32_t)(ptr_off(v) - m.edge_start));
+        }
+        const uint32_t gb = (uint32_t)(wave_ballot(hit) >> gbase) & 0x7fu;
+        const uint64_t link = ((uint64_t)sl[u].y << 32) | sl[u].x;
+        const bool tail = in && l8 == 7 && gb == 0;  // lane 7 of a group without a match
+        const bool follow = tail && link != 0 && hop + 1 < kMaxHops;
+        if (tail && !follow) put(e[u].w, 0u, 0u);
+        const uint64_t fb = wave_ballot(follow);
+        if (follow) {
+          const uint64_t nb = key_vid(link);
+          const uint64_t bkt = FRAMED ? bucket_phys<true>(g, m, nb - m.indrct_start + m.psz) : nb;
+          kb[nn + (uint32_t)__builtin_popcountll(fb & below)] = make_uint4(e[u].x, e[u].y, (uint32_t)bkt, e[u].w);
+        }
+        nn += (uint32_t)__builtin_popcountll(fb);
+      }
+    }
+    __builtin_amdgcn_wave_barrier();
+    n = nn;
+  }
+}
+
 template <bool FRAMED, bool TAGS>
 __device__ __forceinline__ uint32_t probe_finish(const GraphView &g, const DevMeta &m, const ProbePlan &pl,
                                                  WaveProbeLds &w, uint32_t &deg_out, uint32_t &off_out,
                                                  ProbeCarry &carry) {
-  constexpr int U = TAGS ? 2 : 8;  // bucket reads in flight per lane
-  const uint32_t lane = lane_id(), l8 = lane & 7, grp = lane >> 3, gbase = lane & ~7u;
+  const uint32_t lane = lane_id();
   const bool valid = pl.key != 0;
   const uint64_t leaders = pl.leaders;
   if (leaders == 0) {  // every valid lane continues the carried run (wave-uniform)
@@ -274,68 +338,16 @@ __device__ __forceinline__ uint32_t probe_finish(const GraphView &g, const DevMe
     return 0;
   }
   const uint64_t below = lanes_below();
-  const uint32_t klo = (uint32_t)pl.key, khi = (uint32_t)(pl.key >> 32);
-  uint32_t deg = 0, off = 0;
-  bool walk = pl.walk;
-  if constexpr (TAGS) {
-    if (g.tags && pl.tag) {
-      if (pl.slot.x == klo && pl.slot.y == khi) {
-        const uint64_t v = ((uint64_t)pl.slot.w << 32) | pl.slot.z;
-        deg = (uint32_t)ptr_size(v);
-        off = (uint32_t)(ptr_off(v) - m.edge_start);
-      } else {
-        walk = true;  // another key with this tag
-      }
-    }
-  }
+  uint32_t deg, off;
+  const bool walk = !probe_slot<TAGS>(g, m, pl, deg, off);
   const uint64_t walkers = wave_ballot(walk);
   if (walkers) {
-    if (walk) w.kb[__builtin_popcountll(walkers & below)] = make_uint4(klo, khi, pl.bucket, lane);
+    if (walk)
+      w.kb[__builtin_popcountll(walkers & below)] =
+          make_uint4((uint32_t)pl.key, (uint32_t)(pl.key >> 32), pl.bucket, lane);
     __builtin_amdgcn_wave_barrier();
-    uint32_t n = (uint32_t)__builtin_popcountll(walkers);  // pending walks (wave-uniform)
-    for (uint32_t hop = 0; n; hop++) {
-      uint32_t nn = 0;
-      for (uint32_t k0 = 0; k0 < n; k0 += 8 * U) {
-        uint4 e[U], sl[U];
-#pragma unroll
-        for (int u = 0; u < U; u++) {
-          e[u] = make_uint4(0, 0, 0, 0);
-          sl[u] = make_uint4(0, 0, 0, 0);
-          if (k0 + grp + 8u * u < n) {
-            e[u] = w.kb[k0 + grp + 8u * u];
-            sl[u] = g.slots[(uint64_t)e[u].z * kAssoc + l8];
-          }
-        }
-        // (these pending entries are read above before any is rewritten
-        // below -- at most as many are appended as were read, and a wave's
-        // LDS operations complete in order)
-#pragma unroll
-        for (int u = 0; u < U; u++) {
-          if (k0 + 8u * u >= n) break;  // wave-uniform
-          const bool in = k0 + grp + 8u * u < n;
-          const bool hit = in && l8 < 7 && sl[u].x == e[u].x && sl[u].y == e[u].y;
-          if (hit) {
-            const uint64_t v = ((uint64_t)sl[u].w << 32) | sl[u].z;
-            w.res[e[u].w] = make_uint2((uint32_t)ptr_size(v), (uint32_t)(ptr_off(v) - m.edge_start));
-          }
-          const uint32_t gb = (uint32_t)(wave_ballot(hit) >> gbase) & 0x7fu;
-          const uint64_t link = ((uint64_t)sl[u].y << 32) | sl[u].x;
-          const bool tail = in && l8 == 7 && gb == 0;  // lane 7 of a group without a match
-          const bool follow = tail && link != 0 && hop + 1 < kMaxHops;
-          if (tail && !follow) w.res[e[u].w] = make_uint2(0u, 0u);
-          const uint64_t fb = wave_ballot(follow);
-          if (follow) {
-            const uint64_t nb = key_vid(link);
-            const uint64_t bkt = FRAMED ? bucket_phys<true>(g, m, nb - m.indrct_start + m.psz) : nb;
-            w.kb[nn + (uint32_t)__builtin_popcountll(fb & below)] =
-                make_uint4(e[u].x, e[u].y, (uint32_t)bkt, e[u].w);
-          }
-          nn += (uint32_t)__builtin_popcountll(fb);
-        }
-      }
-      __builtin_amdgcn_wave_barrier();
-      n = nn;
-    }
+    walk_pending<FRAMED, TAGS ? 2 : 8>(g, m, w.kb, (uint32_t)__builtin_popcountll(walkers),
+                                       [&](uint32_t id, uint32_t d, uint32_t o) { w.res[id] = make_uint2(d, o); });
     if (walk) {
       const uint2 r = w.res[lane];
       deg = r.x;

@@ -553,20 +553,66 @@ __device__ __forceinline__ void x_probe_tile(const ExecArgs &a, uint32_t q, uint
   }
 }
 
+// The static deal of 1024-row tiles: a workgroup's tiles are a chain of
+// reads each (the tile's query, its record, the rows, tags, slots), so the
+// query search runs on a copy of the tile bases in LDS and the next tile's
+// record is on its way while this one is probed. @@X1@@
+constexpr uint32_t kBaseLds = 1024;
+template <bool SORTED, bool FRAMED>
+__device__ __forceinline__ void x_probe_deal(const ExecArgs &a, uint32_t nq) {
+  constexpr uint32_t kWords = sizeof(StepParams) / 8;
+  static_assert(sizeof(StepParams) % 8 == 0 && kWords <= kBlock, "the record is copied in 8-byte words");
+  __shared__ uint64_t s_pw[kWords];
+  __shared__ uint64_t s_base[kBaseLds + 1];
+  const uint32_t tid = threadIdx.x;
+  const uint64_t n = a.st->nt;
+  uint64_t t = blockIdx.x;
+  if (t >= n) return;
+  const bool staged = nq <= kBaseLds;
+  if (staged) {
+    for (uint32_t i = tid; i <= nq; i += kBlock) s_base[i] = a.tile_base[i];
+    __syncthreads();
+  }
+  const uint64_t *base = staged ? s_base : a.tile_base;
+  uint32_t q = wave_find(base, nq, t);
+  uint64_t qlo = base[q], qhi = base[q + 1], word = 0;
+  if (tid < kWords) word = gmem((const uint64_t *)&a.items[q].p)[tid];
+  while (t < n) {
+    const uint64_t lt = t - qlo;
+    __syncthreads();  // the previous tile's LDS use is over
+    if (tid < kWords) s_pw[tid] = word;
+    t += gridDim.x;
+    if (t < n) {
+      if (t >= qhi) {  // block-uniform
+        q = wave_find(base, nq, t);
+        qlo = base[q];
+        qhi = base[q + 1];
+      }
+      if (tid < kWords) word = gmem((const uint64_t *)&a.items[q].p)[tid];
+    }
+    __syncthreads();
+    probe_tile<1024, SORTED, FRAMED>(a.g, *(const StepParams *)s_pw, lt);
+  }
+}
+
 template <int TR, bool SORTED, bool FRAMED, bool QUEUE>
 __global__ __launch_bounds__(kBlock, TR == 1024 ? 4 : 3) void k_x_probe(ExecArgs a) {
-  __shared__ uint64_t s_pw[sizeof(StepParams) / 8];
   const uint32_t nq = (uint32_t)a.st->nq;
-  uint64_t t, lt;
-  uint32_t q;
-  if constexpr (QUEUE) {
-    __shared__ QueueLds s_wq;
-    BlockQueue wq(s_wq, a.st->queue[0], a.st->nt);
-    while (wq.next(a.tile_base, nq, t, q, lt)) x_probe_tile<TR, SORTED, FRAMED>(a, q, lt, s_pw);
+  if constexpr (TR == 1024 && !QUEUE) {
+    x_probe_deal<SORTED, FRAMED>(a, nq);
   } else {
-    __shared__ uint32_t s_q;
-    StaticDeal wd(s_q, a.st->nt);
-    while (wd.next(a.tile_base, nq, t, q, lt)) x_probe_tile<TR, SORTED, FRAMED>(a, q, lt, s_pw);
+    __shared__ uint64_t s_pw[sizeof(StepParams) / 8];
+    uint64_t t, lt;
+    uint32_t q;
+    if constexpr (QUEUE) {
+      __shared__ QueueLds s_wq;
+      BlockQueue wq(s_wq, a.st->queue[0], a.st->nt);
+      while (wq.next(a.tile_base, nq, t, q, lt)) x_probe_tile<TR, SORTED, FRAMED>(a, q, lt, s_pw);
+    } else {
+      __shared__ uint32_t s_q;
+      StaticDeal wd(s_q, a.st->nt);
+      while (wd.next(a.tile_base, nq, t, q, lt)) x_probe_tile<TR, SORTED, FRAMED>(a, q, lt, s_pw);
+    }
   }
 }
 

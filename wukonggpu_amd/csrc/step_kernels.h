@@ -197,33 +197,90 @@ __device__ __forceinline__ void probe_tile(const GraphView &g, const StepParams 
     }
     return probe_plan<FRAMED, kTags>(g, m, key, before63);
   };
-  ProbeCarry carry;
   uint32_t probed = 0;
-  // round rd is finished while round rd + 1's slots and round rd + 2's tag
-  // words are on their way
+  // The wave's rows' degrees and list offsets into s_cnt and s_aux. Round rd
+  // is finished while round rd + 1's slots and round rd + 2's tag words are on
+  // their way.
   ProbePlan pl[3];
   pl[0] = plan(0, 0);
   if (kRounds > 1) pl[1] = plan(1, lane63_64(pl[0].key));
   probe_pick<kTags>(g, pl[0]);
+  if constexpr (kTags) {
+    // The rows that must walk (few) wait for all rounds: their walks, chains
+    // of dependent reads, then run once per tile, not once per round.
+    uint4 *kb = s_wp[wave].kb;
+    uint32_t pending = 0;                   // (wave-uniform)
+    uint64_t lead[kRounds], have[kRounds];  // leaders and rows with a key (wave-uniform)
+    const uint64_t below = lanes_below();
+    auto put = [&](uint32_t row, uint32_t d, uint32_t o) {
+      s_cnt[row] = d;
+      s_aux[row] = o;
+    };
 #pragma unroll
-  for (int rd = 0; rd < kRounds; rd++) {
-    const uint32_t local = wave * kWaveRows + rd * kWave + lane;
-    const int32_t end_cell = ends[rd];
-    if (rd + 2 < kRounds) pl[(rd + 2) % 3] = plan(rd + 2, lane63_64(pl[(rd + 1) % 3].key));
-    if (rd + 1 < kRounds) probe_pick<kTags>(g, pl[(rd + 1) % 3]);
-    uint32_t deg, off;
-    probed += probe_finish<FRAMED, kTags>(g, m, pl[rd % 3], s_wp[wave], deg, off, carry);
-    if (p.mode == kModeK2U) {
-      s_cnt[local] = deg;
-      s_aux[local] = off;
-    } else {
-      const bool k2k = p.mode == kModeK2K;
-      bool my_found;
-      uint32_t my_ex;
-      rows_member<SORTED, FRAMED>(g, m.edge_start, m.eframe_base, off, deg, k2k ? (uint32_t)end_cell : p.target,
-                                  k2k ? end_cell >= 0 : p.target_ok != 0, my_found, my_ex);
-      s_cnt[local] = my_found ? 1u : 0u;
-      s_aux[local] = my_ex;
+    for (int rd = 0; rd < kRounds; rd++) {
+      const uint32_t local = wave * kWaveRows + rd * kWave + lane;
+      if (rd + 2 < kRounds) pl[(rd + 2) % 3] = plan(rd + 2, lane63_64(pl[(rd + 1) % 3].key));
+      if (rd + 1 < kRounds) probe_pick<kTags>(g, pl[(rd + 1) % 3]);
+      const ProbePlan &cur = pl[rd % 3];
+      lead[rd] = cur.leaders;
+      have[rd] = wave_ballot(cur.key != 0);
+      probed += (uint32_t)__builtin_popcountll(cur.leaders);
+      uint32_t deg, off;
+      const bool walk = !probe_slot<true>(g, m, cur, deg, off);
+      put(local, deg, off);
+      const uint64_t walkers = wave_ballot(walk);
+      const uint32_t nw = (uint32_t)__builtin_popcountll(walkers);
+      if (pending + nw > (uint32_t)kWave) {  // (wave-uniform)
+        wave_lds_sync();
+        walk_pending<false, 2>(g, m, kb, pending, put);
+        pending = 0;
+      }
+      if (walk)
+        kb[pending + (uint32_t)__builtin_popcountll(walkers & below)] =
+            make_uint4((uint32_t)cur.key, (uint32_t)(cur.key >> 32), cur.bucket, local);
+      pending += nw;
+    }
+    if (pending) {
+      wave_lds_sync();
+      walk_pending<false, 2>(g, m, kb, pending, put);
+    }
+    // rows that follow a leader take its result (a run may have begun in an earlier round)
+    uint32_t last = 0;  // the last leader's row so far
+#pragma unroll
+    for (int rd = 0; rd < kRounds; rd++) {
+      const uint32_t first = wave * kWaveRows + rd * kWave;
+      if (have[rd] != lead[rd]) {  // (wave-uniform)
+        wave_lds_sync();
+        const uint64_t mine = lead[rd] & (below | (1ull << lane));
+        const uint32_t src = mine ? first + 63u - (uint32_t)__builtin_clzll(mine) : last;
+        const uint32_t d = s_cnt[src], o = s_aux[src];
+        if ((have[rd] & ~lead[rd]) >> lane & 1) put(first + lane, d, o);
+      }
+      if (lead[rd]) last = first + 63u - (uint32_t)__builtin_clzll(lead[rd]);
+    }
+  } else {
+    ProbeCarry carry;
+#pragma unroll
+    for (int rd = 0; rd < kRounds; rd++) {
+      const uint32_t local = wave * kWaveRows + rd * kWave + lane;
+      if (rd + 2 < kRounds) pl[(rd + 2) % 3] = plan(rd + 2, lane63_64(pl[(rd + 1) % 3].key));
+      if (rd + 1 < kRounds) probe_pick<kTags>(g, pl[(rd + 1) % 3]);
+      probed += probe_finish<FRAMED, kTags>(g, m, pl[rd % 3], s_wp[wave], s_cnt[local], s_aux[local], carry);
+    }
+  }
+  if (p.mode != kModeK2U) {  // filters: kept flags and edges examined in their place
+    wave_lds_sync();
+    const bool k2k = p.mode == kModeK2K;
+#pragma unroll
+    for (int rd = 0; rd < kRounds; rd++) {
+      const uint32_t local = wave * kWaveRows + rd * kWave + lane;
+      const uint32_t deg = s_cnt[local], off = s_aux[local];
+      bool found;
+      uint32_t examined;
+      rows_member<SORTED, FRAMED>(g, m.edge_start, m.eframe_base, off, deg, k2k ? (uint32_t)ends[rd] : p.target,
+                                  k2k ? ends[rd] >= 0 : p.target_ok != 0, found, examined);
+      s_cnt[local] = found ? 1u : 0u;
+      s_aux[local] = examined;
     }
   }
   if (lane == 0) s_probed[wave] = probed;
