@@ -169,9 +169,9 @@ int wkg_set_table_limit(wkg_ctx *ctx, uint64_t max_table_bytes);
 int wkg_set_probe_tile_rows(wkg_ctx *ctx, int rows);
 /* A known_to_unknown step that fans out (at least 4 output rows per input
  * row with edges) keeps, with its output table, which input row each output
- * row repeats. A later known_to_unknown step whose start column is one of
- * those inherited columns (a star's next arm from the same variable) then
- * probes once per input row instead of once per output row; its output is
+ * row repeats. A later known_to_unknown step over at least 2^19 rows whose
+ * start column is one of those inherited columns (a star's next arm from the
+ * same variable) then probes once per input row instead of once per output row; its output is
  * the same, row for row. On by default; 0 turns it off. No counterpart in the
  * reference, which probes every row (core/gpu_hash.cu:145-316). */
 int wkg_set_lineage(wkg_ctx *ctx, int on);

@@ -808,6 +808,16 @@ void wkg_ctx::keep_lineage(const wkg_table *in, ProbePass &pp, uint64_t nz, wkg_
   pp.lin = nullptr;
 }
 
+// Whether a known_to_unknown step on column sc of `in` probes once per parent
+// row (step_k2u_lineage): from 2^19 rows. That path is some ten launches and
+// two round trips (65 us for a few rows); the per-row path takes 20 us up to
+// 100k rows and about 30 at the line (16 interactive queries with two such
+// steps: 557 us, 503 with the line).
+constexpr uint64_t kLineageRows = 1ull << 19;
+bool wkg_ctx::by_lineage(const wkg_table *in, int sc) const {
+  return lineage && in->lin_parent && sc < in->lin_parent->cols && in->rows >= kLineageRows;
+}
+
 // known_to_unknown on column sc of a table whose rows are its parent's
 // compacted rows fanned out (t->lin_*), with sc one of the parent's columns:
 // all rows from one parent row share the key, so the keys are gathered
@@ -1453,7 +1463,7 @@ int wkg_ctx::step_k2u_filter(const wkg_table *in, int sc, int pid, int dir, int 
   *fused = 0;
   *ex_f = 0;
   const bool fits = lineage && !framed && in && in->rows > 512 && in->cols >= 1 && sc >= 0 && sc < in->cols &&
-                    !(in->lin_parent && sc < in->lin_parent->cols) && in->cols + 1 <= kBlock &&
+                    !by_lineage(in, sc) && in->cols + 1 <= kBlock &&
                     in->rows < (1ull << 32) && (in->owned || in->slice_of);
   if (!fits || check_pattern(fpid, fdir) != WKG_OK || (fmode == kModeK2K && (ec < 0 || ec >= in->cols)))
     return step_known(kModeK2U, in, sc, pid, dir, -1, -1, s, out, ex_u);
@@ -1530,7 +1540,7 @@ int wkg_ctx::step_known(int mode, const wkg_table *in, int sc, int pid, int dir,
     if (expanded) *expanded = 0;
     return new_table(0, out_cols, s, out);
   }
-  if (mode == kModeK2U && lineage && in->lin_parent && sc < in->lin_parent->cols)
+  if (mode == kModeK2U && by_lineage(in, sc))
     return step_k2u_lineage(in, sc, pid, dir, s, out, expanded);
   const bool tiny = small_steps && R <= 512;  // (too few rows for the filters below to pay)
   if (mode != kModeK2U && !tiny && lineage && !framed && in->glin_parent && sc == c - 1 &&

@@ -263,6 +263,7 @@ struct wkg_ctx {
   void release_pass(ProbePass &pp, hipStream_t s);
   int expand_pass(const wkg_table *in, int pid, const uint2 *cinfo, const uint64_t *cexcl, uint64_t nz, uint64_t E,
                   hipStream_t s, wkg_table *t, const char *tag = "expand", uint64_t *ext_part = nullptr);
+  bool by_lineage(const wkg_table *in, int sc) const;
   bool wants_lineage(const wkg_table *in, uint64_t nz, uint64_t E) const;
   void keep_lineage(const wkg_table *in, ProbePass &pp, uint64_t nz, wkg_table *t, int pid);
   int step_filter_fanout(int mode, const wkg_table *in, int pid, int dir, int ec, int64_t cval, hipStream_t s,
