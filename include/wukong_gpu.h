@@ -351,7 +351,7 @@ int wkg_step_batch(wkg_ctx *ctx, int n, const wkg_step_desc *steps, void *stream
  * GPU_Engine::execute_one_step would dispatch, core/gpu_engine.hpp:395-467).
  * Per step level, a single-block plan kernel sizes every query's work and
  * carves its tables and scratch out of an HBM arena; persistent kernels then
- * take the probe, finalize and expand tiles of all queries from one shared
+ * take the probe and expand tiles of all queries from one shared
  * work queue (an atomic tile ticket over the concatenated tile space). The
  * whole sequence -- plan upload, every level, the retirement of finished
  * queries' tables and the read-back of the result records -- is captured once in a hipGraph
@@ -420,11 +420,11 @@ int wkg_hw_queues(void);
 
 /* Launch and tile shapes (0 = default). The autotuner below picks them. */
 typedef struct wkg_batch_tuning {
-  int32_t probe_wg_per_cu;   /* persistent probe / finalize grid, workgroups per CU */
+  int32_t probe_wg_per_cu;   /* persistent probe grid, workgroups per CU */
   int32_t expand_wg_per_cu;  /* persistent expand grid */
-  int32_t aux_wg_per_cu;     /* tile scan, merge-path partition, gather */
+  int32_t aux_wg_per_cu;     /* tile scan, gather */
   int32_t probe_tile_rows;   /* rows per probe tile: 1024 or 2048 */
-  int32_t expand_tile_items; /* merged items per expand tile: 512, 1024 or 2048 */
+  int32_t expand_tile_items; /* output rows per expand tile: 512, 1024 or 2048 */
   int32_t schedule;          /* probe and expand tiles: 0 drawn from a shared work
                                 queue, 1 dealt to the workgroups statically */
 } wkg_batch_tuning;

@@ -8,15 +8,14 @@
 //   k_x_probe        persistent: probe tiles of all queries from the work queue
 //   k_x_scan_chunks  persistent: tile sums -> chunk-local prefixes; the block
 //                    that finishes a query's last chunk scans its chunk sums
-//   k_x_finalize     persistent: compaction tiles, one wave per tile
 //   k_x_plan         1 block: per query, read the totals, allocate the
 //                    known_to_unknown output, commit the query's new table,
 //                    give finishing queries their place in the host buffer;
 //                    then size level l+1 (rows, tiles, scan chunks, scratch,
 //                    filter output), carve it out of the HBM arena, write its
 //                    step descriptors and tile prefix
-//   k_x_partition    persistent: merge-path split points of all expands
-//   k_x_expand       persistent: expand tiles from a second work queue
+//   k_x_expand       persistent: expand and compaction tiles, found in the
+//                    probe's lists, from a second work queue
 //   k_x_retire       persistent: finished queries' tables -> host buffer
 //
 // after a first k_x_plan that starts the query states and sizes level 0.
@@ -72,6 +71,8 @@ struct QState {
   uint32_t nsteps;
   uint32_t nchunks;   // tile-scan chunks of the current step
   uint32_t chunks_done;  // chunks scanned so far (the last one scans the chunk sums)
+  char *scr;          // the current step's scratch (StepLayout)
+  int32_t *out;       // the current filter's output
 };
 
 struct ExecState {
@@ -81,19 +82,32 @@ struct ExecState {
   uint64_t w0, w1;     // this level's free window
   uint64_t out_used;   // this level's outputs, bytes from the window's output end
   uint64_t scr_used;   // this level's scratch, bytes from the other end
-  uint64_t nt, nc, np, nx, nu;  // probe tiles, scan chunks, partition entries, expand tiles, retire units
+  uint64_t nt, nc, nx, nu;  // probe tiles, scan chunks, expand tiles, retire units
   uint64_t res_bytes;  // host result buffer bytes used
   uint64_t res_over;   // result bytes refused for lack of host buffer
   uint64_t peak;       // arena high-water mark
-  uint64_t pad[2];
+  uint64_t pad[3];
   // work queues of the probe (0) and expand (1) passes: 8 sub-queue heads
   // each, one 64-byte line apart so their atomics do not serialise on one line
   uint64_t queue[2][kSubQueues][8];
 };
 
+// A finished step's output rows from its probe's lists: known_to_unknown
+// expands them, the filters compact their kept rows.
+struct XRows {
+  const int32_t *T;
+  const uint4 *hits;
+  const uint64_t *tile_sum, *tile_nz, *chunk_sum, *chunk_nz;  // scanned
+  uint64_t ntiles, nz, E;
+  int32_t *O;
+  uint32_t pid, c;
+  int32_t mode;
+  uint32_t tr;
+};
+
 struct Item {
   StepParams p;
-  ExpandParams x;
+  XRows x;
 };
 
 struct ExecArgs {
@@ -106,9 +120,8 @@ struct ExecArgs {
   uint64_t *qsw;
   Item *items;            // [Q] the current passes' parameters (read per tile)
   uint64_t *qtot;         // [Q][4] each query's step totals (StepParams::totals points here)
-  uint64_t *tile_base;    // [Q+1] probe / finalize tiles
+  uint64_t *tile_base;    // [Q+1] probe tiles
   uint64_t *chunk_base;   // [Q+1] tile-scan chunks
-  uint64_t *part_base;    // [Q+1]
   uint64_t *xtile_base;   // [Q+1]
   uint64_t *unit_base;    // [Q+1] retire copy units
   const uint64_t *up_nq;  // uploaded: query count
@@ -194,16 +207,6 @@ __device__ __forceinline__ uint32_t wave_find(const uint64_t *base, uint32_t n, 
     const uint32_t plo = shfl32(pos, k ? k - 1 : 0), phi = shfl32(pos, k < kWave ? k : 0);
     if (k) lo = plo;
     if (k < kWave) hi = phi;
-  }
-  return lo;
-}
-
-// Thread-level binary search with the same contract.
-__device__ __forceinline__ uint32_t thread_find(const uint64_t *base, uint32_t n, uint64_t t) {
-  uint32_t lo = 0, hi = n;
-  while (hi - lo > 1) {
-    const uint32_t mid = (lo + hi) >> 1;
-    if (base[mid] <= t) lo = mid; else hi = mid;
   }
   return lo;
 }
@@ -329,8 +332,8 @@ __device__ __forceinline__ LevelNeed level_need(const QState &s, const wkg_plan_
   n.R = key ? 1 : s.rows;
   n.nt = (n.R + TR - 1) / TR;
   n.nc = n.nt > kScanChunk ? (n.nt + kScanChunk - 1) / kScanChunk : 1;  // an empty step still writes totals
-  // tile_sum | tile_nz | tile_ex | chunk sums x 3 | hits (TR per tile, 16 B) | K2U: cinfo, cexcl
-  n.scratch = al(24 * n.nt + 24 * n.nc) + n.nt * TR * 16 + (d.kind == WKG_STEP_K2U || key ? 2 * al(n.R * 8) : 0);
+  // tile_sum | tile_nz | tile_ex | chunk sums x 3 | hits (TR per tile, 16 B)
+  n.scratch = al(24 * n.nt + 24 * n.nc) + n.nt * TR * 16;
   n.table = (d.kind == WKG_STEP_K2K || d.kind == WKG_STEP_K2C) ? al(n.R * s.cols * 4) : 0;
   return n;
 }
@@ -374,31 +377,6 @@ __device__ __forceinline__ void wave_put(Item *items, uint32_t off, uint32_t q0,
   wave_lds_sync();  // the area is free again
 }
 
-// The field at `off` of items[q0 + lane] for lanes with q0 + lane < n (the
-// others get T{}).
-template <typename T>
-__device__ __forceinline__ T wave_get(const Item *items, uint32_t off, uint32_t q0, uint32_t n, uint64_t *lw) {
-  static_assert(sizeof(T) % 8 == 0 && sizeof(T) / 8 <= kStageWords, "record");
-  constexpr uint32_t W = sizeof(T) / 8;
-  const uint32_t lane = lane_id();
-  uint64_t v[W];
-#pragma unroll
-  for (uint32_t u = 0; u < W; u++) {  // every load is issued before the first is used
-    const uint32_t m = u * kWave + lane, i = m / W, k = m - i * W;
-    v[u] = q0 + i < n ? *(const uint64_t *)((const char *)&items[q0 + i] + off + 8 * k) : 0ull;
-  }
-#pragma unroll
-  for (uint32_t u = 0; u < W; u++) lw[u * kWave + lane] = v[u];
-  wave_lds_sync();
-  uint64_t t[W];
-#pragma unroll
-  for (uint32_t k = 0; k < W; k++) t[k] = lw[lane * W + k];
-  wave_lds_sync();
-  T r;
-  __builtin_memcpy(&r, t, sizeof(T));
-  return r;
-}
-
 // Starts a batch: query states from the upload, the arena stacks empty.
 __device__ __forceinline__ uint32_t begin_phase(const ExecArgs &a) {
   const uint64_t nq = *a.up_nq;
@@ -415,7 +393,7 @@ __device__ __forceinline__ uint32_t begin_phase(const ExecArgs &a) {
     st.nq = nq;
     st.lo_top = 0;
     st.hi_low = a.cap;
-    st.np = st.nx = st.nu = 0;
+    st.nx = st.nu = 0;
     st.res_bytes = st.res_over = st.peak = 0;
   }
   return (uint32_t)nq;
@@ -479,6 +457,8 @@ __device__ __forceinline__ void level_phase(const ExecArgs &a, uint32_t level, u
           p.target_ok = (d.kind == WKG_STEP_K2C && d.vid >= 0 && d.vid <= 0xffffffffLL) ? 1u : 0u;
         }
         char *sb = scr_at(a, level, w0, w1, os, n.scratch);
+        sv.scr = sb;
+        sv.out = nullptr;
         p.totals = a.qtot + 4 * (uint64_t)q;
         p.tile_sum = (uint64_t *)sb;
         p.tile_nz = p.tile_sum + n.nt;
@@ -488,13 +468,7 @@ __device__ __forceinline__ void level_phase(const ExecArgs &a, uint32_t level, u
         p.chunk_ex = p.chunk_nz + n.nc;
         sb += al(24 * n.nt + 24 * n.nc);
         p.hits = (uint4 *)sb;
-        sb += n.nt * TR * 16;
-        if (p.mode == kModeK2U) {
-          p.cinfo = (uint2 *)sb;
-          p.cexcl = (uint64_t *)(sb + al(n.R * 8));
-        } else {
-          p.O = (int32_t *)out_at(a, level, w0, w1, ot, n.table);
-        }
+        if (p.mode != kModeK2U) sv.out = (int32_t *)out_at(a, level, w0, w1, ot, n.table);
         sv.nchunks = (uint32_t)n.nc;
         sv.chunks_done = 0;
         // the fitting queries form a prefix (their cumulative needs are the
@@ -524,7 +498,7 @@ __device__ __forceinline__ void level_phase(const ExecArgs &a, uint32_t level, u
   if (threadIdx.x < kSubQueues) st->queue[0][threadIdx.x][0] = 0;
 }
 
-// ---- probe, tile scan, finalize ----------------------------------------------
+// ---- probe, tile scan ----------------------------------------------------------
 
 // 1024-row tiles: four waves per SIMD, like the per-step probe (the tile
 // loop's state costs a few spills, all outside the probe's round loop; the
@@ -644,125 +618,106 @@ __global__ __launch_bounds__(kBlock) void k_x_scan_chunks(ExecArgs a) {
   }
 }
 
-// One wave per tile, waves interleaved over the tile space (the tiles are
-// short and alike, so a static deal balances).
-template <int TR>
-__global__ __launch_bounds__(kBlock) void k_x_finalize(ExecArgs a) {
-  const uint32_t nq = (uint32_t)a.st->nq;
-  const uint64_t NT = a.st->nt, W = (uint64_t)gridDim.x * (kBlock / kWave);
-  uint32_t q = 0;
-  uint64_t lo = 1, hi = 0;
-  for (uint64_t t = blockIdx.x * (uint64_t)(kBlock / kWave) + threadIdx.x / kWave; t < NT; t += W) {
-    if (t < lo || t >= hi) {  // wave-uniform
-      q = wave_find(a.tile_base, nq, t);
-      lo = a.tile_base[q];
-      hi = a.tile_base[q + 1];
-    }
-    const StepParams p = a.items[q].p;
-    finalize_tile<TR>(p, t - lo);
-  }
-}
-
-// ---- expand plan: outputs, merge-path splits, retirement of finished queries ----
+// ---- expand plan: outputs, retirement of finished queries ----
 
 struct ExpandNeed {
   bool active, k2u, fin;  // fin: the query's last step
   bool bad;               // output beyond the row limit
-  uint64_t table, scratch, nx, rows, cols;
+  uint64_t table, nx, rows, cols;
 };
 
 template <int NV>
-__device__ __forceinline__ ExpandNeed expand_need(const QState &s, const StepParams &p, const uint64_t (&tot)[4],
-                                                  uint32_t level) {
-  ExpandNeed n{false, false, false, false, 0, 0, 0, 0, 0};
+__device__ __forceinline__ ExpandNeed expand_need(const QState &s, int kind, uint64_t rows, uint32_t level) {
+  ExpandNeed n{false, false, false, false, 0, 0, 0, 0};
   if (!level_active(s, level)) return n;
   n.active = true;
   n.fin = level + 1 == s.nsteps;
-  n.k2u = p.mode == kModeK2U;
-  n.rows = tot[0];
-  if (n.k2u) {
-    n.cols = p.c + 1;
-    if (n.rows >= kRowLimit) {
-      n.bad = true;
-      return n;
-    }
-    const uint64_t nz = tot[2];
-    n.table = al(n.rows * n.cols * 4);
-    n.nx = n.rows ? (nz + n.rows + NV - 1) / NV : 0;
-    n.scratch = n.nx ? al((n.nx + 1) * 8) : 0;
-  } else {
-    n.cols = p.c;
+  n.k2u = kind != WKG_STEP_K2K && kind != WKG_STEP_K2C;
+  n.rows = rows;
+  n.cols = s.cols + (n.k2u ? 1 : 0);  // (an index or constant start: from no columns)
+  if (n.k2u && n.rows >= kRowLimit) {
+    n.bad = true;
+    return n;
   }
+  n.table = n.k2u ? al(n.rows * n.cols * 4) : 0;  // (a filter's was made with its scratch)
+  n.nx = (n.rows + NV - 1) / NV;
   return n;
 }
 
 // Commits level `level`'s results; gives the stack tops after it.
-template <int NV>
+template <int TR, int NV>
 __device__ __forceinline__ void expand_phase(const ExecArgs &a, uint32_t level, uint32_t nq, uint64_t &lo_top,
                                              uint64_t &hi_low, PlanLds &pl) {
   __shared__ uint64_t s_tmp[3 * (kPlanBlock / kWave)];
   uint64_t *lw = pl.w[threadIdx.x / kWave];
-  __shared__ unsigned long long s_ut, s_us, s_rb, s_over, s_lo, s_hi;
+  __shared__ unsigned long long s_ut, s_rb, s_over, s_lo, s_hi;
   ExecState *st = a.st;
   const uint64_t w0 = st->w0, w1 = st->w1, ou = st->out_used, su = st->scr_used;
+  const uint32_t lv = level < a.P ? level : a.P - 1;
   const uint64_t room = (w1 - w0) - ou - su;
   const uint64_t rb0 = st->res_bytes;
   const uint64_t lo_prev = st->lo_top, hi_prev = st->hi_low, peak_prev = st->peak, over_prev = st->res_over;
   if (threadIdx.x == 0) {
-    s_ut = s_us = s_rb = s_over = 0;
+    s_ut = s_rb = s_over = 0;
   }
-  uint64_t carry_t = 0, carry_s = 0, carry_p = 0, carry_x = 0, carry_r = 0, carry_u = 0;
+  uint64_t carry_t = 0, carry_x = 0, carry_r = 0, carry_u = 0;
   for (uint32_t c0 = 0; c0 < nq; c0 += kPlanBlock) {
     const uint32_t q = c0 + threadIdx.x;
     const uint32_t qc = q < nq ? q : nq - 1;
     QState sv = qs_get(a, qc);
-    const StepParams p = wave_get<StepParams>(a.items, offsetof(Item, p), q - lane_id(), nq, lw);
-    const uint64_t tot[4] = {a.qtot[4 * (uint64_t)qc], a.qtot[4 * (uint64_t)qc + 1], a.qtot[4 * (uint64_t)qc + 2], 0};
-    const ExpandNeed n = q < nq ? expand_need<NV>(sv, p, tot, level) : ExpandNeed{false, false, false, false, 0, 0, 0, 0, 0};
-    uint64_t sz[2] = {n.table, n.scratch}, szt[2];
-    block_excl_scan_n<2, kPlanBlock, true>(sz, s_tmp, szt);
-    const uint64_t ot = carry_t + sz[0], os = carry_s + sz[1];
-    // arena fit; partition entries, expand tiles, result bytes of finishing queries
-    const bool fit = n.active && !n.bad && ot + n.table + os + n.scratch <= room;
+    const wkg_plan_step d = a.up_steps[(uint64_t)qc * a.P + lv];
+    const uint64_t tot[3] = {a.qtot[4 * (uint64_t)qc], a.qtot[4 * (uint64_t)qc + 1], a.qtot[4 * (uint64_t)qc + 2]};
+    const ExpandNeed n =
+        q < nq ? expand_need<NV>(sv, d.kind, tot[0], level) : ExpandNeed{false, false, false, false, 0, 0, 0, 0};
+    uint64_t sz[1] = {n.table}, szt[1];
+    block_excl_scan_n<1, kPlanBlock, true>(sz, s_tmp, szt);
+    const uint64_t ot = carry_t + sz[0];
+    // arena fit; expand tiles, result bytes of finishing queries
+    const bool fit = n.active && !n.bad && ot + n.table <= room;
     const uint64_t rb = fit && n.fin ? al(n.rows * n.cols * 4) : 0;
-    uint64_t cnt[3] = {fit && n.nx ? n.nx + 1 : 0, fit ? n.nx : 0, rb}, cntt[3];
-    block_excl_scan_n<3, kPlanBlock, true>(cnt, s_tmp, cntt);
-    const uint64_t orb = carry_r + cnt[2];
+    uint64_t cnt[2] = {fit ? n.nx : 0, rb}, cntt[2];
+    block_excl_scan_n<2, kPlanBlock, true>(cnt, s_tmp, cntt);
+    const uint64_t orb = carry_r + cnt[1];
     // host-buffer fit (again a prefix) and copy units
     const bool host_fit = rb0 + orb + rb <= a.hcap;
     uint64_t nu[1] = {fit && n.fin && host_fit ? (rb + kCopyUnit - 1) / kCopyUnit : 0}, nut[1];
     block_excl_scan_n<1, kPlanBlock, true>(nu, s_tmp, nut);
-    const uint64_t pbase = carry_p + cnt[0], xbase = carry_x + cnt[1], ubase = carry_u + nu[0];
+    const uint64_t xbase = carry_x + cnt[0], ubase = carry_u + nu[0];
     if (q < nq) {
-      a.part_base[q] = pbase;
       a.xtile_base[q] = xbase;
       a.unit_base[q] = ubase;
     }
-    ExpandParams x{};
+    XRows x{};
     if (n.active) {
       if (n.bad) {
         sv.status = WKG_ERANGE;
       } else if (!fit) {
         sv.status = WKG_ENOMEM;
       } else {
+        const LevelNeed ln = level_need<TR>(sv, d, level);  // (the step's scratch as its plan laid it out)
+        x.T = sv.T;
+        x.tile_sum = (const uint64_t *)sv.scr;
+        x.tile_nz = x.tile_sum + ln.nt;
+        x.chunk_sum = x.tile_nz + 2 * ln.nt;
+        x.chunk_nz = x.chunk_sum + ln.nc;
+        x.hits = (const uint4 *)(sv.scr + al(24 * ln.nt + 24 * ln.nc));
+        x.ntiles = ln.nt;
+        x.nz = tot[2];
+        x.E = n.rows;
+        x.pid = (uint32_t)d.pid;
+        x.c = sv.cols;
+        x.tr = TR;
         if (n.k2u) {
-          x.pid = p.pid;
-          x.T = p.T;
-          x.c = p.c;
-          x.R = tot[2];
-          x.cinfo = p.cinfo;
-          x.cexcl = p.cexcl;
-          x.part = (const uint64_t *)scr_at(a, level, w0, w1, su + os, n.scratch);
-          x.E = n.rows;
+          x.mode = kModeK2U;
           x.O = (int32_t *)out_at(a, level, w0, w1, ou + ot, n.table);
-          sv.T = x.O;
           sv.expanded += x.E;
           atomicMax(&s_ut, (unsigned long long)(ot + n.table));
-          atomicMax(&s_us, (unsigned long long)(os + n.scratch));
-        } else {  // filters: the kept rows were compacted into p.O
-          sv.T = p.O;
+        } else {
+          x.mode = kModeK2K;
+          x.O = sv.out;
           sv.expanded += tot[1];
         }
+        sv.T = x.O;
         sv.rows = n.rows;
         sv.cols = (uint32_t)n.cols;
         if (n.fin) {
@@ -776,24 +731,20 @@ __device__ __forceinline__ void expand_phase(const ExecArgs &a, uint32_t level, 
         }
       }
     }
-    wave_put(a.items, offsetof(Item, x), q - lane_id(), nq, x, n.active && fit && n.k2u, lw);
+    wave_put(a.items, offsetof(Item, x), q - lane_id(), nq, x, n.active && fit && n.nx, lw);
     if (n.active) qs_put(a, q, sv);
     carry_t += szt[0];
-    carry_s += szt[1];
-    carry_p += cntt[0];
-    carry_x += cntt[1];
-    carry_r += cntt[2];
+    carry_x += cntt[0];
+    carry_r += cntt[1];
     carry_u += nut[0];
   }
   lds_barrier();
   if (threadIdx.x == kPlanBlock - 1) {
-    a.part_base[nq] = carry_p;
     a.xtile_base[nq] = carry_x;
     a.unit_base[nq] = carry_u;
-    st->np = carry_p;
     st->nx = carry_x;
     st->nu = carry_u;
-    const uint64_t out = ou + s_ut, scr = su + s_us;
+    const uint64_t out = ou + s_ut, scr = su;
     uint64_t lo = lo_prev, hi = hi_prev;
     if (level & 1) hi = w1 - out;
     else lo = w0 + out;
@@ -822,42 +773,63 @@ __global__ __launch_bounds__(kPlanBlock) void k_x_plan(ExecArgs a, int level, in
     nq = begin_phase(a);
   } else {
     nq = (uint32_t)a.st->nq;
-    expand_phase<NV>(a, (uint32_t)level, nq, lo_top, hi_low, s_pl);
+    expand_phase<TR, NV>(a, (uint32_t)level, nq, lo_top, hi_low, s_pl);
   }
   // (each thread reads back only the states it stored itself)
   if (level + 1 < levels) level_phase<TR>(a, (uint32_t)(level + 1), nq, lo_top, hi_low, s_pl);
 }
 
-template <int NV>
-__global__ __launch_bounds__(kBlock) void k_x_partition(ExecArgs a) {
-  const uint64_t NP = a.st->np;
-  const uint32_t nq = (uint32_t)a.st->nq;
-  for (uint64_t k = blockIdx.x * (uint64_t)kBlock + threadIdx.x; k < NP; k += (uint64_t)gridDim.x * kBlock) {
-    const uint32_t q = thread_find(a.part_base, nq, k);
-    const ExpandParams &x = a.items[q].x;
-    const uint64_t j = k - a.part_base[q];
-    ((uint64_t *)x.part)[j] = merge_split<NV>(x.cexcl, x.R, x.E, j);
-  }
+// Output rows [lt NV, ...) of a step, found in its probe's lists.
+template <int NV, bool FRAMED>
+__device__ __forceinline__ void x_rows_tile(const ExecArgs &a, uint32_t q, uint64_t lt) {
+  const XRows x = a.items[q].x;
+  HitExpand h{};
+  h.pid = x.pid;
+  h.T = x.T;
+  h.c = x.c;
+  h.tr = x.tr;
+  h.hits = x.hits;
+  h.ntiles = x.ntiles;
+  h.O = x.O;
+  const uint64_t o0 = lt * NV;
+  const uint32_t nout = (uint32_t)(x.E - o0 < (uint64_t)NV ? x.E - o0 : (uint64_t)NV);
+  auto pre = [&](uint64_t t) -> uint64_t { return gmem(x.tile_sum)[t] + gmem(x.chunk_sum)[t / kScanChunk]; };
+  auto nzp = [&](uint64_t t) -> uint64_t {
+    return t >= x.ntiles ? x.nz : gmem(x.tile_nz)[t] + gmem(x.chunk_nz)[t / kScanChunk];
+  };
+  if (x.mode == kModeK2U) expand_hits_block<NV, FRAMED>(a.g, h, o0, nout, false, nullptr, pre, nzp);
+  else compact_hits_block<NV>(h, o0, nout, nzp);
 }
 
+// Expand and compaction of the level's steps (the deal keeps the tile bases
+// in LDS, as the probe's). Straight from the probe's lists: the compaction
+// and partition passes that prepared a merge-path expand took 63 us of the
+// 512-query batch's 470, and the plan kernels read back every step's record.
 template <int VT, bool FRAMED, bool QUEUE>
 __global__ __launch_bounds__(kBlock) void k_x_expand(ExecArgs a) {
   const uint32_t nq = (uint32_t)a.st->nq;
-  uint64_t t, lt;
-  uint32_t q;
+  constexpr int NV = kBlock * VT;
   if constexpr (QUEUE) {
+    uint64_t t, lt;
+    uint32_t q;
     __shared__ QueueLds s_wq;
     BlockQueue wq(s_wq, a.st->queue[1], a.st->nx);
-    while (wq.next(a.xtile_base, nq, t, q, lt)) {
-      const ExpandParams x = a.items[q].x;
-      expand_tile<VT, FRAMED>(a.g, x, lt);
-    }
+    while (wq.next(a.xtile_base, nq, t, q, lt)) x_rows_tile<NV, FRAMED>(a, q, lt);
   } else {
-    __shared__ uint32_t s_q;
-    StaticDeal wd(s_q, a.st->nx);
-    while (wd.next(a.xtile_base, nq, t, q, lt)) {
-      const ExpandParams x = a.items[q].x;
-      expand_tile<VT, FRAMED>(a.g, x, lt);
+    __shared__ uint64_t s_base[kBaseLds + 1];
+    const uint64_t n = a.st->nx;
+    if (blockIdx.x >= n) return;
+    const bool staged = nq <= kBaseLds;
+    if (staged) {
+      for (uint32_t i = threadIdx.x; i <= nq; i += kBlock) s_base[i] = a.xtile_base[i];
+      __syncthreads();
+    }
+    const uint64_t *base = staged ? s_base : a.xtile_base;
+    for (uint64_t t = blockIdx.x; t < n; t += gridDim.x) {
+      const uint32_t q = (uint32_t)__builtin_amdgcn_readfirstlane((int)wave_find(base, nq, t));
+      const uint64_t lt = t - base[q];
+      __syncthreads();  // the previous tile's LDS use is over
+      x_rows_tile<NV, FRAMED>(a, q, lt);
     }
   }
 }
@@ -954,16 +926,13 @@ wkg_batch_tuning normalized(const wkg_batch_tuning &t) {
 }
 
 template <int TR, int VT, bool SORTED, bool FRAMED, bool QUEUE>
-void enqueue_levels(const ExecArgs &a, hipStream_t s, int levels, unsigned gp, unsigned gx, unsigned ga,
-                    unsigned gf) {
+void enqueue_levels(const ExecArgs &a, hipStream_t s, int levels, unsigned gp, unsigned gx, unsigned ga) {
   constexpr int NV = kBlock * VT;
   k_x_plan<TR, NV><<<1, kPlanBlock, 0, s>>>(a, -1, levels);
   for (int l = 0; l < levels; l++) {
     k_x_probe<TR, SORTED, FRAMED, QUEUE><<<gp, kBlock, 0, s>>>(a);
     k_x_scan_chunks<<<ga, kBlock, 0, s>>>(a);
-    k_x_finalize<TR><<<gf, kBlock, 0, s>>>(a);
     k_x_plan<TR, NV><<<1, kPlanBlock, 0, s>>>(a, l, levels);
-    k_x_partition<NV><<<ga, kBlock, 0, s>>>(a);
     k_x_expand<VT, FRAMED, QUEUE><<<gx, kBlock, 0, s>>>(a);
     k_x_retire<<<ga, kBlock, 0, s>>>(a);
   }
@@ -971,21 +940,21 @@ void enqueue_levels(const ExecArgs &a, hipStream_t s, int levels, unsigned gp, u
 
 template <int TR, int VT, bool QUEUE>
 void enqueue_sched(const ExecArgs &a, hipStream_t s, int levels, bool sorted, bool framed, unsigned gp, unsigned gx,
-                   unsigned ga, unsigned gf) {
+                   unsigned ga) {
   if (framed) {
-    if (sorted) enqueue_levels<TR, VT, true, true, QUEUE>(a, s, levels, gp, gx, ga, gf);
-    else enqueue_levels<TR, VT, false, true, QUEUE>(a, s, levels, gp, gx, ga, gf);
+    if (sorted) enqueue_levels<TR, VT, true, true, QUEUE>(a, s, levels, gp, gx, ga);
+    else enqueue_levels<TR, VT, false, true, QUEUE>(a, s, levels, gp, gx, ga);
   } else {
-    if (sorted) enqueue_levels<TR, VT, true, false, QUEUE>(a, s, levels, gp, gx, ga, gf);
-    else enqueue_levels<TR, VT, false, false, QUEUE>(a, s, levels, gp, gx, ga, gf);
+    if (sorted) enqueue_levels<TR, VT, true, false, QUEUE>(a, s, levels, gp, gx, ga);
+    else enqueue_levels<TR, VT, false, false, QUEUE>(a, s, levels, gp, gx, ga);
   }
 }
 
 template <int TR, int VT>
 void enqueue_shape(const ExecArgs &a, hipStream_t s, int levels, bool sorted, bool framed, bool queue, unsigned gp,
-                   unsigned gx, unsigned ga, unsigned gf) {
-  if (queue) enqueue_sched<TR, VT, true>(a, s, levels, sorted, framed, gp, gx, ga, gf);
-  else enqueue_sched<TR, VT, false>(a, s, levels, sorted, framed, gp, gx, ga, gf);
+                   unsigned gx, unsigned ga) {
+  if (queue) enqueue_sched<TR, VT, true>(a, s, levels, sorted, framed, gp, gx, ga);
+  else enqueue_sched<TR, VT, false>(a, s, levels, sorted, framed, gp, gx, ga);
 }
 
 }  // namespace
@@ -1018,18 +987,18 @@ int wkg_batch::set_result_buffer(uint64_t bytes) {
 int wkg_batch::enqueue(int levels) {
   const wkg_batch_tuning t = normalized(tune);
   const unsigned gp = (unsigned)(ncu * t.probe_wg_per_cu), gx = (unsigned)(ncu * t.expand_wg_per_cu),
-                 ga = (unsigned)(ncu * t.aux_wg_per_cu), gf = (unsigned)(ncu * 8);
+                 ga = (unsigned)(ncu * t.aux_wg_per_cu);
   hipError_t e = hipMemcpyAsync(d_up, h_up, up_bytes, hipMemcpyHostToDevice, s);
   if (e != hipSuccess) return ctx->fail(WKG_EDEVICE, "plan upload failed: %s", hipGetErrorString(e));
   const bool sorted = ctx->sorted, framed = ctx->framed, queue = t.schedule == 0;
   if (t.probe_tile_rows == 1024) {
-    if (t.expand_tile_items == 512) enqueue_shape<1024, 2>(args, s, levels, sorted, framed, queue, gp, gx, ga, gf);
-    else if (t.expand_tile_items == 1024) enqueue_shape<1024, 4>(args, s, levels, sorted, framed, queue, gp, gx, ga, gf);
-    else enqueue_shape<1024, 8>(args, s, levels, sorted, framed, queue, gp, gx, ga, gf);
+    if (t.expand_tile_items == 512) enqueue_shape<1024, 2>(args, s, levels, sorted, framed, queue, gp, gx, ga);
+    else if (t.expand_tile_items == 1024) enqueue_shape<1024, 4>(args, s, levels, sorted, framed, queue, gp, gx, ga);
+    else enqueue_shape<1024, 8>(args, s, levels, sorted, framed, queue, gp, gx, ga);
   } else {
-    if (t.expand_tile_items == 512) enqueue_shape<2048, 2>(args, s, levels, sorted, framed, queue, gp, gx, ga, gf);
-    else if (t.expand_tile_items == 1024) enqueue_shape<2048, 4>(args, s, levels, sorted, framed, queue, gp, gx, ga, gf);
-    else enqueue_shape<2048, 8>(args, s, levels, sorted, framed, queue, gp, gx, ga, gf);
+    if (t.expand_tile_items == 512) enqueue_shape<2048, 2>(args, s, levels, sorted, framed, queue, gp, gx, ga);
+    else if (t.expand_tile_items == 1024) enqueue_shape<2048, 4>(args, s, levels, sorted, framed, queue, gp, gx, ga);
+    else enqueue_shape<2048, 8>(args, s, levels, sorted, framed, queue, gp, gx, ga);
   }
   k_x_records<<<1, kBlock, 0, s>>>(args);
   e = hipGetLastError();
@@ -1095,7 +1064,7 @@ int wkg_batch_create(wkg_ctx *ctx, int max_queries, int max_patterns, uint64_t a
   const uint64_t o_tot = al(o_items + Q * sizeof(Item));
   const uint64_t o_base = al(o_tot + Q * 32);
   const uint64_t base_bytes = al((Q + 1) * 8);
-  const uint64_t o_up = o_base + 5 * base_bytes;
+  const uint64_t o_up = o_base + 4 * base_bytes;
   b->up_bytes = al(8 + Q * 4) + Q * P * sizeof(wkg_plan_step);
   b->ctl_bytes = o_up + b->up_bytes;
   b->down_bytes = o_res + Q * sizeof(wkg_batch_result);
@@ -1125,9 +1094,8 @@ int wkg_batch_create(wkg_ctx *ctx, int max_queries, int max_patterns, uint64_t a
   a.qtot = (uint64_t *)(b->dctl + o_tot);
   a.tile_base = (uint64_t *)(b->dctl + o_base);
   a.chunk_base = (uint64_t *)(b->dctl + o_base + base_bytes);
-  a.part_base = (uint64_t *)(b->dctl + o_base + 2 * base_bytes);
-  a.xtile_base = (uint64_t *)(b->dctl + o_base + 3 * base_bytes);
-  a.unit_base = (uint64_t *)(b->dctl + o_base + 4 * base_bytes);
+  a.xtile_base = (uint64_t *)(b->dctl + o_base + 2 * base_bytes);
+  a.unit_base = (uint64_t *)(b->dctl + o_base + 3 * base_bytes);
   a.up_nq = (const uint64_t *)b->d_up;
   a.up_nsteps = (const uint32_t *)(b->d_up + 8);
   a.up_steps = (const wkg_plan_step *)(b->d_up + al(8 + Q * 4));
