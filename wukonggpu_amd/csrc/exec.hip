@@ -196,7 +196,8 @@ __device__ __forceinline__ uint32_t block_find(const uint64_t *base, uint32_t n,
 }
 
 // The same search done by one wave for itself (the result is wave-uniform).
-__device__ __forceinline__ uint32_t wave_find(const uint64_t *base, uint32_t n, uint64_t t) {
+template <class T>
+__device__ __forceinline__ uint32_t wave_find(const T *base, uint32_t n, uint64_t t) {
   const uint32_t lane = lane_id();
   uint32_t lo = 0, hi = n;
   while (hi - lo > 1) {
@@ -781,7 +782,7 @@ __global__ __launch_bounds__(kPlanBlock) void k_x_plan(ExecArgs a, int level, in
 
 // Output rows [lt NV, ...) of a step, found in its probe's lists.
 template <int NV, bool FRAMED>
-__device__ __forceinline__ void x_rows_tile(const ExecArgs &a, uint32_t q, uint64_t lt) {
+__device__ __forceinline__ void x_rows_tile(RowsLds<NV> &lds, const ExecArgs &a, uint32_t q, uint64_t lt) {
   const XRows x = a.items[q].x;
   HitExpand h{};
   h.pid = x.pid;
@@ -797,8 +798,8 @@ __device__ __forceinline__ void x_rows_tile(const ExecArgs &a, uint32_t q, uint6
   auto nzp = [&](uint64_t t) -> uint64_t {
     return t >= x.ntiles ? x.nz : gmem(x.tile_nz)[t] + gmem(x.chunk_nz)[t / kScanChunk];
   };
-  if (x.mode == kModeK2U) expand_hits_block<NV, FRAMED>(a.g, h, o0, nout, false, nullptr, pre, nzp);
-  else compact_hits_block<NV>(h, o0, nout, nzp);
+  if (x.mode == kModeK2U) expand_hits_block<NV, FRAMED>(lds, a.g, h, o0, nout, false, nullptr, pre, nzp);
+  else compact_hits_block<NV>(lds, h, o0, nout, nzp);
 }
 
 // Expand and compaction of the level's steps (the deal keeps the tile bases
@@ -809,27 +810,28 @@ template <int VT, bool FRAMED, bool QUEUE>
 __global__ __launch_bounds__(kBlock) void k_x_expand(ExecArgs a) {
   const uint32_t nq = (uint32_t)a.st->nq;
   constexpr int NV = kBlock * VT;
+  __shared__ RowsLds<NV> s_rows;
   if constexpr (QUEUE) {
     uint64_t t, lt;
     uint32_t q;
     __shared__ QueueLds s_wq;
     BlockQueue wq(s_wq, a.st->queue[1], a.st->nx);
-    while (wq.next(a.xtile_base, nq, t, q, lt)) x_rows_tile<NV, FRAMED>(a, q, lt);
+    while (wq.next(a.xtile_base, nq, t, q, lt)) x_rows_tile<NV, FRAMED>(s_rows, a, q, lt);
   } else {
-    __shared__ uint64_t s_base[kBaseLds + 1];
+    __shared__ uint32_t s_base[kBaseLds + 1];
     const uint64_t n = a.st->nx;
     if (blockIdx.x >= n) return;
-    const bool staged = nq <= kBaseLds;
+    const bool staged = nq <= kBaseLds && n < (1ull << 32);
     if (staged) {
-      for (uint32_t i = threadIdx.x; i <= nq; i += kBlock) s_base[i] = a.xtile_base[i];
+      for (uint32_t i = threadIdx.x; i <= nq; i += kBlock) s_base[i] = (uint32_t)a.xtile_base[i];
       __syncthreads();
     }
-    const uint64_t *base = staged ? s_base : a.xtile_base;
     for (uint64_t t = blockIdx.x; t < n; t += gridDim.x) {
-      const uint32_t q = (uint32_t)__builtin_amdgcn_readfirstlane((int)wave_find(base, nq, t));
-      const uint64_t lt = t - base[q];
+      const uint32_t q = (uint32_t)__builtin_amdgcn_readfirstlane(
+          (int)(staged ? wave_find(s_base, nq, t) : wave_find(a.xtile_base, nq, t)));
+      const uint64_t lt = t - (staged ? s_base[q] : a.xtile_base[q]);
       __syncthreads();  // the previous tile's LDS use is over
-      x_rows_tile<NV, FRAMED>(a, q, lt);
+      x_rows_tile<NV, FRAMED>(s_rows, a, q, lt);
     }
   }
 }

@@ -220,10 +220,14 @@ __device__ __forceinline__ void probe_tile(const GraphView &g, const StepParams 
     for (int rd = 0; rd < kRounds; rd++) {
       const uint32_t local = wave * kWaveRows + rd * kWave + lane;
       if (rd + 2 < kRounds) pl[(rd + 2) % 3] = plan(rd + 2, lane63_64(pl[(rd + 1) % 3].key));
-      if (rd + 1 < kRounds) probe_pick<kTags>(g, pl[(rd + 1) % 3]);
+      if (rd + 1 < kRounds && pl[(rd + 1) % 3].leaders) probe_pick<kTags>(g, pl[(rd + 1) % 3]);
       const ProbePlan &cur = pl[rd % 3];
       lead[rd] = cur.leaders;
       have[rd] = wave_ballot(cur.key != 0);
+      if (!cur.leaders) {  // (wave-uniform: a long run goes on, or no keys)
+        put(local, 0, 0);
+        continue;
+      }
       probed += (uint32_t)__builtin_popcountll(cur.leaders);
       uint32_t deg, off;
       const bool walk = !probe_slot<true>(g, m, cur, deg, off);
@@ -747,21 +751,34 @@ __device__ __forceinline__ void find_hit(const HitExpand &a, uint64_t o, FP pre,
   hit = n + wave_last_le(cnt, local, [&](uint64_t k) -> uint64_t { return a.hits[tile * a.tr + k].w; });
 }
 
+// A block's LDS, shared by the two forms below.
+template <int NV>
+struct RowsLds {
+  int32_t start[NV + 1];             // per hit: its first output row, from the block's first
+  uint32_t off[NV + 1], row[NV + 1]; // per hit: list offset, input row
+  uint32_t edge[NV];                 // per tile of the block (first), per output row (then)
+  alignas(4) uint16_t map[NV];       // the hit that starts at an output row; then every row's hit
+  uint64_t t[2], n[2];               // tile and hit of the block's first row and of its end
+  uint32_t wmax[kBlock / kWave];
+};
+
 // Output rows [o0, o0 + nout), nout <= NV, of a known_to_unknown step. pre(t)
 // and nzp(t): output rows and hits before tile t (nzp(ntiles): all hits). split:
 // (tile, hit) of the block's first row and of the next block's (the last
 // block's: of the last row), or null: then they are searched here. With
 // compact, the hits that start in the block also go to cinfo / cexcl.
 template <int NV, bool FRAMED, class FP, class FN>
-__device__ __forceinline__ void expand_hits_block(const GraphView &g, const HitExpand &a, uint64_t o0, uint32_t nout,
-                                                  bool compact, const uint2 *split, FP pre, FN nzp) {
+__device__ __forceinline__ void expand_hits_block(RowsLds<NV> &lds, const GraphView &g, const HitExpand &a,
+                                                  uint64_t o0, uint32_t nout, bool compact, const uint2 *split, FP pre, FN nzp) {
   constexpr int PER = NV / kBlock;
-  __shared__ int32_t s_start[NV + 1];    // per hit: its first output row, from the block's first
-  __shared__ uint32_t s_off[NV + 1], s_row[NV + 1];
-  __shared__ uint32_t s_edge[NV];        // per tile of the block (first), per output row (then)
-  __shared__ __align__(4) uint16_t s_map[NV];  // the hit that starts at an output row; then every row's hit
-  __shared__ uint64_t s_t[2], s_n[2];    // tile and hit of the block's first row and of its end
-  __shared__ uint32_t s_wmax[kBlock / kWave];
+  auto &s_start = lds.start;
+  auto &s_off = lds.off;
+  auto &s_row = lds.row;
+  auto &s_edge = lds.edge;
+  auto &s_map = lds.map;
+  auto &s_t = lds.t;
+  auto &s_n = lds.n;
+  auto &s_wmax = lds.wmax;
   const uint32_t tid = threadIdx.x, lane = lane_id(), wave = tid / kWave;
   for (uint32_t i = tid; i < NV / 2; i += kBlock) ((uint32_t *)s_map)[i] = 0;
   if (split) {
@@ -851,9 +868,10 @@ __device__ __forceinline__ void expand_hits_block(const GraphView &g, const HitE
 
 // Kept rows [o0, o0 + nout) of a filter step (a hit each).
 template <int NV, class FN>
-__device__ __forceinline__ void compact_hits_block(const HitExpand &a, uint64_t o0, uint32_t nout, FN nzp) {
-  __shared__ uint32_t s_row[NV];
-  __shared__ uint64_t s_t[2];  // tile of the block's first and last row
+__device__ __forceinline__ void compact_hits_block(RowsLds<NV> &lds, const HitExpand &a, uint64_t o0, uint32_t nout,
+                                                   FN nzp) {
+  auto &s_row = lds.row;
+  auto &s_t = lds.t;  // tile of the block's first and last row
   const uint32_t tid = threadIdx.x, wave = tid / kWave;
   if (wave < 2) {
     const uint64_t t = wave_last_le(a.ntiles, wave ? o0 + nout - 1 : o0, nzp);
@@ -899,8 +917,9 @@ template <bool FRAMED>
 __global__ __launch_bounds__(kBlock) void k_expand_hits(GraphView g, HitExpand a, ScannedTiles t) {
   const uint64_t b = t.block0 + blockIdx.x, o0 = b * (uint64_t)kHitNV;
   const uint32_t nout = (uint32_t)(t.E - o0 < (uint64_t)kHitNV ? t.E - o0 : (uint64_t)kHitNV);
+  __shared__ RowsLds<kHitNV> s_rows;
   expand_hits_block<kHitNV, FRAMED>(
-      g, a, o0, nout, a.cinfo != nullptr, t.split + b, [&](uint64_t i) -> uint64_t { return t.pre(i); },
+      s_rows, g, a, o0, nout, a.cinfo != nullptr, t.split + b, [&](uint64_t i) -> uint64_t { return t.pre(i); },
       [&](uint64_t i) -> uint64_t { return t.nzp(i, a.ntiles); });
 }
 
@@ -926,6 +945,7 @@ struct FollowStep {
 template <bool FRAMED>
 __global__ __launch_bounds__(kBlock) void k_follow(GraphView g, HitExpand a, FollowStep f) {
   constexpr int PT = kScanChunk / kBlock;
+  __shared__ RowsLds<kFollowNV> s_rows;
   __shared__ uint64_t s_pre[kScanChunk];
   __shared__ uint32_t s_nzp[kScanChunk + 1];
   __shared__ uint64_t s_tmp[2 * (kBlock / kWave)];
@@ -991,9 +1011,9 @@ __global__ __launch_bounds__(kBlock) void k_follow(GraphView g, HitExpand a, Fol
   for (uint64_t o0 = blockIdx.x * NV; o0 < E; o0 += gridDim.x * NV) {
     const uint32_t nout = (uint32_t)(E - o0 < NV ? E - o0 : NV);
     if (f.mode == kModeK2U)
-      expand_hits_block<kFollowNV, FRAMED>(g, a, o0, nout, a.cinfo && E >= 4 * nz, nullptr, pre, nzp);
+      expand_hits_block<kFollowNV, FRAMED>(s_rows, g, a, o0, nout, a.cinfo && E >= 4 * nz, nullptr, pre, nzp);
     else
-      compact_hits_block<kFollowNV>(a, o0, nout, nzp);
+      compact_hits_block<kFollowNV>(s_rows, a, o0, nout, nzp);
     __syncthreads();  // the block's LDS is reused
   }
 }
