@@ -531,7 +531,7 @@ __device__ __forceinline__ void x_probe_tile(const ExecArgs &a, uint32_t q, uint
 // The static deal of 1024-row tiles: a workgroup's tiles are a chain of
 // reads each (the tile's query, its record, the rows, tags, slots), so the
 // query search runs on a copy of the tile bases in LDS and the next tile's
-// record is on its way while this one is probed. @@X1@@
+// record is on its way while this one is probed.
 constexpr uint32_t kBaseLds = 1024;
 template <bool SORTED, bool FRAMED>
 __device__ __forceinline__ void x_probe_deal(const ExecArgs &a, uint32_t nq) {
