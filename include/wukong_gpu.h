@@ -184,11 +184,14 @@ int wkg_set_lineage(wkg_ctx *ctx, int on);
  * holding it; its output and work count are the per-row filter's. No
  * counterpart in the reference (core/gpu_hash.cu:320-466 tests every row). */
 int wkg_set_group_filter_rows(wkg_ctx *ctx, uint64_t rows);
-/* Such a filter over long lists shared by many parents runs a block of a
- * list's entries against 64 of its parents per workgroup and lists the kept
- * rows (at most kept_cap of them, 0: 2^22; with more it reruns with one
- * parent per workgroup). On by default; 0 always runs one parent per
- * workgroup. The output and work count are the same either way. */
+/* Such a filter over long lists shared by many parents (sorted lists) hashes
+ * the targets of each list's parents and looks the neighbours of every
+ * distinct list entry up among them; with more kept rows than that lists
+ * (2^15), or unsorted lists, it runs a block of a list's entries against 64
+ * of its parents per workgroup and lists the kept rows (at most kept_cap of
+ * them, 0: 2^22; with more it reruns with one parent per workgroup). On by
+ * default; 0 always runs one parent per workgroup. The output and work count
+ * are the same either way. */
 int wkg_set_fanout_blocks(wkg_ctx *ctx, int on, uint64_t kept_cap);
 /* The calling thread's per-step calls on ctx (stream NULL) get a stream and
  * a pinned read-back block of their own until _end, so several threads can

@@ -2361,7 +2361,9 @@ __device__ __forceinline__ void list_element(const GraphView &g, uint64_t estart
   }
 }
 
-__global__ __launch_bounds__(kBlock) void k_list_filter(GraphView g, ListFilter f, uint32_t total, uint32_t nl) {
+__global__ __launch_bounds__(kBlock) void k_list_filter(GraphView g, ListFilter f, uint32_t total, uint32_t nl,
+                                                        uint32_t block0) {
+  const uint32_t block = block0 + blockIdx.x;
   constexpr int RD = kListTile / kBlock;
   __shared__ WaveProbeLds s_wp[kBlock / kWave];
   const uint32_t lane = lane_id(), wave = threadIdx.x / kWave;
@@ -2369,9 +2371,9 @@ __global__ __launch_bounds__(kBlock) void k_list_filter(GraphView g, ListFilter 
   uint32_t l[RD], j[RD], e[RD], deg[RD], off[RD];
   bool in[RD];
   {
-    const uint32_t w0 = blockIdx.x * (uint32_t)kListTile + wave * RD * kWave;
+    const uint32_t w0 = block * (uint32_t)kListTile + wave * RD * kWave;
     if (w0 >= total) {  // (waves are independent: no barrier below)
-      if (lane == 0) f.ex[blockIdx.x * (kBlock / kWave) + wave] = 0;
+      if (lane == 0) f.ex[block * (kBlock / kWave) + wave] = 0;
       return;
     }
     // the wave's first list, and whether all its rows are in it
@@ -2446,14 +2448,14 @@ __global__ __launch_bounds__(kBlock) void k_list_filter(GraphView g, ListFilter 
     }
     if (deg[r] > kListInline) {
       const uint32_t n = (deg[r] + kListChunk - 1) / kListChunk;
-      const uint32_t q = blockIdx.x % kListQueues;
+      const uint32_t q = block % kListQueues;
       const uint64_t b = atomicAdd(&f.long_n[q * kListPad], (unsigned long long)n);
       for (uint32_t c = 0; c < n && b + c < f.long_cap; c++)
         f.longs[q * f.long_cap + b + c] = make_uint4(f.l_base[l[r]] + j[r], off[r], deg[r], c * kListChunk);
     }
   }
   ex = lane63_64(wave_incl_scan(ex));
-  if (lane == 0) f.ex[blockIdx.x * (kBlock / kWave) + wave] = ex;
+  if (lane == 0) f.ex[block * (kBlock / kWave) + wave] = ex;
 }
 
 // The long filter lists, a chunk per workgroup at a time; the first workgroup

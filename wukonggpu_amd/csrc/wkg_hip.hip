@@ -1419,7 +1419,10 @@ int wkg_ctx::step_filter_lists(int mode, const wkg_table *in, int pid, int dir, 
   {
     // per distinct entry: itself, its tag word and its bucket's line
     ProfScope ps(this, s, "fanout_filter", 140.0 * (double)total);
-    k_list_filter<<<(unsigned)nwg, kBlock, 0, s>>>(g, f, (uint32_t)total, (uint32_t)nl);
+    const uint64_t per = std::max<uint64_t>(thread_launch_rows() / kListTile, 1);  // split launches, as the probe's
+    for (uint64_t b0 = 0; b0 < nwg; b0 += per)
+      k_list_filter<<<(unsigned)std::min(per, nwg - b0), kBlock, 0, s>>>(g, f, (uint32_t)total, (uint32_t)nl,
+                                                                         (uint32_t)b0);
     k_list_long<<<16 * kListQueues, kBlock, 0, s>>>(g, f, (uint32_t)nl, (uint32_t)nex);
   }
   if ((le = hipGetLastError()) != hipSuccess)
