@@ -38,6 +38,23 @@ def test_split_matches_oracle(dev_small, rows, cols, col, nparts):
         v.free()
 
 
+# a part's slab counts scanned by one workgroup (up to 8192 slabs) or in
+# chunks of 2048: the last whole size, the first in chunks, a last chunk of
+# one slab, of all 2048, and slabs of 16 rows a part
+@pytest.mark.parametrize("rows,nparts", [
+    (8192 * 1024, 3), (8192 * 1024 + 1, 3), (8193 * 1024, 64), (10241 * 1024 - 7, 8), (10240 * 1024, 1),
+    (8200 * 16 * 65, 65)])
+def test_split_count_scan_chunks(dev_small, rows, nparts):
+    rng = np.random.default_rng(rows + nparts)
+    t = rng.integers(1 << 17, 1 << 27, size=(rows, 1), dtype=np.int32)
+    t[: rows // 2] -= t[: rows // 2] % nparts  # the first half's owners: part 0
+    print(f"split {rows}x1 into {nparts}", flush=True)
+    out, prow, phead = dev_small.table_split(dev_small.table(t), 0, nparts)
+    want, wrows, wheads = split_table(t, 0, nparts)
+    assert np.array_equal(out.to_host(), want) and np.array_equal(prow, wrows) and np.array_equal(phead, wheads)
+    out.free()
+
+
 def test_split_skewed_and_negative_cells(dev_small):
     # all rows in one part, and cells above 2^31 (read as unsigned)
     rng = np.random.default_rng(3)

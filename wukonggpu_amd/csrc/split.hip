@@ -17,10 +17,10 @@
 // than 64 parts, so the count array stays under a byte per row), one wave per
 // slab:
 //   count:   rows per part in the slab -> cnt[part][slab];
-//   scan:    per part, by one workgroup: its slabs' counts become base, the
-//            part's rows before the slab, and their sum total[part]; a
-//            part's first row is the totals of the parts before it, which the
-//            scatter's waves add up themselves;
+//   scan:    per part, by one workgroup or in chunks: its slabs' counts
+//            become base, the part's rows before the slab, and their sum
+//            total[part]; a part's first row is the totals of the parts before
+//            it, which the scatter's waves add up themselves;
 //   scatter: each 64-row chunk ranks its rows inside their parts, then the
 //            rows are copied to their places (rows of one part are
 //            contiguous there too); with 9..64 parts and rows of 1, 2 or 4
@@ -160,33 +160,50 @@ __global__ __launch_bounds__(kSplitBlock) void k_split_count(SplitArgs a) {
   }
 }
 
-// Part blockIdx.x's slab counts -> rows before each slab, and their sum.
-// (The scan was rocPRIM's over the whole count array with a kernel for the
-// parts' first rows: three launches of some 5 us.)
+// A part's slab counts -> rows before each slab, and their sum. A workgroup
+// scans one chunk of K counts a thread; block b has chunk b % nchunks of part
+// b / nchunks, and adds the chunks before it from k_split_sums. Up to 8192
+// slabs (8.4M rows) a part is one chunk (K = 8) and there are no sums: 6 us at
+// 1M rows in 8 parts, 12 at 8M. Longer parts go in chunks of 2048 (K = 2),
+// two launches: 11 us at 33.5M rows in 8 parts, 15 at 134M, where one
+// workgroup walking a part 8192 counts at a time took 38 and 147 and the
+// library's scan of the whole array 14 and 20.
 constexpr int kScanBlock = 1024;
-__global__ __launch_bounds__(kScanBlock) void k_split_scan(SplitArgs a) {
+constexpr uint64_t kScanWhole = 8 * kScanBlock, kScanChunk = 2 * kScanBlock;
+template <int K>
+__global__ __launch_bounds__(kScanBlock) void k_split_scan(SplitArgs a, uint64_t nchunks, const uint64_t *sums) {
+  __shared__ uint64_t s_tmp[2 * kScanBlock / kWave];
+  const uint64_t p = blockIdx.x / nchunks, chunk = blockIdx.x % nchunks;
+  const uint32_t *cnt = a.cnt + p * a.nslabs;
+  uint64_t *base = a.base + p * a.nslabs;
+  const uint64_t lo = (chunk * kScanBlock + threadIdx.x) * K;
+  uint64_t c[K], v[2] = {0, 0}, tot[2];  // this chunk's counts; the chunks before it
+#pragma unroll
+  for (int k = 0; k < K; k++) c[k] = lo + k < a.nslabs ? cnt[lo + k] : 0;
+  for (uint64_t i = threadIdx.x; i < chunk; i += kScanBlock) v[1] += sums[p * nchunks + i];
+#pragma unroll
+  for (int k = 0; k < K; k++) v[0] += c[k];
+  block_excl_scan_n<2, kScanBlock>(v, s_tmp, tot);
+  uint64_t run = tot[1] + v[0];
+#pragma unroll
+  for (int k = 0; k < K; k++)
+    if (lo + k < a.nslabs) {
+      base[lo + k] = run;
+      run += c[k];
+    }
+  if (chunk + 1 == nchunks && threadIdx.x == 0) a.total[p] = tot[1] + tot[0];
+}
+
+// The sum of each chunk of kScanChunk counts of each part.
+__global__ __launch_bounds__(kScanBlock) void k_split_sums(SplitArgs a, uint64_t nchunks, uint64_t *sums) {
   __shared__ uint64_t s_tmp[kScanBlock / kWave];
-  const uint32_t *cnt = a.cnt + blockIdx.x * a.nslabs;
-  uint64_t *base = a.base + blockIdx.x * a.nslabs;
-  uint64_t before = 0;
-  for (uint64_t s0 = 0; s0 < a.nslabs; s0 += 8 * kScanBlock) {  // 8 slabs a thread at a time
-    const uint64_t lo = s0 + threadIdx.x * 8;
-    uint64_t c[8], v[1] = {0}, tot[1];
-#pragma unroll
-    for (int k = 0; k < 8; k++) c[k] = lo + k < a.nslabs ? cnt[lo + k] : 0;
-#pragma unroll
-    for (int k = 0; k < 8; k++) v[0] += c[k];
-    block_excl_scan_n<1, kScanBlock>(v, s_tmp, tot);
-    uint64_t run = before + v[0];
-#pragma unroll
-    for (int k = 0; k < 8; k++)
-      if (lo + k < a.nslabs) {
-        base[lo + k] = run;
-        run += c[k];
-      }
-    before += tot[0];
-  }
-  if (threadIdx.x == 0) a.total[blockIdx.x] = before;
+  const uint64_t p = blockIdx.x / nchunks, chunk = blockIdx.x % nchunks;
+  const uint32_t *cnt = a.cnt + p * a.nslabs;
+  uint64_t v[1] = {0}, tot[1];
+  for (uint64_t i = chunk * kScanChunk + threadIdx.x; i < min((chunk + 1) * kScanChunk, a.nslabs); i += kScanBlock)
+    v[0] += cnt[i];
+  block_excl_scan_n<1, kScanBlock>(v, s_tmp, tot);
+  if (threadIdx.x == 0) sums[blockIdx.x] = tot[0];
 }
 
 // First row of part `lane` (at most 64 parts; every lane of the wave).
@@ -503,8 +520,10 @@ int wkg_table_split(wkg_ctx *ctx, const wkg_table *in, int col, int nparts, void
     a.nslabs = (in->rows + a.slab - 1) / a.slab;
     const uint64_t ncnt = a.nslabs * (uint64_t)nparts;
     auto up = [](uint64_t b) { return (b + 255) & ~uint64_t(255); };
+    const uint64_t nchunks = a.nslabs <= kScanWhole ? 1 : (a.nslabs + kScanChunk - 1) / kScanChunk;
     const uint64_t b_cnt = up(ncnt * 4), b_base = up(ncnt * 8), b_total = up((uint64_t)nparts * 8);
-    char *scr = (char *)ctx->pool->alloc(b_cnt + b_base + b_total, s, wkg_ctx::err_slot());
+    const uint64_t b_sums = nchunks > 1 ? up(nchunks * (uint64_t)nparts * 8) : 0;
+    char *scr = (char *)ctx->pool->alloc(b_cnt + b_base + b_total + b_sums, s, wkg_ctx::err_slot());
     if (!scr) {
       ctx->drop_table(t);
       return WKG_ENOMEM;
@@ -521,7 +540,14 @@ int wkg_table_split(wkg_ctx *ctx, const wkg_table *in, int col, int nparts, void
     }
     {
       ProfScope ps(ctx, s, "split_scan", 12.0 * (double)ncnt);
-      k_split_scan<<<(unsigned)nparts, kScanBlock, 0, s>>>(a);
+      uint64_t *sums = (uint64_t *)(scr + b_cnt + b_base + b_total);
+      const unsigned grid = (unsigned)(nchunks * (uint64_t)nparts);
+      if (nchunks == 1) {
+        k_split_scan<8><<<grid, kScanBlock, 0, s>>>(a, 1, nullptr);
+      } else {
+        k_split_sums<<<grid, kScanBlock, 0, s>>>(a, nchunks, sums);
+        k_split_scan<2><<<grid, kScanBlock, 0, s>>>(a, nchunks, sums);
+      }
     }
     hipError_t e = hipGetLastError();
     if (e == hipSuccess) {
