@@ -1541,6 +1541,53 @@ __global__ __launch_bounds__(kBlock) void k_keep_groups(KeptRows k, const uint2 
   }
 }
 
+// The groups of an arm that was probed row by row: the arm's compacted rows
+// (cinfo, cexcl: nz rows, E output rows) hold all child rows of a kept parent
+// row i or none, so its first child row is searched among them.
+struct ArmRows {
+  const uint2 *cinfo;
+  const uint64_t *cexcl;
+  uint64_t nz, E;
+  const uint2 *pinfo;      // the input's lineage: parent row of compacted row i,
+  const uint64_t *excl_p;  // and its first child row
+  uint64_t np;
+  __device__ __forceinline__ bool find(uint64_t i, uint64_t &at) const {
+    const uint64_t r = excl_p[i];
+    uint64_t lo = 0, hi = nz;
+    while (lo < hi) {
+      const uint64_t mid = (lo + hi) >> 1;
+      if (cinfo[mid].x < r) lo = mid + 1;
+      else hi = mid;
+    }
+    at = lo;
+    return lo < nz && cinfo[lo].x == r;
+  }
+};
+
+// Parent row i: its list's length (0: not kept) and whether it is kept.
+__global__ __launch_bounds__(kBlock) void k_arm_lift(ArmRows a, uint64_t *deg, uint64_t *kept) {
+  for (uint64_t i = blockIdx.x * (uint64_t)kBlock + threadIdx.x; i < a.np; i += (uint64_t)gridDim.x * kBlock) {
+    uint64_t at;
+    const bool k = a.find(i, at);
+    deg[i] = k ? (at + 1 < a.nz ? a.cexcl[at + 1] : a.E) - a.cexcl[at] : 0;
+    kept[i] = k;
+  }
+}
+
+// The kept parent rows' groups, as k_keep_groups'; the prefixes are the
+// two-level scan's of what k_arm_lift wrote.
+__global__ __launch_bounds__(kBlock) void k_arm_groups(ArmRows a, StepParams q, uint2 *ginfo, uint64_t *gs,
+                                                       uint64_t *go) {
+  for (uint64_t i = blockIdx.x * (uint64_t)kBlock + threadIdx.x; i < a.np; i += (uint64_t)gridDim.x * kBlock) {
+    uint64_t at;
+    if (!a.find(i, at)) continue;
+    const uint64_t m = q.tile_nz[i] + q.chunk_nz[i / kScanChunk];
+    ginfo[m] = make_uint2(a.pinfo[i].x, a.cinfo[at].y);
+    gs[m] = q.tile_sum[i] + q.chunk_sum[i / kScanChunk];
+    go[m] = a.cexcl[at];
+  }
+}
+
 // The group table: G[m] = (end cell of the grandparent row (0 without an
 // end column), f_m), the list of G row m at segment offset ginfo[m].y.
 __global__ __launch_bounds__(kBlock) void k_group_table(const int32_t *P, uint32_t pc, int32_t ec, const uint2 *ginfo,

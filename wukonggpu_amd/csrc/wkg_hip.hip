@@ -646,6 +646,12 @@ int wkg_ctx::expand_hits(const wkg_table *in, int pid, const ProbePass &pp, hipS
   return WKG_OK;
 }
 
+// A star arm's groups in the making (arm_lift, arm_groups).
+struct ArmScan {
+  uint64_t *scr = nullptr;  // null: none
+  StepParams q{};           // its prefix arrays and signal
+};
+
 // The rest of a known_to_unknown step after its probe pass: t is its output
 // if follow_pass already expanded it; else the output table is made here and
 // expanded from the probe's lists or, for fan-outs, from the compacted rows by
@@ -655,20 +661,31 @@ int wkg_ctx::expand_hits(const wkg_table *in, int pid, const ProbePass &pp, hipS
 // output row (2M rows to 18M of 4 cells: 81 + 13 + 10 us by merge path, 77 + 14
 // from the lists), so the merge path is ahead above some 50 output rows per
 // row with edges; 24M keys to 9.3M rows of 2 cells: 127 + 54 + 15 and 128 + 14 us.
-int wkg_ctx::finish_k2u(const wkg_table *in, int pid, ProbePass &pp, hipStream_t s, wkg_table *t, wkg_table **out) {
+// star: the step's column is one of the input's lineage parent (star_arm); an
+// output that filters may decide by groups then gets its groups, found
+// while the expand runs.
+int wkg_ctx::finish_k2u(const wkg_table *in, int pid, ProbePass &pp, hipStream_t s, wkg_table *t, wkg_table **out,
+                        bool star) {
   const uint64_t E = pp.cnt[0], nz = pp.cnt[2];
   const int out_cols = in->cols + 1;
   int rc = WKG_OK;
+  ArmScan arm;
   if (table_limit && in->rows >= 2 && E * (uint64_t)out_cols * 4 > table_limit) {  // (one row cannot be split)
     rc = fail(WKG_ENOMEM, "a %llu-row output is above the table limit", (unsigned long long)E);
   } else if (!t && !(rc = new_table(E, out_cols, s, &t))) {
-    if (!pp.lin && E < (1ull << 32) && E < 32 * nz) {
+    if (star && nz && E >= group_filter_rows && in->lin_parent->bytes <= pool->budget / 16 &&
+        !(rc = compact_pass(pp, s)))
+      rc = arm_lift(in, pp, s, arm);
+    if (rc) {
+    } else if (!pp.lin && E < (1ull << 32) && E < 32 * nz) {
       if (wants_lineage(in, nz, E)) rc = lineage_rows(pp, s);
       if (!rc) rc = expand_hits(in, pid, pp, s, t);
     } else if (!(rc = compact_pass(pp, s))) {
       rc = expand_pass(in, pid, pp.cinfo, pp.cexcl, nz, E, s, t);
     }
   }
+  if (!rc && arm.scr) rc = arm_groups(in, pid, pp, s, arm, t);
+  pool->release(arm.scr, s);
   if (rc) {
     release_pass(pp, s);
     drop_table(t);
@@ -677,6 +694,69 @@ int wkg_ctx::finish_k2u(const wkg_table *in, int pid, ProbePass &pp, hipStream_t
   keep_lineage(in, pp, nz, t, pid);
   release_pass(pp, s);
   *out = t;
+  return WKG_OK;
+}
+
+static ArmRows arm_rows(const wkg_table *in, const ProbePass &pp) {
+  return {pp.cinfo, pp.cexcl, pp.cnt[2], pp.cnt[0], in->lin_info, in->lin_excl, in->lin_n};
+}
+
+// The lists and kept flags of the parent rows of a compacted pass over a star
+// arm, scanned like tile sums (no scratch: no groups).
+int wkg_ctx::arm_lift(const wkg_table *in, const ProbePass &pp, hipStream_t s, ArmScan &arm) {
+  const uint64_t np = in->lin_n, nchunks = (np + kScanChunk - 1) / kScanChunk;
+  if (!(arm.scr = (uint64_t *)pool->alloc((4 + 2 * np + 3 * nchunks) * 8, s, err_slot()))) return WKG_OK;
+  StepParams &q = arm.q;
+  q.totals = arm.scr;
+  q.tile_sum = arm.scr + 4;     // list lengths -> prefix
+  q.tile_nz = q.tile_sum + np;  // kept flags -> prefix
+  q.tile_ex = q.tile_nz;        // (read before it is rewritten)
+  q.ntiles = np;
+  q.chunk_sum = q.tile_nz + np;
+  q.chunk_nz = q.chunk_sum + nchunks;
+  q.chunk_ex = q.chunk_nz + nchunks;
+  q.sg = next_signal();
+  {
+    ProfScope ps(this, s, "lineage", 48.0 * (double)np);
+    k_arm_lift<<<(unsigned)std::min<uint64_t>((np + kBlock - 1) / kBlock, 65535), kBlock, 0, s>>>(
+        arm_rows(in, pp), q.tile_sum, q.tile_nz);
+    k_scan_chunks<<<(unsigned)nchunks, kBlock, 0, s>>>(q);
+    if (nchunks > 1) k_scan_top<<<1, kBlock, 0, s>>>(q, nchunks);
+  }
+  LAUNCHCHK(this);
+  return WKG_OK;
+}
+
+// The output's groups from that scan, kept under step_k2u_lineage's rule.
+int wkg_ctx::arm_groups(const wkg_table *in, int pid, const ProbePass &pp, hipStream_t s, const ArmScan &arm,
+                        wkg_table *t) {
+  if (int rc = wait_signal(arm.q.sg, s)) return rc;
+  const uint64_t dtot = rb_host()[0], nk = rb_host()[2], np = in->lin_n;
+  wkg_table *gp = in->lin_parent;
+  if (t->rows < 4 * dtot || gp->bytes + nk * 24 > pool->budget / 16) return WKG_OK;
+  void *glin = pool->alloc(nk * 24, s, err_slot());
+  if (!glin) return WKG_OK;
+  uint2 *ginfo = (uint2 *)glin;
+  uint64_t *gs = (uint64_t *)glin + nk, *go = gs + nk;
+  {
+    ProfScope ps(this, s, "lineage", 64.0 * (double)np);
+    k_arm_groups<<<(unsigned)std::min<uint64_t>((np + kBlock - 1) / kBlock, 65535), kBlock, 0, s>>>(
+        arm_rows(in, pp), arm.q, ginfo, gs, go);
+  }
+  const hipError_t le = hipGetLastError();
+  if (le != hipSuccess) {
+    pool->release(glin, s);
+    return fail(WKG_EDEVICE, "lineage launch failed: %s", hipGetErrorString(le));
+  }
+  gp->refs++;
+  t->glin_parent = gp;
+  t->glin_info = ginfo;
+  t->glin_s = gs;
+  t->glin_o = go;
+  t->glin_n = nk;
+  t->glin_dtot = dtot;
+  t->glin_pid = pid;
+  t->glin_alloc = glin;
   return WKG_OK;
 }
 
@@ -808,15 +888,18 @@ void wkg_ctx::keep_lineage(const wkg_table *in, ProbePass &pp, uint64_t nz, wkg_
   pp.lin = nullptr;
 }
 
-// Whether a known_to_unknown step on column sc of `in` probes once per parent
-// row (step_k2u_lineage): from 2^19 rows. That path is some ten launches and
-// two round trips (65 us for a few rows); the per-row path takes 20 us up to
-// 100k rows and about 30 at the line (16 interactive queries with two such
-// steps: 557 us, 503 with the line).
-constexpr uint64_t kLineageRows = 1ull << 19;
-bool wkg_ctx::by_lineage(const wkg_table *in, int sc) const {
-  return lineage && in->lin_parent && sc < in->lin_parent->cols && in->rows >= kLineageRows;
+// Whether column sc of `in` is one that its lineage parent's rows share
+// (step_k2u_lineage can probe it once per parent row).
+bool wkg_ctx::star_arm(const wkg_table *in, int sc) const {
+  return lineage && in->lin_parent && sc < in->lin_parent->cols;
 }
+
+// Such a step probes once per parent row (step_k2u_lineage) from 2^19 input
+// rows. That path is some ten launches and two round trips (65 us for a few
+// rows); the per-row path takes 20 us up to 100k rows and about 30 at the
+// line (16 interactive queries with two such steps: 557 us, 503 with the
+// line). Both leave the output's groups where a filter may use them.
+constexpr uint64_t kLineageRows = 1ull << 19;
 
 // known_to_unknown on column sc of a table whose rows are its parent's
 // compacted rows fanned out (t->lin_*), with sc one of the parent's columns:
@@ -1466,7 +1549,7 @@ int wkg_ctx::step_k2u_filter(const wkg_table *in, int sc, int pid, int dir, int 
   *fused = 0;
   *ex_f = 0;
   const bool fits = lineage && !framed && in && in->rows > 512 && in->cols >= 1 && sc >= 0 && sc < in->cols &&
-                    !by_lineage(in, sc) && in->cols + 1 <= kBlock &&
+                    !star_arm(in, sc) && in->cols + 1 <= kBlock &&
                     in->rows < (1ull << 32) && (in->owned || in->slice_of);
   if (!fits || check_pattern(fpid, fdir) != WKG_OK || (fmode == kModeK2K && (ec < 0 || ec >= in->cols)))
     return step_known(kModeK2U, in, sc, pid, dir, -1, -1, s, out, ex_u);
@@ -1543,8 +1626,8 @@ int wkg_ctx::step_known(int mode, const wkg_table *in, int sc, int pid, int dir,
     if (expanded) *expanded = 0;
     return new_table(0, out_cols, s, out);
   }
-  if (mode == kModeK2U && by_lineage(in, sc))
-    return step_k2u_lineage(in, sc, pid, dir, s, out, expanded);
+  const bool star = mode == kModeK2U && star_arm(in, sc);
+  if (star && R >= kLineageRows) return step_k2u_lineage(in, sc, pid, dir, s, out, expanded);
   const bool tiny = small_steps && R <= 512;  // (too few rows for the filters below to pay)
   if (mode != kModeK2U && !tiny && lineage && !framed && in->glin_parent && sc == c - 1 &&
       (mode == kModeK2C || ec < in->glin_parent->cols) && R >= group_filter_rows && R >= 4 * in->glin_dtot)
@@ -1577,11 +1660,15 @@ int wkg_ctx::step_known(int mode, const wkg_table *in, int sc, int pid, int dir,
     return WKG_OK;
   }
   const uint64_t E = pp.cnt[0];
-  if ((rc = finish_k2u(in, pid, pp, s, t, out))) return rc;
+  if (star && t && E >= group_filter_rows) {  // (expanded already, perhaps not compacted: the groups need that)
+    release_pass(pp, s);
+    drop_table(t);
+    return step_k2u_lineage(in, sc, pid, dir, s, out, expanded);
+  }
+  if ((rc = finish_k2u(in, pid, pp, s, t, out, star))) return rc;
   if (expanded) *expanded = E;
   return WKG_OK;
 }
-
 
 int wkg_thread_launch_rows(wkg_ctx *ctx, uint64_t rows) {
   if (!ctx) return WKG_EINVAL;

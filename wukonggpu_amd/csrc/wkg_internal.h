@@ -61,6 +61,8 @@ struct Pool {
   std::unordered_map<void *, size_t> live;
 };
 
+struct ArmScan;  // wkg_ctx::arm_lift
+
 struct wkg_table {
   int32_t *d;
   uint64_t rows;
@@ -256,14 +258,17 @@ struct wkg_ctx {
   int lineage_rows(ProbePass &pp, hipStream_t s);
   int compact_pass(ProbePass &pp, hipStream_t s);
   int expand_hits(const wkg_table *in, int pid, const ProbePass &pp, hipStream_t s, wkg_table *t);
-  int finish_k2u(const wkg_table *in, int pid, ProbePass &pp, hipStream_t s, wkg_table *t, wkg_table **out);
+  int finish_k2u(const wkg_table *in, int pid, ProbePass &pp, hipStream_t s, wkg_table *t, wkg_table **out,
+                 bool star = false);
+  int arm_lift(const wkg_table *in, const ProbePass &pp, hipStream_t s, ArmScan &arm);
+  int arm_groups(const wkg_table *in, int pid, const ProbePass &pp, hipStream_t s, const ArmScan &arm, wkg_table *t);
   bool follows(uint64_t R, int *tr) const;
   int follow_pass(int mode, const wkg_table *in, int sc, int pid, int dir, int ec, int64_t cval, int tr, hipStream_t s,
                   ProbePass &pp, wkg_table **t);
   void release_pass(ProbePass &pp, hipStream_t s);
   int expand_pass(const wkg_table *in, int pid, const uint2 *cinfo, const uint64_t *cexcl, uint64_t nz, uint64_t E,
                   hipStream_t s, wkg_table *t, const char *tag = "expand", uint64_t *ext_part = nullptr);
-  bool by_lineage(const wkg_table *in, int sc) const;
+  bool star_arm(const wkg_table *in, int sc) const;
   bool wants_lineage(const wkg_table *in, uint64_t nz, uint64_t E) const;
   void keep_lineage(const wkg_table *in, ProbePass &pp, uint64_t nz, wkg_table *t, int pid);
   int step_filter_fanout(int mode, const wkg_table *in, int pid, int dir, int ec, int64_t cval, hipStream_t s,
