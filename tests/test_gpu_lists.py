@@ -37,7 +37,8 @@ def graph():
 
 # parents, distinct targets among them, filter predicate
 @pytest.mark.parametrize("parents,targets,pid", [(513, 6000, 3), (2000, 300, 3), (5000, 1, 3), (3000, 50000, 3),
-                                                 (700, 1, 4), (513, 1, 4), (100000, 6000, 3)])
+                                                 (700, 1, 4), (513, 1, 4), (100000, 6000, 3),
+                                                 (2048, 1, 3), (2049, 2, 3), (4096, 5, 3)])
 def test_fused_filter(graph, parents, targets, pid):
     gs, dev = graph
     rng = np.random.default_rng(parents + targets)

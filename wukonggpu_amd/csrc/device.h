@@ -390,6 +390,17 @@ __device__ __forceinline__ uint64_t wave_incl_scan(uint64_t x) {
   return x;
 }
 
+// The same of u32 values.
+__device__ __forceinline__ uint32_t wave_incl_scan32(uint32_t x) {
+  const uint32_t lane = lane_id();
+#pragma unroll
+  for (int d = 1; d < kWave; d <<= 1) {
+    const uint32_t y = shfl32(x, (lane - d) & 63);
+    if (lane >= (uint32_t)d) x += y;
+  }
+  return x;
+}
+
 // Exclusive block scan over kBlock threads; `total` gets the block sum.
 // `tmp` is kBlock/kWave u64 of LDS.
 __device__ __forceinline__ uint64_t block_excl_scan(uint64_t v, uint64_t *tmp, uint64_t &total) {

@@ -2262,8 +2262,9 @@ struct ListFilter {
   // distinct lists, in first-come order: offset, entries before, length, parents
   uint32_t *l_off, *l_base, *l_len, *l_np;
   uint32_t *seen, *seen_list, mask1;  // offset -> list (open addressing)
-  uint32_t *p_list, *p_tgt, *next;    // per parent: list, target, next parent of the same two (+1)
-  uint32_t *head, *count, log2;       // (list, target) -> first parent (+1), parents (open addressing, 2^log2)
+  uint32_t *p_list, *p_tgt, *p_slot;  // per parent: list, target, its slot below
+  uint32_t *head, *count, log2;       // (list, target) -> a parent (+1), parents (open addressing, 2^log2)
+  uint32_t *start, *order;            // the slot's parents: order[start .. start + count)
   uint32_t *bits, blog2;              // two bits of a word per (list, target), 2^blog2 words
   unsigned long long *ctr;            // kList*
   uint4 *kept;                        // (row, parent, entry, 0)
@@ -2296,11 +2297,14 @@ __device__ __forceinline__ uint32_t pair_bits(uint32_t h) { return (1u << (h & 3
 // are separated by barriers; words changed by atomics are read as atomics).
 // Up to kListLds parents the hash tables are built in LDS and copied out: the
 // parents of a popular list all meet at its words, which serialises in memory
-// (800 parents: 54 us, in LDS 31 us).
+// (800 parents: 54 us, in LDS 31 us). The parents of one list and target end
+// up side by side, so that whoever keeps a row for each of them can do so with
+// a wave's lanes at once.
 constexpr uint32_t kListLds = 2048;
 __global__ __launch_bounds__(1024) void k_list_parents(ListFilter fg, Signal sg) {
   __shared__ uint32_t s_tab[(4 * 2 + 2) * kListLds];  // seen, seen_list, head, count: two slots a parent; l_np, bits
   __shared__ unsigned long long s_ctr[kListCtrs];
+  __shared__ uint32_t s_used;  // parents placed in order
   const uint32_t tid = threadIdx.x, np = (uint32_t)fg.np;
   ListFilter f = fg;
   const bool lds = np <= kListLds;
@@ -2312,11 +2316,13 @@ __global__ __launch_bounds__(1024) void k_list_parents(ListFilter fg, Signal sg)
     f.l_np = s_tab + 8 * kListLds;
     f.bits = s_tab + 9 * kListLds;
     f.ctr = s_ctr;
+    f.start = f.seen_list;  // (which is done with by then)
   }
   for (uint32_t i = tid; i <= f.mask1; i += 1024) f.seen[i] = kNoList;
   for (uint32_t i = tid; i < 1u << f.log2; i += 1024) f.head[i] = f.count[i] = 0;
   for (uint32_t i = tid; i < 1u << f.blog2; i += 1024) f.bits[i] = 0;
   for (uint32_t i = tid; i < np; i += 1024) f.l_np[i] = 0;
+  if (tid == 0) s_used = 0;
   if (tid < kListCtrs) f.ctr[tid] = 0;
   if (tid < kListQueues) f.long_n[tid * kListPad] = 0;
   __threadfence();
@@ -2341,38 +2347,54 @@ __global__ __launch_bounds__(1024) void k_list_parents(ListFilter fg, Signal sg)
       }
       if (old == off) break;
     }
-    f.next[i] = s;  // (the list's slot, for now)
+    f.p_slot[i] = s;  // (the list's slot, for now)
   }
   if (units) atomicAdd(&f.ctr[kListUnits], (unsigned long long)units);
   __threadfence();
   __syncthreads();
   for (uint32_t i = tid; i < np; i += 1024) {
-    const uint32_t l = f.seen_list[f.next[i]];
+    const uint32_t l = f.seen_list[f.p_slot[i]];
     f.p_list[i] = l;
     f.p_tgt[i] = f.ec >= 0 ? (uint32_t)f.P[(uint64_t)f.info[i].x * f.pc + (uint32_t)f.ec] : f.target;
     atomicAdd(&f.l_np[l], 1u);
   }
   __threadfence();
   __syncthreads();
+  // each parent's slot and its place among the slot's parents (in seen, which is done with)
+  uint32_t *rank = f.seen;
   for (uint32_t i = tid; i < np; i += 1024) {
     const uint32_t l = f.p_list[i], t = f.p_tgt[i];
-    if (f.ec >= 0 ? (int32_t)t < 0 : !f.target_ok) continue;
-    const uint32_t h = pair_hash(l, t);
-    atomicOr(&f.bits[h >> (32 - f.blog2)], pair_bits(h));
-    for (uint32_t s = pair_slot(f, h);; s = (s + 1) & ((1u << f.log2) - 1)) {
-      const uint32_t old = atomicCAS(&f.head[s], 0u, i + 1);
-      if (old != 0 && (f.p_list[old - 1] != l || f.p_tgt[old - 1] != t)) continue;
-      f.next[i] = old ? atomicExch(&f.head[s], i + 1) : 0u;
-      atomicAdd(&f.count[s], 1u);
-      break;
+    uint32_t slot = kNoList;
+    if (f.ec >= 0 ? (int32_t)t >= 0 : f.target_ok) {
+      const uint32_t h = pair_hash(l, t);
+      atomicOr(&f.bits[h >> (32 - f.blog2)], pair_bits(h));
+      for (slot = pair_slot(f, h);; slot = (slot + 1) & ((1u << f.log2) - 1)) {
+        const uint32_t old = atomicCAS(&f.head[slot], 0u, i + 1);
+        if (old == 0 || (f.p_list[old - 1] == l && f.p_tgt[old - 1] == t)) break;
+      }
+      rank[i] = atomicAdd(&f.count[slot], 1u);
     }
+    f.p_slot[i] = slot;
   }
   __threadfence();
   __syncthreads();
+  for (uint32_t s0 = 0; s0 < 1u << f.log2; s0 += 1024) {  // (one add a wave)
+    const uint32_t s = s0 + tid;
+    const uint32_t n = s < 1u << f.log2 ? __hip_atomic_load(&f.count[s], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0u;
+    const uint32_t inc = wave_incl_scan32(n);
+    uint32_t base = 0;
+    if (lane_id() == kWave - 1) base = atomicAdd(&s_used, inc);
+    base = lane63(base);
+    if (n) f.start[s] = base + inc - n;
+  }
+  __syncthreads();
+  for (uint32_t i = tid; i < np; i += 1024)
+    if (f.p_slot[i] != kNoList) f.order[f.start[f.p_slot[i]] + rank[i]] = i;
   if (lds) {
     for (uint32_t i = tid; i < 1u << f.log2; i += 1024) {
       fg.head[i] = f.head[i];
       fg.count[i] = f.count[i];
+      fg.start[i] = f.start[i];
     }
     for (uint32_t i = tid; i < 1u << f.blog2; i += 1024) fg.bits[i] = f.bits[i];
     for (uint32_t i = tid; i < np; i += 1024) fg.l_np[i] = f.l_np[i];
@@ -2386,25 +2408,51 @@ __global__ __launch_bounds__(1024) void k_list_parents(ListFilter fg, Signal sg)
   }
 }
 
-// Element idx (x) of the filter list of list l's entry j (e): the parents of
-// l with target x keep row (parent, j).
-__device__ __forceinline__ void list_element(const GraphView &g, uint64_t estart, const ListFilter &f, uint32_t l,
-                                             uint32_t j, uint32_t e, uint32_t off, uint32_t deg, uint32_t idx,
-                                             uint32_t x) {
+// Element idx (x) of a filter list that list l's entry found: the parents of
+// l with target x, order[first .. first + the result), keep a row each.
+__device__ __forceinline__ uint32_t list_match(const GraphView &g, uint64_t estart, const ListFilter &f, uint32_t l,
+                                               uint32_t off, uint32_t idx, uint32_t x, uint32_t &first) {
   const uint32_t h = pair_hash(l, x), b = pair_bits(h);
-  if ((f.bits[h >> (32 - f.blog2)] & b) != b) return;
+  if ((f.bits[h >> (32 - f.blog2)] & b) != b) return 0;
   for (uint32_t s = pair_slot(f, h);; s = (s + 1) & ((1u << f.log2) - 1)) {
     const uint32_t hd = f.head[s];
-    if (!hd) return;
+    if (!hd) return 0;
     if (f.p_list[hd - 1] != l || f.p_tgt[hd - 1] != x) continue;
-    if (idx && g.edges[estart + off + idx - 1] == x) return;  // (only the first match counts)
-    const uint32_t n = f.count[s];
-    uint64_t k = atomicAdd(&f.ctr[kListKept], (unsigned long long)n);
-    atomicAdd(&f.ctr[kListSpared], (unsigned long long)n * (deg - (idx + 1)));
-    if (k + n <= f.cap)
-      for (uint32_t p = hd; p; p = f.next[p - 1])
-        f.kept[k++] = make_uint4((uint32_t)(f.excl[p - 1] + j), p - 1, e, 0u);
-    return;
+    if (idx && g.edges[estart + off + idx - 1] == x) return 0;  // (only the first match counts)
+    first = f.start[s];
+    return f.count[s];
+  }
+}
+
+// The whole wave: each lane's n parents from order[first] on keep their row
+// of entry j (e); spare: the edges that each of them need not examine. The
+// wave's rows are one sequence, a lane each, and take one add of the
+// counters. (A lane that wrote its own n rows one after another, along a
+// chain of parents, took 250 ns a row: 4096 parents of one list, one target
+// for all, 1196 us a call, now 328.)
+__device__ __forceinline__ void list_keep(const ListFilter &f, uint32_t n, uint32_t first, uint32_t j, uint32_t e,
+                                          uint32_t spare) {
+  if (!wave_ballot(n != 0)) return;
+  const uint32_t lane = lane_id();
+  const uint32_t inc = wave_incl_scan32(n), all = lane63(inc), before = inc - n;
+  const uint64_t spared = lane63_64(wave_incl_scan((uint64_t)n * spare));
+  uint64_t base = 0;
+  if (lane == 0) {
+    base = atomicAdd(&f.ctr[kListKept], (unsigned long long)all);
+    atomicAdd(&f.ctr[kListSpared], (unsigned long long)spared);
+  }
+  base = shfl64(base, 0);
+  for (uint32_t t0 = 0; t0 < all && base + t0 < f.cap; t0 += kWave) {  // (wave-uniform)
+    const uint32_t t = t0 + lane;
+    uint32_t src = 0;  // the last lane whose rows start at or before t (lanes without any share their next's)
+#pragma unroll
+    for (uint32_t step = kWave / 2; step; step >>= 1)
+      if (shfl32(before, src + step) <= t) src += step;
+    const uint32_t q = shfl32(first, src) + (t - shfl32(before, src)), kj = shfl32(j, src), ke = shfl32(e, src);
+    if (t < all && base + t < f.cap) {
+      const uint32_t p = f.order[q];
+      f.kept[base + t] = make_uint4((uint32_t)(f.excl[p] + kj), p, ke, 0u);
+    }
   }
 }
 
@@ -2471,17 +2519,13 @@ __global__ __launch_bounds__(kBlock) void k_list_filter(GraphView g, ListFilter 
   }
 #pragma unroll
   for (int r = 0; r < RD; r++) {
-    if (deg[r] && deg[r] <= kListInline) list_element(g, m.edge_start, f, l[r], j[r], e[r], off[r], deg[r], 0, x[r]);
+    uint32_t n = 0, first = 0;
+    if (deg[r] && deg[r] <= kListInline) n = list_match(g, m.edge_start, f, l[r], off[r], 0, x[r], first);
+    list_keep(f, n, first, j[r], e[r], deg[r] - 1);
     // the further elements of all lanes' lists as one sequence, a lane each
     const uint32_t more = deg[r] > 1 && deg[r] <= kListInline ? deg[r] - 1 : 0u;
     if (wave_ballot(more != 0)) {
-      uint32_t inc = more;
-#pragma unroll
-      for (int d = 1; d < kWave; d <<= 1) {
-        const uint32_t y = shfl32(inc, (lane - d) & 63);
-        if (lane >= (uint32_t)d) inc += y;
-      }
-      const uint32_t all = lane63(inc), before = inc - more;
+      const uint32_t inc = wave_incl_scan32(more), all = lane63(inc), before = inc - more;
       for (uint32_t t0 = 0; t0 < all; t0 += kWave) {  // (wave-uniform)
         const uint32_t t = t0 + lane;
         uint32_t src = 0;  // the last lane whose elements start at or before t (lanes without any share their next's)
@@ -2490,7 +2534,8 @@ __global__ __launch_bounds__(kBlock) void k_list_filter(GraphView g, ListFilter 
           if (shfl32(before, src + step) <= t) src += step;
         const uint32_t q = t - shfl32(before, src) + 1, ol = shfl32(l[r], src), oo = shfl32(off[r], src);
         const uint32_t od = shfl32(deg[r], src), oj = shfl32(j[r], src), oe = shfl32(e[r], src);
-        if (t < all) list_element(g, m.edge_start, f, ol, oj, oe, oo, od, q, g.edges[m.edge_start + oo + q]);
+        n = t < all ? list_match(g, m.edge_start, f, ol, oo, q, g.edges[m.edge_start + oo + q], first) : 0u;
+        list_keep(f, n, first, oj, oe, od - (q + 1));
       }
     }
     if (deg[r] > kListInline) {
@@ -2533,7 +2578,9 @@ __global__ __launch_bounds__(kBlock) void k_list_long(GraphView g, ListFilter f,
 #pragma unroll
     for (int u = 0; u < (int)(kListChunk / kBlock); u++) {
       const uint32_t q = it.w + threadIdx.x + u * kBlock;
-      if (q < it.z) list_element(g, m.edge_start, f, l, j, e, it.y, it.z, q, v[u]);
+      uint32_t first = 0;
+      const uint32_t n = q < it.z ? list_match(g, m.edge_start, f, l, it.y, q, v[u], first) : 0u;
+      list_keep(f, n, first, j, e, it.z - (q + 1));
     }
   }
 }

@@ -1449,9 +1449,9 @@ int wkg_ctx::step_filter_lists(int mode, const wkg_table *in, int pid, int dir, 
   f.mask1 = (1u << f.log2) - 1;
   f.blog2 = std::max(log2_up(np), 8u);  // 32 bits per parent
   f.cap = std::min<uint64_t>(std::min<uint64_t>(R, fanout_kept_cap), kListKeptCap);
-  // counters | lists x 4, parents x 3 | two hash tables of two words a slot | bits
+  // counters | lists x 4, parents x 4 | two hash tables, of two and three words a slot | bits
   const uint64_t slots = 1ull << f.log2;
-  const uint64_t words = 2 * kListCtrs + 2 * kListQueues * kListPad + 7 * np + 4 * slots + (1ull << f.blog2);
+  const uint64_t words = 2 * kListCtrs + 2 * kListQueues * kListPad + 8 * np + 5 * slots + (1ull << f.blog2);
   uint32_t *buf = (uint32_t *)pool->alloc(words * 4, s, err_slot());
   if (!buf) return WKG_ENOMEM;
   uint32_t *w = buf;
@@ -1468,11 +1468,13 @@ int wkg_ctx::step_filter_lists(int mode, const wkg_table *in, int pid, int dir, 
   f.l_np = take(np);
   f.p_list = take(np);
   f.p_tgt = take(np);
-  f.next = take(np);
+  f.p_slot = take(np);
+  f.order = take(np);
   f.seen = take(slots);
   f.seen_list = take(slots);
   f.head = take(slots);
   f.count = take(slots);
+  f.start = take(slots);
   f.bits = take(1ull << f.blog2);
   char *rows = nullptr;  // kept rows | long lists
   auto done = [&](int r) {
