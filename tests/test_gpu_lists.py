@@ -18,7 +18,7 @@ DEGREES = [0, 1, 1, 2, 3, 4, 5, 15, 16, 17, 18, 63, 0, 1, 0, 1, 2, 1, 1, 0]
 def graph():
     rng = np.random.default_rng(6)
     tri = []
-    for h, n in enumerate((ENTRIES, 1500, 700, 300)):  # subject VB + h: a list of n entries
+    for h, n in enumerate((ENTRIES, 1500, 700, 300, 0, 40)):  # subject VB + h: a list of n entries
         e = VB + 1000 + np.sort(rng.choice(ENTRIES, size=n, replace=False))
         tri += [(VB + h, 2, x) for x in e]
     for i in range(ENTRIES):  # entry i's filter list
@@ -60,3 +60,27 @@ def test_fused_filter(graph, parents, targets, pid):
         out, fused, e1, e2 = dev.k2u_filter(dt, 0, 2, 1, kind, pid, 1, end, const)
         assert fused and (e1, e2) == (ex1, ex2)
         assert np.array_equal(out.to_host().reshape(want.shape), want)
+
+
+@pytest.mark.parametrize("parents,subject", [(2000, VB + 5), (7000, VB + 1), (20000, VB + 2)])
+def test_declined_before_any_launch(graph, parents, subject):
+    """Short lists, and more parents than one workgroup should hash, go to the
+    other forms without a launch of the list form."""
+    gs, dev = graph
+    tab = np.full((parents, 2), subject, dtype=np.int32)
+    tab[:, 1] = VB + 10000 + np.arange(parents) % 6000
+    mid, _ = oracle.run_step(gs, [VB, 2, 1, -1, -1, 2, 1, -3], 1, tab, threads=8)
+    want, wex = oracle.run_step(gs, [VB, 2, 1, -1, -3, 3, 1, -2], 1, mid, threads=8)
+    dt = dev.table(tab)
+    launches = []
+    try:
+        for on in (True, False):
+            dev.set_fanout_blocks(on)
+            dev.profile(True)
+            out, fused, _, ex = dev.k2u_filter(dt, 0, 2, 1, STEP_K2K, 3, 1, 1, -1)
+            assert fused and ex == wex and np.array_equal(out.to_host().reshape(want.shape), want)
+            launches.append(dev.profile_read("lineage")[0])
+            dev.profile(False)
+    finally:
+        dev.set_fanout_blocks(True)
+    assert launches[0] == launches[1]

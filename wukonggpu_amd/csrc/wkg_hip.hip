@@ -1149,7 +1149,13 @@ int wkg_ctx::step_filter_fanout(int mode, const wkg_table *in, int pid, int dir,
   const uint64_t np = in->lin_n, R = in->rows;
   const int c = in->cols;
   if (np == 0 || np > kMaxParents) return kNotTaken;
-  if (sorted && fanout_blocks) {
+  // The list form costs about 60 us and 26 ns a parent (k_list_parents is one
+  // workgroup), the others at least 150 us and 3.3 ns per 1000 pairs: 4096
+  // parents of 4.3M pairs 132-157 us against 157-265, 20000 of 400M pairs 570
+  // against 1480, but 16384 of 4.3M pairs 295-375 against 234-470 and 100000 of
+  // 200M 1780 against 1080. Lists that average under 256 entries go to the
+  // row tiles below (100000 parents of 60: 820 us; hashed first, 2900).
+  if (sorted && fanout_blocks && np <= 4096 + R / 8192 && np * 256 <= R) {
     const int lrc = step_filter_lists(mode, in, pid, dir, ec, cval, s, out, expanded);
     if (lrc != kOtherForm) return lrc;
   }
@@ -1453,7 +1459,7 @@ int wkg_ctx::step_filter_lists(int mode, const wkg_table *in, int pid, int dir, 
   const uint64_t slots = 1ull << f.log2;
   const uint64_t words = 2 * kListCtrs + 2 * kListQueues * kListPad + 8 * np + 5 * slots + (1ull << f.blog2);
   uint32_t *buf = (uint32_t *)pool->alloc(words * 4, s, err_slot());
-  if (!buf) return WKG_ENOMEM;
+  if (!buf) return kOtherForm;
   uint32_t *w = buf;
   auto take = [&](uint64_t n) {
     uint32_t *r = w;
@@ -1492,11 +1498,11 @@ int wkg_ctx::step_filter_lists(int mode, const wkg_table *in, int pid, int dir, 
   if ((rc = wait_signal(sg, s))) return done(rc);
   const uint64_t total = rb_host()[0], nl = rb_host()[1], units = rb_host()[2];
   if (R < 4 * total) return done(kNotTaken);
-  if (units * 256 > R) return done(kOtherForm);  // short lists: their rows, tile by tile
+  if (units * 256 > R) return done(kOtherForm);  // short lists among long ones: their rows, tile by tile
   f.long_cap = (total / 16 + 65536) / kListQueues;
   const uint64_t nwg = (total + kListTile - 1) / kListTile, nex = nwg * (kBlock / kWave);
   rows = (char *)pool->alloc((f.cap + kListQueues * f.long_cap) * 16 + nex * 8, s, err_slot());
-  if (!rows) return done(WKG_ENOMEM);
+  if (!rows) return done(kOtherForm);
   f.kept = (uint4 *)rows;
   f.longs = f.kept + f.cap;
   f.ex = (uint64_t *)(f.longs + kListQueues * f.long_cap);
