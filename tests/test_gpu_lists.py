@@ -84,3 +84,34 @@ def test_declined_before_any_launch(graph, parents, subject):
     finally:
         dev.set_fanout_blocks(True)
     assert launches[0] == launches[1]
+
+
+@pytest.mark.parametrize("pid,parents,targets", [(3, 900, 400), (4, 700, 1)])
+def test_kept_list_overflow(graph, pid, parents, targets):
+    """Kept rows at the size of their list and one more: then they go through
+    bits, from a written fan-out and from one that never was."""
+    gs, dev = graph
+    rng = np.random.default_rng(pid)
+    tab = np.stack([VB + rng.integers(0, 4, parents), VB + 10000 + rng.integers(0, targets, parents)], axis=1)
+    tab = tab.astype(np.int32)
+    mid, _ = oracle.run_step(gs, [VB, 2, 1, -1, -1, 2, 1, -3], 1, tab, threads=8)
+    want, wex = oracle.run_step(gs, [VB, 2, 1, -1, -3, pid, 1, -2], 1, mid, threads=8)
+    kept = want.shape[0]
+    dt = dev.table(tab)
+    wide, _ = dev.k2u(dt, 0, 2, 1)
+    try:
+        for cap, over in ((kept, kept > 32768), (kept - 1, True), (1, True)):
+            dev.set_fanout_blocks(True, cap)
+            dev.profile(True)
+            out, fused, _, ex = dev.k2u_filter(dt, 0, 2, 1, STEP_K2K, pid, 1, 1, -1)
+            assert fused and ex == wex and np.array_equal(out.to_host().reshape(want.shape), want)
+            out, ex = dev.k2k(wide, 2, pid, 1, 1)
+            assert ex == wex and np.array_equal(out.to_host().reshape(want.shape), want)
+            out, ex = dev.k2c(wide, 2, pid, 1, VB + 10000)
+            c, cex = oracle.run_step(gs, [VB, 2, 1, -1, -3, pid, 1, VB + 10000], 1, mid, threads=8)
+            assert ex == cex and np.array_equal(out.to_host().reshape(c.shape), c)
+            assert dev.profile_read("fanout_filters")[2] == 3  # each by one form alone
+            assert dev.profile_read("fanout_kept_overflow")[2] == 2 * over + (c.shape[0] > min(cap, 32768))
+            dev.profile(False)
+    finally:
+        dev.set_fanout_blocks(True)

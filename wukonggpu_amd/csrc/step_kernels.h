@@ -1999,8 +1999,8 @@ __global__ __launch_bounds__(kBlock) void k_fanout_units(GraphView g, StepParams
   }
 }
 
-// The fan-out filter for long shared lists of many kept rows (or unsorted
-// filter lists), a block of list entries at a time: a workgroup takes kFBRows entries of one distinct list and up to
+// The fan-out filter for long shared lists of unsorted images or of many
+// parents, a block of list entries at a time: a workgroup takes kFBRows entries of one distinct list and up to
 // kFBGroup (= 64) of the parents sharing that list, and tests every parent
 // against every entry's list, holding the block in registers:
 //  - thread t takes entries t, t + 256, ...: their D entries are read once;
@@ -2233,7 +2233,7 @@ __global__ __launch_bounds__(kBlock) void k_fanout_blocks(GraphView g, StepParam
   }
 }
 
-// ---- the fan-out filter through its lists (sorted images, few kept rows) ----
+// ---- the fan-out filter through its lists (sorted images) ----
 // The pairs (parent, list entry) of a fan-out need not be tested one by one:
 // row (i, j) is kept iff parent i's target is in the filter list of entry j
 // of i's list, so the targets of the parents sharing a list are hashed once
@@ -2243,7 +2243,8 @@ __global__ __launch_bounds__(kBlock) void k_fanout_blocks(GraphView g, StepParam
 // per element of the lists it finds, whatever the number of parents; the work
 // count is, per list, its parents times its entries' degrees, less what the
 // reference's early exit spares each kept row. Kept rows are listed
-// unordered and ranked by their row (k_list_rows).
+// unordered and ranked by their row (k_list_rows); where they are more than
+// the list holds, the pass is made again with a bit per row.
 // What bounds it: the probe of the distinct entries (cache misses); nearly
 // all lookups end at a bit of a filter in L1. The cycle's closing filter over
 // 1.9G pairs of 1.6M distinct entries: its query 618 -> 205 us (pair by pair in
@@ -2269,6 +2270,7 @@ struct ListFilter {
   unsigned long long *ctr;            // kList*
   uint4 *kept;                        // (row, parent, entry, 0)
   uint64_t cap;
+  uint32_t *rbits;                    // or a bit per row (BITS)
   uint64_t *ex;                       // per wave of k_list_filter: its share of the work count
   // long filter lists in kListQueues queues of long_cap items (a workgroup
   // appends to one of them: thousands of workgroups adding to one word take
@@ -2283,7 +2285,8 @@ constexpr uint32_t kNoList = 0xffffffffu;  // (segments hold fewer than 2^32 edg
 constexpr uint32_t kListInline = 16;       // longer filter lists go to k_list_long,
 constexpr uint32_t kListChunk = 1024;      // this many elements an item
 constexpr int kListTile = 512;             // list entries per workgroup
-constexpr uint64_t kListKeptCap = 32768;   // ranking compares all kept rows with each other
+constexpr uint64_t kListKeptCap = 32768;   // ranking compares all kept rows with each other; more: bits
+constexpr int kListBitRows = 1024;         // rows per tile of the bits
 
 __device__ __forceinline__ uint32_t pair_hash(uint32_t l, uint32_t t) {
   uint32_t h = (l * 0x9E3779B1u + t) * 0x85EBCA6Bu;
@@ -2430,6 +2433,7 @@ __device__ __forceinline__ uint32_t list_match(const GraphView &g, uint64_t esta
 // counters. (A lane that wrote its own n rows one after another, along a
 // chain of parents, took 250 ns a row: 4096 parents of one list, one target
 // for all, 1196 us a call, now 328.)
+template <bool BITS>
 __device__ __forceinline__ void list_keep(const ListFilter &f, uint32_t n, uint32_t first, uint32_t j, uint32_t e,
                                           uint32_t spare) {
   if (!wave_ballot(n != 0)) return;
@@ -2442,20 +2446,24 @@ __device__ __forceinline__ void list_keep(const ListFilter &f, uint32_t n, uint3
     atomicAdd(&f.ctr[kListSpared], (unsigned long long)spared);
   }
   base = shfl64(base, 0);
-  for (uint32_t t0 = 0; t0 < all && base + t0 < f.cap; t0 += kWave) {  // (wave-uniform)
+  for (uint32_t t0 = 0; t0 < all && (BITS || base + t0 < f.cap); t0 += kWave) {  // (wave-uniform)
     const uint32_t t = t0 + lane;
     uint32_t src = 0;  // the last lane whose rows start at or before t (lanes without any share their next's)
 #pragma unroll
     for (uint32_t step = kWave / 2; step; step >>= 1)
       if (shfl32(before, src + step) <= t) src += step;
     const uint32_t q = shfl32(first, src) + (t - shfl32(before, src)), kj = shfl32(j, src), ke = shfl32(e, src);
-    if (t < all && base + t < f.cap) {
-      const uint32_t p = f.order[q];
-      f.kept[base + t] = make_uint4((uint32_t)(f.excl[p] + kj), p, ke, 0u);
+    if (t < all && (BITS || base + t < f.cap)) {
+      const uint32_t p = f.order[q], row = (uint32_t)(f.excl[p] + kj);
+      if (BITS) atomicOr(&f.rbits[row >> 5], 1u << (row & 31));
+      else f.kept[base + t] = make_uint4(row, p, ke, 0u);
     }
   }
 }
 
+// With BITS every kept row becomes a bit of rbits; else it is listed, and once
+// the list has overflown the rest of the pass is not needed.
+template <bool BITS>
 __global__ __launch_bounds__(kBlock) void k_list_filter(GraphView g, ListFilter f, uint32_t total, uint32_t nl,
                                                         uint32_t block0) {
   const uint32_t block = block0 + blockIdx.x;
@@ -2471,6 +2479,7 @@ __global__ __launch_bounds__(kBlock) void k_list_filter(GraphView g, ListFilter 
       if (lane == 0) f.ex[block * (kBlock / kWave) + wave] = 0;
       return;
     }
+    if (!BITS && __hip_atomic_load(&f.ctr[kListKept], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) > f.cap) return;
     // the wave's first list, and whether all its rows are in it
     const uint32_t l0 = (uint32_t)wave_last_le(nl, w0, [&](uint64_t i) -> uint64_t { return f.l_base[i]; });
     const uint32_t b0 = f.l_base[l0], o0 = f.l_off[l0];
@@ -2521,7 +2530,7 @@ __global__ __launch_bounds__(kBlock) void k_list_filter(GraphView g, ListFilter 
   for (int r = 0; r < RD; r++) {
     uint32_t n = 0, first = 0;
     if (deg[r] && deg[r] <= kListInline) n = list_match(g, m.edge_start, f, l[r], off[r], 0, x[r], first);
-    list_keep(f, n, first, j[r], e[r], deg[r] - 1);
+    list_keep<BITS>(f, n, first, j[r], e[r], deg[r] - 1);
     // the further elements of all lanes' lists as one sequence, a lane each
     const uint32_t more = deg[r] > 1 && deg[r] <= kListInline ? deg[r] - 1 : 0u;
     if (wave_ballot(more != 0)) {
@@ -2535,7 +2544,7 @@ __global__ __launch_bounds__(kBlock) void k_list_filter(GraphView g, ListFilter 
         const uint32_t q = t - shfl32(before, src) + 1, ol = shfl32(l[r], src), oo = shfl32(off[r], src);
         const uint32_t od = shfl32(deg[r], src), oj = shfl32(j[r], src), oe = shfl32(e[r], src);
         n = t < all ? list_match(g, m.edge_start, f, ol, oo, q, g.edges[m.edge_start + oo + q], first) : 0u;
-        list_keep(f, n, first, oj, oe, od - (q + 1));
+        list_keep<BITS>(f, n, first, oj, oe, od - (q + 1));
       }
     }
     if (deg[r] > kListInline) {
@@ -2552,6 +2561,7 @@ __global__ __launch_bounds__(kBlock) void k_list_filter(GraphView g, ListFilter 
 
 // The long filter lists, a chunk per workgroup at a time; the first workgroup
 // also adds up the work count.
+template <bool BITS>
 __global__ __launch_bounds__(kBlock) void k_list_long(GraphView g, ListFilter f, uint32_t nl, uint32_t nex) {
   const uint32_t queue = blockIdx.x % kListQueues;
   const uint64_t all = f.long_n[queue * kListPad], n = all < f.long_cap ? all : f.long_cap;
@@ -2564,6 +2574,7 @@ __global__ __launch_bounds__(kBlock) void k_list_long(GraphView g, ListFilter f,
     (void)block_excl_scan(v, s_tmp, sum);
     if (threadIdx.x == 0) f.ctr[kListEx] = sum;
   }
+  if (!BITS && f.ctr[kListKept] > f.cap) return;  // (a wave as a whole; no barrier below)
   const DevMeta ml = g.meta[f.lpid], m = g.meta[f.pid];
   for (uint64_t i = blockIdx.x / kListQueues; i < n; i += gridDim.x / kListQueues) {
     const uint4 it = f.longs[queue * f.long_cap + i];
@@ -2580,9 +2591,25 @@ __global__ __launch_bounds__(kBlock) void k_list_long(GraphView g, ListFilter f,
       const uint32_t q = it.w + threadIdx.x + u * kBlock;
       uint32_t first = 0;
       const uint32_t n = q < it.z ? list_match(g, m.edge_start, f, l, it.y, q, v[u], first) : 0u;
-      list_keep(f, n, first, j, e, it.z - (q + 1));
+      list_keep<BITS>(f, n, first, j, e, it.z - (q + 1));
     }
   }
+}
+
+// Kept rows of each tile of 1024 rows, for the tile scan; the work count is
+// the list pass's.
+__global__ __launch_bounds__(kBlock) void k_bit_tiles(StepParams p, const uint32_t *bits) {
+  const uint64_t lt = blockIdx.x * (uint64_t)kBlock + threadIdx.x;
+  if (lt >= p.ntiles) return;
+  const uint4 *w = (const uint4 *)(bits + lt * (kListBitRows / 32));
+  uint32_t n = 0;
+#pragma unroll
+  for (int k = 0; k < kListBitRows / 128; k++) {
+    const uint4 v = gload(w + k);
+    n += __builtin_popcount(v.x) + __builtin_popcount(v.y) + __builtin_popcount(v.z) + __builtin_popcount(v.w);
+  }
+  p.tile_sum[lt] = p.tile_nz[lt] = n;
+  p.tile_ex[lt] = 0;
 }
 
 // The n kept rows in row order: the 16 lanes of a group count the rows before

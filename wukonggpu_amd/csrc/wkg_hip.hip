@@ -1423,11 +1423,11 @@ int wkg_ctx::step_filter_fanout(int mode, const wkg_table *in, int pid, int dir,
   return done(WKG_OK);
 }
 
-// step_filter_fanout's form for long shared lists of a sorted image with at
-// most kListKeptCap kept rows (kOtherForm: not so; kNotTaken: no form is
-// worth it): every distinct list entry is probed once and the elements of its
-// filter list are looked up among the targets of the list's parents. The
-// lists are deduplicated and the targets hashed on the device.
+// step_filter_fanout's form for long shared lists of a sorted image
+// (kOtherForm: not so; kNotTaken: no form is worth it): every distinct list
+// entry is probed once and the elements of its filter list are looked up among
+// the targets of the list's parents. The lists are deduplicated and the
+// targets hashed on the device.
 int wkg_ctx::step_filter_lists(int mode, const wkg_table *in, int pid, int dir, int ec, int64_t cval, hipStream_t s,
                                wkg_table **out, uint64_t *expanded) {
   const uint64_t np = in->lin_n, R = in->rows;
@@ -1482,8 +1482,10 @@ int wkg_ctx::step_filter_lists(int mode, const wkg_table *in, int pid, int dir, 
   f.count = take(slots);
   f.start = take(slots);
   f.bits = take(1ull << f.blog2);
-  char *rows = nullptr;  // kept rows | long lists
+  char *rows = nullptr;     // kept rows | long lists
+  uint64_t *scr = nullptr;  // kept rows as bits, their tile scan
   auto done = [&](int r) {
+    if (scr) pool->release(scr, s);
     if (rows) pool->release(rows, s);
     pool->release(buf, s);
     return r;
@@ -1507,27 +1509,86 @@ int wkg_ctx::step_filter_lists(int mode, const wkg_table *in, int pid, int dir, 
   f.longs = f.kept + f.cap;
   f.ex = (uint64_t *)(f.longs + kListQueues * f.long_cap);
   const GraphView g = view();
-  {
+  auto pass = [&](auto bits) {
     // per distinct entry: itself, its tag word and its bucket's line
     ProfScope ps(this, s, "fanout_filter", 140.0 * (double)total);
     const uint64_t per = std::max<uint64_t>(thread_launch_rows() / kListTile, 1);  // split launches, as the probe's
     for (uint64_t b0 = 0; b0 < nwg; b0 += per)
-      k_list_filter<<<(unsigned)std::min(per, nwg - b0), kBlock, 0, s>>>(g, f, (uint32_t)total, (uint32_t)nl,
-                                                                         (uint32_t)b0);
-    k_list_long<<<16 * kListQueues, kBlock, 0, s>>>(g, f, (uint32_t)nl, (uint32_t)nex);
-  }
+      k_list_filter<bits.value><<<(unsigned)std::min(per, nwg - b0), kBlock, 0, s>>>(g, f, (uint32_t)total,
+                                                                                    (uint32_t)nl, (uint32_t)b0);
+    k_list_long<bits.value><<<16 * kListQueues, kBlock, 0, s>>>(g, f, (uint32_t)nl, (uint32_t)nex);
+  };
+  pass(std::false_type{});
   if ((le = hipGetLastError()) != hipSuccess)
     return done(fail(WKG_EDEVICE, "fan-out filter launch failed: %s", hipGetErrorString(le)));
   uint64_t c[kListCtrs];
   if ((rc = read_words((const uint64_t *)f.ctr, kListCtrs, s, c))) return done(rc);
+  // More kept rows than the list holds: the pass once more with a bit per
+  // row, then the row tiles' compaction. (Calls over 20M pairs: 1M kept rows
+  // 300 us, all kept 1520; through the block filter, which such a pass was
+  // once left to, 3950 and 4730 us. At the line, 33k kept rows 237 us ranked
+  // and 36k rows 241 us through bits.)
+  const bool bits = c[kListKept] > f.cap;
+  StepParams p{};
+  if (bits) {
+    prof_add_bytes("fanout_kept_overflow", 1.0);  // a count
+    constexpr uint64_t TR = kListBitRows;
+    const uint64_t ntiles = (R + TR - 1) / TR, nchunks = (ntiles + kScanChunk - 1) / kScanChunk;
+    const uint64_t bit_words = ntiles * TR / 64, scan_words = 4 + 3 * ntiles + 3 * nchunks;
+    if (!(scr = (uint64_t *)pool->alloc((bit_words + scan_words) * 8, s, err_slot()))) return done(kOtherForm);
+    f.rbits = (uint32_t *)scr;
+    p.T = in->d;
+    p.c = (uint32_t)in->cols;
+    p.R = R;
+    p.totals = scr + bit_words;
+    p.tile_sum = p.totals + 4;
+    p.tile_nz = p.tile_sum + ntiles;
+    p.tile_ex = p.tile_nz + ntiles;
+    p.chunk_sum = p.tile_ex + ntiles;
+    p.chunk_nz = p.chunk_sum + nchunks;
+    p.chunk_ex = p.chunk_nz + nchunks;
+    p.ntiles = ntiles;
+    auto zero = [&](void *a, uint64_t n) {
+      k_zero_u64<<<(unsigned)std::min<uint64_t>((n + kBlock - 1) / kBlock, 65535), kBlock, 0, s>>>((uint64_t *)a, n);
+    };
+    zero(f.ctr, kListCtrs + kListQueues * kListPad);  // (the queues' counters follow)
+    zero(f.rbits, bit_words);
+    pass(std::true_type{});
+    {
+      ProfScope ps(this, s, "scan_tiles", (double)R / 8 + 72.0 * (double)ntiles);
+      k_bit_tiles<<<(unsigned)((ntiles + kBlock - 1) / kBlock), kBlock, 0, s>>>(p, f.rbits);
+      k_scan_chunks<<<(unsigned)nchunks, kBlock, 0, s>>>(p);
+      if (nchunks > 1) k_scan_top<<<1, kBlock, 0, s>>>(p, nchunks);
+    }
+    if ((le = hipGetLastError()) != hipSuccess)
+      return done(fail(WKG_EDEVICE, "fan-out filter launch failed: %s", hipGetErrorString(le)));
+    if ((rc = read_words((const uint64_t *)f.ctr, kListCtrs, s, c))) return done(rc);
+  }
+  if (c[kListLost]) return done(kOtherForm);
   const uint64_t kept = c[kListKept];
-  if (kept > f.cap || c[kListLost]) return done(kOtherForm);
   wkg_table *t = nullptr;
   if ((rc = new_table(kept, in->cols, s, &t))) return done(rc);
   if (kept) {
     ProfScope ps(this, s, "compact", 8.0 * (double)kept * in->cols);
-    constexpr uint64_t per = kBlock / kRankLanes;
-    k_list_rows<<<(unsigned)((kept + per - 1) / per), kBlock, 0, s>>>(f, (uint32_t)kept, t->d);
+    if (bits) {
+      FanoutFilter ff{};
+      ff.excl = f.excl;
+      ff.info = f.info;
+      ff.np = np;
+      ff.P = f.P;
+      ff.pc = f.pc;
+      p.O = t->d;
+      const uint64_t per = std::max<uint64_t>(thread_launch_rows() / kListBitRows, 4) & ~uint64_t(3);
+      for (uint64_t t0 = 0; t0 < p.ntiles; t0 += per) {
+        p.tile0 = t0;
+        const unsigned grid = (unsigned)((std::min<uint64_t>(per, p.ntiles - t0) + kBlock / kWave - 1) / (kBlock / kWave));
+        if (in->d) k_compact_bits<kListBitRows><<<grid, kBlock, 0, s>>>(p, f.rbits, nullptr);
+        else k_compact_lineage<kListBitRows><<<grid, kBlock, 0, s>>>(g, p, f.rbits, nullptr, ff, h_meta[in->lin_pid].edge_start);
+      }
+    } else {
+      constexpr uint64_t per = kBlock / kRankLanes;
+      k_list_rows<<<(unsigned)((kept + per - 1) / per), kBlock, 0, s>>>(f, (uint32_t)kept, t->d);
+    }
   }
   if ((le = hipGetLastError()) != hipSuccess) {
     drop_table(t);
