@@ -79,3 +79,30 @@ def test_steps(graph, rows, cols, hits, kind):
         want, wex = oracle.run_step(gs, pre + [-1, 2, 1, -2], 1, tab, threads=8)
         f, ex = dev.k2k(dt, 0, 2, 1, 1)
         assert ex == wex and np.array_equal(f.to_host(), want)
+
+
+@pytest.mark.parametrize("rows,hits", [(300, 1), (60000, 10), (60000, 0)])
+def test_held_results_cost_their_size(graph, rows, hits):
+    """A few hundred small results held at once take their own size of the
+    table budget, whatever room their steps began with."""
+    gs, _ = graph
+    budget = 64 << 20
+    dev = Device(0, table_budget_bytes=budget)
+    try:
+        dev.load(gs)
+        tab = _table(np.random.default_rng(rows), rows, 2, hits, SINGLE, 30000)
+        want, _ = oracle.run_step(gs, [VB, 2, 1, -1, -1, 2, 1, -3], 1, tab)
+        dt = dev.table(tab)
+        base = dev.pool_stats()["live_bytes"]
+        held = [dev.k2u(dt, 0, 2, 1)[0] for _ in range(400)]
+        assert dev.pool_stats()["live_bytes"] - base <= 400 * 4096 + budget // 256
+        rest = (budget - base - 400 * 4096) // (2 << 20) * (2 << 20)  # large blocks are multiples of 2 MiB
+        big = dev.table(np.zeros((rest // 4, 1), dtype=np.int32))  # the rest of the budget is there to use
+        for t in held:
+            assert np.array_equal(t.to_host().reshape(want.shape), want)
+            t.free()
+        big.free()
+        t, _ = dev.k2u(dt, 0, 2, 1)
+        assert np.array_equal(t.to_host().reshape(want.shape), want)
+    finally:
+        dev.close()

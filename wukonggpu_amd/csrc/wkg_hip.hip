@@ -87,19 +87,19 @@ void *Pool::alloc(size_t bytes, hipStream_t s, std::string &err) {
   for (auto it = cached.lower_bound(sz); it != cached.end() && it->first <= sz + sz / 4; ++it) {
     if (it->second.stream != s) continue;
     void *p = it->second.ptr;
-    live[p] = it->first;
+    live[p] = Live{it->first, 0};
     live_bytes += it->first;
     cached_bytes -= it->first;
     cached.erase(it);
     return p;
   }
-  if (live_bytes + sz > budget) {
+  if (live_bytes - rest_bytes + sz > budget) {
     err = "HBM table budget exhausted: need " + std::to_string(sz) + " bytes, " +
-          std::to_string(budget - std::min<uint64_t>(budget, live_bytes)) + " of " + std::to_string(budget) +
+          std::to_string(budget - std::min<uint64_t>(budget, live_bytes - rest_bytes)) + " of " + std::to_string(budget) +
           " left";
     return nullptr;
   }
-  if (live_bytes + cached_bytes + sz > budget) trim_locked(sz);
+  if (live_bytes - rest_bytes + cached_bytes + sz > budget) trim_locked(sz);
   void *p = nullptr;
   hipError_t e = hipMalloc(&p, sz);
   if (e != hipSuccess) {
@@ -111,7 +111,7 @@ void *Pool::alloc(size_t bytes, hipStream_t s, std::string &err) {
     err = std::string("hipMalloc failed: ") + hipGetErrorString(e);
     return nullptr;
   }
-  live[p] = sz;
+  live[p] = Live{sz, 0};
   live_bytes += sz;
   mallocs++;
   return p;
@@ -124,11 +124,32 @@ void Pool::release(void *p, hipStream_t s) {
   std::lock_guard<std::mutex> lk(mu);
   auto it = live.find(p);
   if (it == live.end()) return;
-  const size_t sz = it->second;
+  const size_t sz = it->second.size;
+  rest_bytes -= it->second.rest;
   live.erase(it);
   live_bytes -= sz;
   cached.emplace(sz, Cached{p, s});
   cached_bytes += sz;
+}
+
+bool Pool::keep_part(void *p, size_t bytes, size_t used) {
+  if (BumpArena *b = thread_arena()) {
+    auto up = [](uint64_t n) { return (n + 255) & ~uint64_t(255); };
+    const uint64_t at = (uint64_t)((char *)p - b->base);
+    if ((char *)p >= b->base && at < b->cap) {
+      if (at + up(bytes) == b->used) b->used = at + up(used);
+      return true;
+    }
+  }
+  std::lock_guard<std::mutex> lk(mu);
+  auto it = live.find(p);
+  if (it == live.end()) return true;
+  const size_t want = round_size(used);
+  const uint64_t rest = it->second.size > want ? it->second.size - want : 0;
+  if (rest_bytes - it->second.rest + rest > budget / 256) return false;
+  rest_bytes += rest - it->second.rest;
+  it->second.rest = rest;
+  return true;
 }
 
 // Frees cached blocks, largest first, until `need` more bytes fit the
@@ -138,7 +159,7 @@ void Pool::trim_locked(uint64_t need) {
   if (cached.empty()) return;
   trims++;
   (void)hipDeviceSynchronize();
-  while (!cached.empty() && (need == 0 || live_bytes + cached_bytes + need > budget)) {
+  while (!cached.empty() && (need == 0 || live_bytes - rest_bytes + cached_bytes + need > budget)) {
     auto it = std::prev(cached.end());
     (void)hipFree(it->second.ptr);
     cached_bytes -= it->first;
@@ -775,25 +796,25 @@ int wkg_ctx::follow_pass(int mode, const wkg_table *in, int sc, int pid, int dir
                          hipStream_t s, ProbePass &pp, wkg_table **out) {
   const uint64_t R = in->rows;
   const int c = in->cols, out_cols = mode == kModeK2U ? c + 1 : c;
-  // the guess: twice the input's rows, within 8 MB and a 256th of the table
-  // budget (a table keeps its memory when it turns out shorter)
-  uint64_t cap = R;
-  if (mode == kModeK2U) {
-    uint64_t most = std::min<uint64_t>(8ull << 20, pool->budget / 256);
-    if (table_limit) most = std::min(most, table_limit);
-    cap = std::min(std::max<uint64_t>(2 * R, 8192), most / (4 * (uint64_t)out_cols));
-  }
   wkg_table *t = nullptr;
+  uint64_t cap = R;
   int rc;
-  if (cap && (rc = new_table(cap, out_cols, s, &t))) {
-    if (mode != kModeK2U) return rc;
-    t = nullptr;
-    cap = 0;
-  }
+  if (mode != kModeK2U && (rc = new_table(R, c, s, &t))) return rc;
   StepParams p{};
   if ((rc = pass_setup(this, mode, in, sc, pid, dir, ec, cval, t ? t->d : nullptr, s, tr, 0, pp, p))) {
     drop_table(t);
     return rc;
+  }
+  if (mode == kModeK2U) {
+    // the guess: twice the input's rows, within 8 MB and a 256th of the table
+    // budget, of memory that the step can do without (so it comes last)
+    uint64_t most = std::min<uint64_t>(8ull << 20, pool->budget / 256);
+    if (table_limit) most = std::min(most, table_limit);
+    cap = std::min(std::max<uint64_t>(2 * R, 8192), most / (4 * (uint64_t)out_cols));
+    if (cap && new_table(cap, out_cols, s, &t)) {
+      t = nullptr;
+      cap = 0;
+    }
   }
   pp.hits = p.hits;
   pp.tr = tr;
@@ -845,6 +866,7 @@ int wkg_ctx::follow_pass(int mode, const wkg_table *in, int sc, int pid, int dir
     prof_add_bytes("probe_rows", (double)R);           // and rows looked up
   }
   if (rows > cap) {
+    if (t) (void)pool->keep_part(t->d, t->bytes, 0);
     drop_table(t);
     t = nullptr;
   } else {
@@ -854,12 +876,30 @@ int wkg_ctx::follow_pass(int mode, const wkg_table *in, int sc, int pid, int dir
       if (pp.lin) pool->release(pp.lin, s);
       pp.lin = nullptr;
     }
+    const uint64_t bytes = rows * (uint64_t)out_cols * 4;
+    if (mode == kModeK2U && t && !pool->keep_part(t->d, t->bytes, bytes)) {
+      // (the guesses hold too much already: the rows to a table of their size, a short copy; none: an empty one)
+      wkg_table *fit = nullptr;
+      if (!new_table(rows, out_cols, s, &fit)) {
+        if (rows) {
+          ProfScope ps(this, s, "fit", 2.0 * (double)bytes);
+          le = hipMemcpyAsync(fit->d, t->d, bytes, hipMemcpyDeviceToDevice, s);
+        }
+        drop_table(t);
+        t = fit;
+        if (le != hipSuccess) {
+          release_pass(pp, s);
+          drop_table(t);
+          return fail(WKG_EDEVICE, "table copy failed: %s", hipGetErrorString(le));
+        }
+      }
+    }
     if (!t && (rc = new_table(0, out_cols, s, &t))) {
       release_pass(pp, s);
       return rc;
     }
     t->rows = rows;
-    t->bytes = rows * (uint64_t)out_cols * 4;
+    t->bytes = bytes;
   }
   *out = t;
   return WKG_OK;

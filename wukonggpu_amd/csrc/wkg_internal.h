@@ -48,6 +48,12 @@ struct Pool {
   ~Pool();
   void *alloc(size_t bytes, hipStream_t s, std::string &err);
   void release(void *p, hipStream_t s);
+  // A live block of which only the first `used` bytes are wanted any more.
+  // The rest stays with it (true) while such rests are at most a 256th of the
+  // budget together, and does not count against the budget; false: too
+  // much, the caller moves to a block that fits. The thread's latest bump
+  // allocation (of `bytes`) is cut.
+  bool keep_part(void *p, size_t bytes, size_t used);
   void trim();
   void stats(uint64_t *live, uint64_t *cached_b, uint64_t *nmalloc, uint64_t *ntrim);
   uint64_t budget;
@@ -55,10 +61,14 @@ struct Pool {
   uint64_t mallocs = 0, trims = 0;  // hipMalloc calls; cache drops (each a device synchronisation)
 
  private:
+  struct Live {
+    size_t size, rest;  // rest: kept but not wanted
+  };
   void trim_locked(uint64_t need);
   std::mutex mu;
   std::multimap<size_t, Cached> cached;
-  std::unordered_map<void *, size_t> live;
+  std::unordered_map<void *, Live> live;
+  uint64_t rest_bytes = 0;
 };
 
 struct ArmScan;  // wkg_ctx::arm_lift
