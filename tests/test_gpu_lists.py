@@ -14,8 +14,8 @@ ENTRIES = 3000  # of the longest list; entry i is vertex VB + 1000 + i
 DEGREES = [0, 1, 1, 2, 3, 4, 5, 15, 16, 17, 18, 63, 0, 1, 0, 1, 2, 1, 1, 0]
 
 
-@pytest.fixture(scope="module")
-def graph():
+@pytest.fixture(scope="module", params=[True, False], ids=["tags", "no tags"])
+def graph(request):
     rng = np.random.default_rng(6)
     tri = []
     for h, n in enumerate((ENTRIES, 1500, 700, 300, 0, 40)):  # subject VB + h: a list of n entries
@@ -29,7 +29,7 @@ def graph():
             tri.append((VB + 1000 + i, 4, VB + 10000))  # predicate 4: half of all entries, one object
     gs = GStore.build(Triples.from_arrays(*(np.array(x) for x in zip(*tri))))
     dev = Device(0)
-    dev.load(gs)
+    dev.load(gs, graph_budget_bytes=0 if request.param else gs.image_nbytes())  # (which leaves no room for tag words)
     dev.set_group_filter_rows(0)
     yield gs, dev
     dev.close()

@@ -430,7 +430,7 @@ int wkg_ctx::finish_resident(uint32_t flags, hipStream_t s, uint64_t tag_bytes) 
       d_tags = nullptr;
     }
   }
-  resident_bytes = num_slots * 16 + std::max<uint64_t>(num_edges, 1) * 4;
+  resident_bytes = num_slots * 16 + std::max<uint64_t>(num_edges, 1) * 4 + (d_tags ? num_main * sizeof(uint2) : 0);
   loaded = true;
   if (!budget_request) {  // default table budget: 75% of what is left
     size_t fr = 0, tot = 0;
