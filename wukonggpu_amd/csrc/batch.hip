@@ -34,14 +34,17 @@ __device__ __forceinline__ uint32_t find_item(const uint64_t *base, uint32_t n, 
   return lo;
 }
 
-template <bool SORTED, bool FRAMED>
+// (A resident graph without tag words takes the whole-bucket form: the tagged
+// form's walks have two reads in flight, not eight, and with every key
+// walking a 3M-row step took 201 us in it, 191 so.)
+template <bool SORTED, bool FRAMED, bool TAGS>
 __global__ __launch_bounds__(kBlock, 3) void k_batch_probe(GraphView g, const BatchItem *items,
                                                         const uint64_t *tile_base, uint32_t n) {
   __shared__ uint32_t s_q;
   if (threadIdx.x == 0) s_q = find_item(tile_base, n, blockIdx.x);
   __syncthreads();
   const uint32_t q = s_q;
-  probe_tile<kTileRows, SORTED, FRAMED>(g, items[q].p, blockIdx.x - tile_base[q]);
+  probe_tile<kTileRows, SORTED, FRAMED, TAGS>(g, items[q].p, blockIdx.x - tile_base[q]);
 }
 
 __global__ __launch_bounds__(kBlock) void k_batch_scan(const BatchItem *items) {
@@ -199,11 +202,14 @@ extern "C" int wkg_step_batch(wkg_ctx *ctx, int n, const wkg_step_desc *steps, v
     for (int i = 0; i < n; i++) pb += (double)R[i] * (4.0 + (mode[i] == kModeK2K ? 4.0 : 0.0) + 128.0);
     ProfScope ps(ctx, s, "batch_probe", pb);
     if (ctx->framed) {
-      if (ctx->sorted) k_batch_probe<true, true><<<(unsigned)NT, kBlock, 0, s>>>(g, d_items, d_tileb, n);
-      else k_batch_probe<false, true><<<(unsigned)NT, kBlock, 0, s>>>(g, d_items, d_tileb, n);
+      if (ctx->sorted) k_batch_probe<true, true, false><<<(unsigned)NT, kBlock, 0, s>>>(g, d_items, d_tileb, n);
+      else k_batch_probe<false, true, false><<<(unsigned)NT, kBlock, 0, s>>>(g, d_items, d_tileb, n);
+    } else if (!g.tags) {
+      if (ctx->sorted) k_batch_probe<true, false, false><<<(unsigned)NT, kBlock, 0, s>>>(g, d_items, d_tileb, n);
+      else k_batch_probe<false, false, false><<<(unsigned)NT, kBlock, 0, s>>>(g, d_items, d_tileb, n);
     } else {
-      if (ctx->sorted) k_batch_probe<true, false><<<(unsigned)NT, kBlock, 0, s>>>(g, d_items, d_tileb, n);
-      else k_batch_probe<false, false><<<(unsigned)NT, kBlock, 0, s>>>(g, d_items, d_tileb, n);
+      if (ctx->sorted) k_batch_probe<true, false, true><<<(unsigned)NT, kBlock, 0, s>>>(g, d_items, d_tileb, n);
+      else k_batch_probe<false, false, true><<<(unsigned)NT, kBlock, 0, s>>>(g, d_items, d_tileb, n);
     }
   }
   {

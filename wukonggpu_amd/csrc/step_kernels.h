@@ -161,11 +161,10 @@ __device__ __forceinline__ void rows_member(const GraphView &g, uint64_t estart,
 // step). Wave w owns the tile's rows [w * TR/4, (w+1) * TR/4) and probes
 // them 64 consecutive rows per round, carrying the last key across rounds.
 // Writes the tile's list of rows with output and its sums.
-template <int TR, bool SORTED, bool FRAMED>
+template <int TR, bool SORTED, bool FRAMED, bool TAGS = !FRAMED>
 __device__ __forceinline__ void probe_tile(const GraphView &g, const StepParams &p, uint64_t lt) {
   constexpr int kRounds = TR / kBlock;  // one row per lane per round
   constexpr int kRowsPerThread = TR / kBlock;
-  constexpr bool kTags = !FRAMED;
   static_assert(TR % kBlock == 0, "tile rows must be a multiple of the block");
   __shared__ uint32_t s_cnt[TR];  // degree, or kept flag
   __shared__ uint32_t s_aux[TR];  // segment offset, or edges examined
@@ -195,7 +194,7 @@ __device__ __forceinline__ void probe_tile(const GraphView &g, const StepParams 
       if (p.key) key = p.key;
       else if (cells[rd] >= 0) key = make_key((uint32_t)cells[rd], p.pid, p.dir);
     }
-    return probe_plan<FRAMED, kTags>(g, m, key, before63);
+    return probe_plan<FRAMED, TAGS>(g, m, key, before63);
   };
   uint32_t probed = 0;
   // The wave's rows' degrees and list offsets into s_cnt and s_aux. Round rd
@@ -204,8 +203,8 @@ __device__ __forceinline__ void probe_tile(const GraphView &g, const StepParams 
   ProbePlan pl[3];
   pl[0] = plan(0, 0);
   if (kRounds > 1) pl[1] = plan(1, lane63_64(pl[0].key));
-  probe_pick<kTags>(g, pl[0]);
-  if constexpr (kTags) {
+  probe_pick<TAGS>(g, pl[0]);
+  if constexpr (TAGS) {
     // The rows that must walk (few) wait for all rounds: their walks, chains
     // of dependent reads, then run once per tile, not once per round.
     uint4 *kb = s_wp[wave].kb;
@@ -220,7 +219,7 @@ __device__ __forceinline__ void probe_tile(const GraphView &g, const StepParams 
     for (int rd = 0; rd < kRounds; rd++) {
       const uint32_t local = wave * kWaveRows + rd * kWave + lane;
       if (rd + 2 < kRounds) pl[(rd + 2) % 3] = plan(rd + 2, lane63_64(pl[(rd + 1) % 3].key));
-      if (rd + 1 < kRounds && pl[(rd + 1) % 3].leaders) probe_pick<kTags>(g, pl[(rd + 1) % 3]);
+      if (rd + 1 < kRounds && pl[(rd + 1) % 3].leaders) probe_pick<TAGS>(g, pl[(rd + 1) % 3]);
       const ProbePlan &cur = pl[rd % 3];
       lead[rd] = cur.leaders;
       have[rd] = wave_ballot(cur.key != 0);
@@ -268,8 +267,8 @@ __device__ __forceinline__ void probe_tile(const GraphView &g, const StepParams 
     for (int rd = 0; rd < kRounds; rd++) {
       const uint32_t local = wave * kWaveRows + rd * kWave + lane;
       if (rd + 2 < kRounds) pl[(rd + 2) % 3] = plan(rd + 2, lane63_64(pl[(rd + 1) % 3].key));
-      if (rd + 1 < kRounds) probe_pick<kTags>(g, pl[(rd + 1) % 3]);
-      probed += probe_finish<FRAMED, kTags>(g, m, pl[rd % 3], s_wp[wave], s_cnt[local], s_aux[local], carry);
+      if (rd + 1 < kRounds) probe_pick<TAGS>(g, pl[(rd + 1) % 3]);
+      probed += probe_finish<FRAMED, TAGS>(g, m, pl[rd % 3], s_wp[wave], s_cnt[local], s_aux[local], carry);
     }
   }
   if (p.mode != kModeK2U) {  // filters: kept flags and edges examined in their place
