@@ -87,6 +87,21 @@ def test_split_many_tiles_property(dev_small):
     assert np.array_equal(got[np.argsort(got[:, 1])], t)
 
 
+@pytest.mark.parametrize("rows", [1, 1023, 1025, 8192 * 1024, 8192 * 1024 + 1, 5 * 2048 * 1024 - 1, 5 * 2048 * 1024 + 1])
+def test_split_scan_edges(dev_small, rows):
+    # slabs of 1024 rows: a part's counts in one chunk up to 8192 of them, then in chunks of 2048
+    t = np.stack([np.random.default_rng(rows).integers(1, 1 << 30, rows, dtype=np.int32),
+                  np.arange(rows, dtype=np.int32)], axis=1)
+    d = dev_small.table(t)
+    for n in (3, 64):
+        out, prow, phead = dev_small.table_split(d, 0, n)
+        owner = t[:, 0] % n
+        assert np.array_equal(out.to_host(), t[np.argsort(owner, kind="stable")])
+        want = np.bincount(owner, minlength=n)
+        assert np.array_equal(prow, want) and np.array_equal(phead, np.cumsum(want) - want)
+        out.free()
+
+
 def test_concat_edges(dev_small):
     rng = np.random.default_rng(5)
     a, b = _table(rng, 10, 2), _table(rng, 3, 2)
