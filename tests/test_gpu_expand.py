@@ -51,6 +51,7 @@ CASES = [
     (1100003, 3, 300000, (DOZEN, 4000)),   # fans out: from the lists, with lineage
     (1100003, 2, 150, (HUB, 1)),           # fans out more: by merge path
     (1100000, 2, 0, (SINGLE, 30000)),
+    (1100000, 46, 330000, (DOZEN, 4000)),  # an input past the memory-side cache that fans out: by merge path
 ]
 
 

@@ -682,6 +682,12 @@ struct ArmScan {
 // output row (2M rows to 18M of 4 cells: 81 + 13 + 10 us by merge path, 77 + 14
 // from the lists), so the merge path is ahead above some 50 output rows per
 // row with edges; 24M keys to 9.3M rows of 2 cells: 127 + 54 + 15 and 128 + 14 us.
+// The merge path is also ahead where the input no longer stays in the 256 MB
+// memory-side cache between the probe and the expand and the output is 3.5
+// times as large (streams): its smaller blocks, at odd offsets, write 3.1
+// TB/s between the reads from memory, the others 2.7 (a step of 3M rows of
+// 40 cells to 21.6M: 1309 and 1430 us; 3M rows of 12 cells, in the cache, the
+// other way round: 399 before and 347 from the lists).
 // star: the step's column is one of the input's lineage parent (star_arm); an
 // output that filters may decide by groups then gets its groups, found
 // while the expand runs.
@@ -689,6 +695,7 @@ int wkg_ctx::finish_k2u(const wkg_table *in, int pid, ProbePass &pp, hipStream_t
                         bool star) {
   const uint64_t E = pp.cnt[0], nz = pp.cnt[2];
   const int out_cols = in->cols + 1;
+  const bool streams = in->bytes >= (192ull << 20) && 2 * E * out_cols >= 7 * in->rows * (uint64_t)in->cols;
   int rc = WKG_OK;
   ArmScan arm;
   if (table_limit && in->rows >= 2 && E * (uint64_t)out_cols * 4 > table_limit) {  // (one row cannot be split)
@@ -698,7 +705,7 @@ int wkg_ctx::finish_k2u(const wkg_table *in, int pid, ProbePass &pp, hipStream_t
         !(rc = compact_pass(pp, s)))
       rc = arm_lift(in, pp, s, arm);
     if (rc) {
-    } else if (!pp.lin && E < (1ull << 32) && E < 32 * nz) {
+    } else if (!pp.lin && E < (1ull << 32) && E < 32 * nz && !streams) {
       if (wants_lineage(in, nz, E)) rc = lineage_rows(pp, s);
       if (!rc) rc = expand_hits(in, pid, pp, s, t);
     } else if (!(rc = compact_pass(pp, s))) {
