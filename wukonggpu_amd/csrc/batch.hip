@@ -199,7 +199,7 @@ extern "C" int wkg_step_batch(wkg_ctx *ctx, int n, const wkg_step_desc *steps, v
   const GraphView g = ctx->view();
   if (NT) {
     double pb = 0;
-    for (int i = 0; i < n; i++) pb += (double)R[i] * (4.0 + (mode[i] == kModeK2K ? 4.0 : 0.0) + 128.0);
+    for (int i = 0; i < n; i++) pb += (double)R[i] * (4.0 + (mode[i] == kModeK2K ? 4.0 : 0.0)) + ctx->key_bytes((double)R[i], (double)R[i]);
     ProfScope ps(ctx, s, "batch_probe", pb);
     if (ctx->framed) {
       if (ctx->sorted) k_batch_probe<true, true, false><<<(unsigned)NT, kBlock, 0, s>>>(g, d_items, d_tileb, n);

@@ -2270,7 +2270,7 @@ struct ListFilter {
   uint4 *kept;                        // (row, parent, entry, 0)
   uint64_t cap;
   uint32_t *rbits;                    // or a bit per row (BITS)
-  uint64_t *ex;                       // per wave of k_list_filter: its share of the work count
+  uint64_t *ex;                       // per wave of k_list_filter: its share of the work count (mod 2^64)
   // long filter lists in kListQueues queues of long_cap items (a workgroup
   // appends to one of them: thousands of workgroups adding to one word take
   // 17 ns each): (entry, offset, degree, first element)
@@ -2278,7 +2278,8 @@ struct ListFilter {
   unsigned long long *long_n;         // per queue, kListPad words apart
   uint64_t long_cap;
 };
-enum { kListSums = 0, kListUnits, kListKept, kListEx, kListSpared, kListLost, kListCtrs };
+// (kListBits: three words, the totals of the tile scan over the bits)
+enum { kListSums = 0, kListUnits, kListKept, kListEx, kListSpared, kListLost, kListBits, kListCtrs = kListBits + 3 };
 constexpr uint32_t kListQueues = 64, kListPad = 16;
 constexpr uint32_t kNoList = 0xffffffffu;  // (segments hold fewer than 2^32 edges)
 constexpr uint32_t kListInline = 16;       // longer filter lists go to k_list_long,
@@ -2380,14 +2381,15 @@ __global__ __launch_bounds__(1024) void k_list_parents(ListFilter fg, Signal sg)
   }
   __threadfence();
   __syncthreads();
-  for (uint32_t s0 = 0; s0 < 1u << f.log2; s0 += 1024) {  // (one add a wave)
-    const uint32_t s = s0 + tid;
-    const uint32_t n = s < 1u << f.log2 ? __hip_atomic_load(&f.count[s], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0u;
+  for (uint32_t i0 = 0; i0 < np; i0 += 1024) {  // a slot's first parent makes its room (one add a wave)
+    const uint32_t i = i0 + tid, slot = i < np ? f.p_slot[i] : kNoList;
+    const bool lead = slot != kNoList && rank[i] == 0;
+    const uint32_t n = lead ? __hip_atomic_load(&f.count[slot], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0u;
     const uint32_t inc = wave_incl_scan32(n);
     uint32_t base = 0;
     if (lane_id() == kWave - 1) base = atomicAdd(&s_used, inc);
     base = lane63(base);
-    if (n) f.start[s] = base + inc - n;
+    if (lead) f.start[slot] = fg.start[slot] = base + inc - n;
   }
   __syncthreads();
   for (uint32_t i = tid; i < np; i += 1024)
@@ -2396,7 +2398,6 @@ __global__ __launch_bounds__(1024) void k_list_parents(ListFilter fg, Signal sg)
     for (uint32_t i = tid; i < 1u << f.log2; i += 1024) {
       fg.head[i] = f.head[i];
       fg.count[i] = f.count[i];
-      fg.start[i] = f.start[i];
     }
     for (uint32_t i = tid; i < 1u << f.blog2; i += 1024) fg.bits[i] = f.bits[i];
     for (uint32_t i = tid; i < np; i += 1024) fg.l_np[i] = f.l_np[i];
@@ -2427,41 +2428,42 @@ __device__ __forceinline__ uint32_t list_match(const GraphView &g, uint64_t esta
 }
 
 // The whole wave: each lane's n parents from order[first] on keep their row
-// of entry j (e); spare: the edges that each of them need not examine. The
-// wave's rows are one sequence, a lane each, and take one add of the
-// counters. (A lane that wrote its own n rows one after another, along a
-// chain of parents, took 250 ns a row: 4096 parents of one list, one target
-// for all, 1196 us a call, now 328.)
+// of entry j (e); spare: the edges that each of them need not examine, summed
+// per lane in spared. The wave's rows are one sequence, a lane each, and take
+// one add of the counter. (A lane that wrote its own n rows one after another,
+// along a chain of parents, took 250 ns a row: 4096 parents of one list, one
+// target for all, 1196 us a call, now 328.) With BITS every kept row becomes a
+// bit of rbits; else it is listed, and false says that the list has
+// overflown: the rest of the pass is not needed.
 template <bool BITS>
-__device__ __forceinline__ void list_keep(const ListFilter &f, uint32_t n, uint32_t first, uint32_t j, uint32_t e,
-                                          uint32_t spare) {
-  if (!wave_ballot(n != 0)) return;
+__device__ __forceinline__ bool list_keep(const ListFilter &f, uint32_t n, uint32_t first, uint32_t j, uint32_t e,
+                                          uint32_t spare, uint64_t &spared) {
+  if (!wave_ballot(n != 0)) return true;
   const uint32_t lane = lane_id();
   const uint32_t inc = wave_incl_scan32(n), all = lane63(inc), before = inc - n;
-  const uint64_t spared = lane63_64(wave_incl_scan((uint64_t)n * spare));
+  spared += (uint64_t)n * spare;
   uint64_t base = 0;
-  if (lane == 0) {
-    base = atomicAdd(&f.ctr[kListKept], (unsigned long long)all);
-    atomicAdd(&f.ctr[kListSpared], (unsigned long long)spared);
+  if constexpr (!BITS) {
+    if (lane == 0) base = atomicAdd(&f.ctr[kListKept], (unsigned long long)all);
+    base = shfl64(base, 0);
+    if (base + all > f.cap) return false;
   }
-  base = shfl64(base, 0);
-  for (uint32_t t0 = 0; t0 < all && (BITS || base + t0 < f.cap); t0 += kWave) {  // (wave-uniform)
+  for (uint32_t t0 = 0; t0 < all; t0 += kWave) {  // (wave-uniform)
     const uint32_t t = t0 + lane;
     uint32_t src = 0;  // the last lane whose rows start at or before t (lanes without any share their next's)
 #pragma unroll
     for (uint32_t step = kWave / 2; step; step >>= 1)
       if (shfl32(before, src + step) <= t) src += step;
     const uint32_t q = shfl32(first, src) + (t - shfl32(before, src)), kj = shfl32(j, src), ke = shfl32(e, src);
-    if (t < all && (BITS || base + t < f.cap)) {
+    if (t < all) {
       const uint32_t p = f.order[q], row = (uint32_t)(f.excl[p] + kj);
       if (BITS) atomicOr(&f.rbits[row >> 5], 1u << (row & 31));
       else f.kept[base + t] = make_uint4(row, p, ke, 0u);
     }
   }
+  return true;
 }
 
-// With BITS every kept row becomes a bit of rbits; else it is listed, and once
-// the list has overflown the rest of the pass is not needed.
 template <bool BITS>
 __global__ __launch_bounds__(kBlock) void k_list_filter(GraphView g, ListFilter f, uint32_t total, uint32_t nl,
                                                         uint32_t block0) {
@@ -2478,7 +2480,6 @@ __global__ __launch_bounds__(kBlock) void k_list_filter(GraphView g, ListFilter 
       if (lane == 0) f.ex[block * (kBlock / kWave) + wave] = 0;
       return;
     }
-    if (!BITS && __hip_atomic_load(&f.ctr[kListKept], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) > f.cap) return;
     // the wave's first list, and whether all its rows are in it
     const uint32_t l0 = (uint32_t)wave_last_le(nl, w0, [&](uint64_t i) -> uint64_t { return f.l_base[i]; });
     const uint32_t b0 = f.l_base[l0], o0 = f.l_off[l0];
@@ -2518,7 +2519,7 @@ __global__ __launch_bounds__(kBlock) void k_list_filter(GraphView g, ListFilter 
     if (r + 1 < RD) probe_pick<true>(g, pl[(r + 1) % 3]);
     (void)probe_finish<false, true>(g, m, pl[r % 3], s_wp[wave], deg[r], off[r], carry);
   }
-  uint64_t ex = 0;
+  uint64_t ex = 0, spared = 0;  // work counts: all lists whole, and what kept rows need not examine
   uint32_t x[RD];
 #pragma unroll
   for (int r = 0; r < RD; r++) {
@@ -2529,7 +2530,7 @@ __global__ __launch_bounds__(kBlock) void k_list_filter(GraphView g, ListFilter 
   for (int r = 0; r < RD; r++) {
     uint32_t n = 0, first = 0;
     if (deg[r] && deg[r] <= kListInline) n = list_match(g, m.edge_start, f, l[r], off[r], 0, x[r], first);
-    list_keep<BITS>(f, n, first, j[r], e[r], deg[r] - 1);
+    if (!list_keep<BITS>(f, n, first, j[r], e[r], deg[r] - 1, spared)) return;
     // the further elements of all lanes' lists as one sequence, a lane each
     const uint32_t more = deg[r] > 1 && deg[r] <= kListInline ? deg[r] - 1 : 0u;
     if (wave_ballot(more != 0)) {
@@ -2543,7 +2544,7 @@ __global__ __launch_bounds__(kBlock) void k_list_filter(GraphView g, ListFilter 
         const uint32_t q = t - shfl32(before, src) + 1, ol = shfl32(l[r], src), oo = shfl32(off[r], src);
         const uint32_t od = shfl32(deg[r], src), oj = shfl32(j[r], src), oe = shfl32(e[r], src);
         n = t < all ? list_match(g, m.edge_start, f, ol, oo, q, g.edges[m.edge_start + oo + q], first) : 0u;
-        list_keep<BITS>(f, n, first, oj, oe, od - (q + 1));
+        if (!list_keep<BITS>(f, n, first, oj, oe, od - (q + 1), spared)) return;
       }
     }
     if (deg[r] > kListInline) {
@@ -2554,7 +2555,7 @@ __global__ __launch_bounds__(kBlock) void k_list_filter(GraphView g, ListFilter 
         f.longs[q * f.long_cap + b + c] = make_uint4(f.l_base[l[r]] + j[r], off[r], deg[r], c * kListChunk);
     }
   }
-  ex = lane63_64(wave_incl_scan(ex));
+  ex = lane63_64(wave_incl_scan(ex - spared));
   if (lane == 0) f.ex[block * (kBlock / kWave) + wave] = ex;
 }
 
@@ -2573,7 +2574,7 @@ __global__ __launch_bounds__(kBlock) void k_list_long(GraphView g, ListFilter f,
     (void)block_excl_scan(v, s_tmp, sum);
     if (threadIdx.x == 0) f.ctr[kListEx] = sum;
   }
-  if (!BITS && f.ctr[kListKept] > f.cap) return;  // (a wave as a whole; no barrier below)
+  uint64_t spared = 0;
   const DevMeta ml = g.meta[f.lpid], m = g.meta[f.pid];
   for (uint64_t i = blockIdx.x / kListQueues; i < n; i += gridDim.x / kListQueues) {
     const uint4 it = f.longs[queue * f.long_cap + i];
@@ -2590,9 +2591,11 @@ __global__ __launch_bounds__(kBlock) void k_list_long(GraphView g, ListFilter f,
       const uint32_t q = it.w + threadIdx.x + u * kBlock;
       uint32_t first = 0;
       const uint32_t n = q < it.z ? list_match(g, m.edge_start, f, l, it.y, q, v[u], first) : 0u;
-      list_keep<BITS>(f, n, first, j, e, it.z - (q + 1));
+      if (!list_keep<BITS>(f, n, first, j, e, it.z - (q + 1), spared)) return;  // (a wave as a whole; no barrier below)
     }
   }
+  spared = lane63_64(wave_incl_scan(spared));
+  if (spared && lane_id() == 0) atomicAdd(&f.ctr[kListSpared], (unsigned long long)spared);
 }
 
 // Kept rows of each tile of 1024 rows, for the tile scan; the work count is

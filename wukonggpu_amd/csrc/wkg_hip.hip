@@ -503,9 +503,9 @@ int wkg_ctx::probe_pass(int mode, const wkg_table *in, int sc, int pid, int dir,
   const GraphView g = view();
   {
     // the input table (4 R c: its rows are read whole, as cache lines); K2U
-    // adds one 128-byte bucket per key probed and a 16-byte hit per row with
-    // edges once the counts are known; the filters are charged one bucket per row
-    const double b = 4.0 * (double)R * c + (mode == kModeK2U ? 0.0 : 128.0 * (double)R);
+    // adds its keys' lookups and a 16-byte hit per row with edges once the
+    // counts are known; the filters are charged a present key per row
+    const double b = 4.0 * (double)R * c + (mode == kModeK2U ? 0.0 : key_bytes((double)R, (double)R));
     ProfScope ps(this, s, mode == kModeK2U ? "probe" : "probe_filter", b);
     launch_probe(TR, framed, sorted || mode == kModeK2U, g, p, s);
   }
@@ -530,7 +530,7 @@ int wkg_ctx::probe_pass(int mode, const wkg_table *in, int sc, int pid, int dir,
   memcpy(pp.cnt, rb_host(), 3 * sizeof(uint64_t));
   if (mode == kModeK2U) {
     if (compact) prof_add_bytes("finalize", 32.0 * pp.cnt[2]);
-    prof_add_bytes("probe", 128.0 * (double)pp.cnt[1] + 16.0 * (double)pp.cnt[2]);
+    prof_add_bytes("probe", key_bytes((double)pp.cnt[1], (double)std::min(pp.cnt[1], pp.cnt[2])) + 16.0 * (double)pp.cnt[2]);
     prof_add_bytes("probe_keys", (double)pp.cnt[1]);  // counts, not bytes: keys probed (run leaders)
     prof_add_bytes("probe_rows", (double)R);           // and rows looked up
   } else if (O) {
@@ -828,7 +828,7 @@ int wkg_ctx::follow_pass(int mode, const wkg_table *in, int sc, int pid, int dir
   pp.ntiles = p.ntiles;
   const GraphView g = view();
   {
-    const double b = 4.0 * (double)R * c + (mode == kModeK2U ? 0.0 : 128.0 * (double)R);
+    const double b = 4.0 * (double)R * c + (mode == kModeK2U ? 0.0 : key_bytes((double)R, (double)R));
     ProfScope ps(this, s, mode == kModeK2U ? "probe" : "probe_filter", b);
     launch_probe(tr, framed, sorted || mode == kModeK2U, g, p, s);
   }
@@ -868,7 +868,7 @@ int wkg_ctx::follow_pass(int mode, const wkg_table *in, int sc, int pid, int dir
   memcpy(pp.cnt, rb_host(), 3 * sizeof(uint64_t));
   const uint64_t rows = pp.cnt[0], nz = pp.cnt[2];
   if (mode == kModeK2U) {
-    prof_add_bytes("probe", 128.0 * (double)pp.cnt[1] + 16.0 * (double)nz);
+    prof_add_bytes("probe", key_bytes((double)pp.cnt[1], (double)std::min(pp.cnt[1], nz)) + 16.0 * (double)nz);
     prof_add_bytes("probe_keys", (double)pp.cnt[1]);  // counts, not bytes: keys probed (run leaders)
     prof_add_bytes("probe_rows", (double)R);           // and rows looked up
   }
@@ -1572,23 +1572,22 @@ int wkg_ctx::step_filter_lists(int mode, const wkg_table *in, int pid, int dir, 
   if ((rc = read_words((const uint64_t *)f.ctr, kListCtrs, s, c))) return done(rc);
   // More kept rows than the list holds: the pass once more with a bit per
   // row, then the row tiles' compaction. (Calls over 20M pairs: 1M kept rows
-  // 300 us, all kept 1520; through the block filter, which such a pass was
-  // once left to, 3950 and 4730 us. At the line, 33k kept rows 237 us ranked
-  // and 36k rows 241 us through bits.)
+  // 210 us, all kept 1480; through the block filter, which such a pass was
+  // once left to, 3950 and 4730 us. At the line the ranking takes 110 us and
+  // the second pass with its scan 45 over 80000 list entries, 120 over 2.8M.)
   const bool bits = c[kListKept] > f.cap;
   StepParams p{};
   if (bits) {
     prof_add_bytes("fanout_kept_overflow", 1.0);  // a count
     constexpr uint64_t TR = kListBitRows;
     const uint64_t ntiles = (R + TR - 1) / TR, nchunks = (ntiles + kScanChunk - 1) / kScanChunk;
-    const uint64_t bit_words = ntiles * TR / 64, scan_words = 4 + 3 * ntiles + 3 * nchunks;
+    const uint64_t bit_words = ntiles * TR / 64, scan_words = 3 * ntiles + 3 * nchunks;
     if (!(scr = (uint64_t *)pool->alloc((bit_words + scan_words) * 8, s, err_slot()))) return done(kOtherForm);
     f.rbits = (uint32_t *)scr;
     p.T = in->d;
     p.c = (uint32_t)in->cols;
     p.R = R;
-    p.totals = scr + bit_words;
-    p.tile_sum = p.totals + 4;
+    p.tile_sum = scr + bit_words;
     p.tile_nz = p.tile_sum + ntiles;
     p.tile_ex = p.tile_nz + ntiles;
     p.chunk_sum = p.tile_ex + ntiles;
@@ -1598,6 +1597,7 @@ int wkg_ctx::step_filter_lists(int mode, const wkg_table *in, int pid, int dir, 
     auto zero = [&](void *a, uint64_t n) {
       k_zero_u64<<<(unsigned)std::min<uint64_t>((n + kBlock - 1) / kBlock, 65535), kBlock, 0, s>>>((uint64_t *)a, n);
     };
+    p.totals = (uint64_t *)f.ctr + kListBits;  // (so one read-back brings all counts)
     zero(f.ctr, kListCtrs + kListQueues * kListPad);  // (the queues' counters follow)
     zero(f.rbits, bit_words);
     pass(std::true_type{});
@@ -1612,7 +1612,7 @@ int wkg_ctx::step_filter_lists(int mode, const wkg_table *in, int pid, int dir, 
     if ((rc = read_words((const uint64_t *)f.ctr, kListCtrs, s, c))) return done(rc);
   }
   if (c[kListLost]) return done(kOtherForm);
-  const uint64_t kept = c[kListKept];
+  const uint64_t kept = bits ? c[kListBits] : c[kListKept];
   wkg_table *t = nullptr;
   if ((rc = new_table(kept, in->cols, s, &t))) return done(rc);
   if (kept) {

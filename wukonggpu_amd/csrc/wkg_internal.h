@@ -289,6 +289,9 @@ struct wkg_ctx {
                        uint64_t *expanded);
   int step_filter_groups(int mode, const wkg_table *in, int pid, int dir, int ec, int64_t cval, hipStream_t s,
                          wkg_table **out, uint64_t *expanded);
+  // Bytes of a lookup for the profile: a tag word, and the slot of a key that
+  // is there; without tag words the whole bucket either way.
+  double key_bytes(double keys, double present) const { return d_tags ? 8 * keys + 16 * present : 128 * keys; }
   // residency
   int set_image_metas(uint64_t nslots, uint64_t nedges, const wkg_pred_meta_abi *m_in, int nmetas);
   int finish_resident(uint32_t flags, hipStream_t s, uint64_t tag_bytes = ~uint64_t(0));
