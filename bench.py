@@ -117,7 +117,7 @@ def _expand_roofline(dev, n_queries, traffic_file, extra=None):
             t = json.load(f)
         traffic, src = t["hbm_bytes_per_launch"], t["source"]
     r = {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
-         "frac": achieved / HBM_PEAK_GBS, "traffic": traffic, "kernel": "expand (k_expand)",
+         "frac": achieved / HBM_PEAK_GBS, "traffic": traffic, "kernel": "expand (k_expand_hits and k_expand)",
          "launches_per_query": n_exp / max(n_queries, 1), "alg_bytes_per_launch": b_exp / max(n_exp, 1),
          "avg_launch_ms": ms_exp / max(n_exp, 1), "traffic_source": src}
     if extra:
@@ -169,6 +169,8 @@ def main():
                     help="run only the config-2/3 graph under a graph budget (framed residency)")
     ap.add_argument("--framed-budget", type=int, default=1 << 30,
                     help="graph budget of the framed-residency measurement, bytes (0: skip it)")
+    ap.add_argument("--detail", default="",
+                    help="write the whole result (distributions, kernel times, notes, every digit) to this file")
     ap.add_argument("--shape", default="",
                     help="with --mix-only: the executor shape as key=value pairs (probe_wg_per_cu=3,...) "
                          "instead of autotuning")
@@ -186,18 +188,18 @@ def main():
     if args.exchange_only:
         from wukonggpu_amd import Device
         dev = Device(0)
-        print(json.dumps({"table_exchange": table_exchange(dev, args.seed)}), flush=True)
+        _emit({"table_exchange": table_exchange(dev, args.seed)}, args.detail)
         dev.close()
         return
     if args.cycle_only:
-        print(json.dumps(run_config5(args, quick=True)), flush=True)
+        _emit(run_config5(args, quick=True), args.detail)
         return
     if profiler_pass:
-        print(json.dumps(run_config23(args)), flush=True)
+        _emit(run_config23(args), args.detail)
         return
     if args.config != "all":
         fn = {"1": run_config1, "2": run_config23, "4": run_config4, "5": run_config5}[args.config]
-        print(json.dumps(fn(args)), flush=True)
+        _emit(fn(args), args.detail)
         return
 
     line = run_config5(args)
@@ -212,7 +214,40 @@ def main():
         extra[name]["leg_s"] = time.time() - t
     line.update(extra)
     line["bench_wall_s"] = time.time() - T_START
-    print(json.dumps(line), flush=True)
+    _emit(line, args.detail)
+
+
+DETAIL_KEYS = {"cdf_us", "cdf_rates", "kernels_per_query", "kernels_per_heavy_query", "per_kernel_ms", "note", "what",
+               "served_knee_lanes_only", "served_lanes_only", "rows_per_s", "frac_of_peak", "scatter_ms",
+               "issued", "issued_heavy", "stream_exhausted", "traffic_source", "ms_per_query_with_kernel_events",
+               "row_half_splits_per_query", "heavy_tuning", "tuning", "cpu_model", "nproc"}
+SERVED_KEYS = {"offered_qps", "achieved_qps", "p50_ms", "p99_ms", "light_p99_ms", "heavy_p99_ms"}
+
+
+def _compact(x):
+    """The printed form of a result: four significant digits, without latency
+    distributions, per-kernel times, notes and the minor fields of a served
+    rate (the whole line then fits the 16 kB that callers keep)."""
+    if isinstance(x, dict):
+        served = "offered_qps" in x
+        return {k: _compact(v) for k, v in x.items() if k not in DETAIL_KEYS and (not served or k in SERVED_KEYS)}
+    if isinstance(x, (list, tuple)):
+        return [_compact(v) for v in x]
+    if isinstance(x, float):
+        return float(f"{x:.4g}")
+    return x
+
+
+def _emit(obj, detail=""):
+    """Prints the result as one JSON line; `detail` names a file for all of it."""
+    if detail:
+        with open(detail, "w") as f:
+            json.dump(obj, f, indent=1)
+    line = _compact(obj)
+    for k in ("value", "ms_per_step"):  # the headline in full
+        if k in obj:
+            line[k] = obj[k]
+    print(json.dumps(line, separators=(",", ":")), flush=True)
 
 
 def _line(value, unit, steps, warmup, ms, config, extra, higher=True, dtype="u32"):
@@ -436,7 +471,7 @@ def run_config23(args, nested=False):
         return obj
 
     if args.probe_only:
-        return done({"probe_random_keys": random_key_probe(dev, w, args.seed, HBM_PEAK_GBS * 1e9 / 128)})
+        return done({"probe_random_keys": random_key_probe(dev, w, args.seed)})
     if args.served_heavy_only:
         sq, sflags = workloads.served_mix(P, type_ids, w.info["t0"], args.served_n, args.seed + 11)
         hq = [q for q, f in zip(sq, sflags) if f]
@@ -515,30 +550,28 @@ def run_config23(args, nested=False):
     log(f"heavy query: {r.table.shape[0]} result rows, {edges} expanded edges, "
         f"{elapsed / args.steps * 1e3:.2f} ms/query, {value / 1e9:.2f} G expanded edges/s; k_expand "
         f"{roof['achieved']:.0f} GB/s = {roof['frac']:.2f} of peak")
-    line_peak = HBM_PEAK_GBS * 1e9 / 128
     probe_roofline = {
-        "bound": "random-access", "peak": line_peak, "unit": "128-byte bucket lines/s",
+        "bound": "hbm", "peak": HBM_PEAK_GBS, "unit": "GB/s",
         "kernel": "probe (k_probe, known_to_unknown steps)", "measured_random_lines_4GiB": lines_ps,
         "heavy_query": {
             "keys_probed_per_query": probe_keys / args.steps, "rows_per_query": probe_rows / args.steps,
             "keys_per_s": probe_keys / (ms_pr * 1e-3) if ms_pr > 0 else 0.0,
             "rows_per_s": probe_rows / (ms_pr * 1e-3) if ms_pr > 0 else 0.0,
             "alg_GBps": alg_pr / (ms_pr * 1e-3) / 1e9 if ms_pr > 0 else 0.0,
-            "note": "runs of equal keys share one bucket walk, so this probe is bound by reading its "
-                    "input table (4 R c bytes), not by bucket lines; alg_GBps counts 4 R c + 128 per key "
-                    "probed + 16 per row with edges",
+            "note": "runs of equal keys are looked up once, so this probe is bound by reading its input "
+                    "table (4 R c bytes), not by lookups; alg_GBps counts 4 R c + 8 per key probed (tag word) "
+                    "+ 16 per key that is there (slot) + 16 per row with edges",
         },
     }
     if args.heavy_only:
         return done(_line(value, "expanded edges/s", args.steps, args.warmup, elapsed / args.steps * 1e3,
                           {"workload": "config-2 heavy query"}, {"roofline": roof}))
-    rk = random_key_probe(dev, w, args.seed, line_peak)
-    rk["frac_of_random_lines_4GiB"] = rk["achieved"] / lines_ps
-    probe_roofline.update({"achieved": rk["achieved"], "frac": rk["frac_of_peak"], "random_keys": rk})
-    log(f"probe on random keys: {rk['keys_probed'] / 1e6:.1f} M keys in {rk['ms_per_launch']:.2f} ms = "
-        f"{rk['achieved'] / 1e9:.2f} G keys/s = {rk['frac_of_peak']:.2f} of HBM peak / 128 B; random lines "
-        f"over 4 GiB {lines_ps / 1e9:.1f} G/s, over the {rk['segment_bytes'] / 2**20:.0f} MiB segment "
-        f"{rk['random_lines_same_working_set'] / 1e9:.1f} G/s ({rk['frac_of_random_lines_same_working_set']:.2f})")
+    rk = random_key_probe(dev, w, args.seed)
+    probe_roofline.update({"achieved": rk["alg_GBps"], "frac": rk["frac_of_peak"], "random_keys": rk})
+    log(f"probe on random keys: {rk['keys_probed'] / 1e6:.1f} M keys ({rk['present'] / rk['rows']:.2f} there) in "
+        f"{rk['ms_per_launch']:.2f} ms = {rk['keys_per_s'] / 1e9:.2f} G keys/s, {rk['alg_GBps']:.0f} GB/s = "
+        f"{rk['frac_of_peak']:.2f} of HBM peak; random lines over its {rk['segment_bytes'] / 2**20:.0f} MiB of "
+        f"buckets {rk['random_lines_segment'] / 1e9:.1f} G/s")
 
     # ---- the heavy query through the device-resident executor ---------------------------
     eng.configure(max_queries=1024, max_patterns=8, arena_bytes=32 << 30)
@@ -1024,24 +1057,30 @@ def compare_device_build(w, Device, main_load=0.75, host_gs=None, host_s=None):
             "device_triples_per_s": n / dev_s, "image_equal_host": same}
 
 
-def random_key_probe(dev, w, seed, line_peak):
+def random_key_probe(dev, w, seed):
     """One known_to_unknown step (predicate 2 OUT) over 64M rows of uniformly
-    random vertex ids, timed with HIP events over 3 launches: keys probed per
-    second against HBM peak / 128 B and against random 128-byte line reads
-    over a buffer the size of the predicate's bucket segment."""
+    random vertex ids, timed with HIP events over 3 launches: the bytes it
+    cannot do without (its rows, a tag word per key, the slots of the keys
+    that are there and their hits) against the HBM peak. Beside them the keys
+    per second and the rate of random 128-byte line reads over a buffer the
+    size of the bucket segment: what a lookup through the buckets would be
+    held to (a tag word is 8 bytes, and they stay in the L2s)."""
     import numpy as np
     rng_p = np.random.default_rng(seed + 7)
     n_rand = 1 << 26
-    col = (1 << 17) + rng_p.integers(0, w.info["entities"], size=(n_rand, 1), dtype=np.int64)
-    t_rand = dev.table(col.astype(np.int32))
-    del col
+    ids = rng_p.integers(0, w.info["entities"], size=(n_rand, 1), dtype=np.int64)
+    there = np.zeros(w.info["entities"], dtype=bool)
+    there[w.gstore.get_edges(0, 2, 0).astype(np.int64) - (1 << 17)] = True
+    present = int(there[ids].sum())
+    t_rand = dev.table(((1 << 17) + ids).astype(np.int32))
+    del ids
     out_t, _ = dev.k2u(t_rand, 0, 2, 1)  # warm
     out_t.free()
     dev.profile(True)
     for _ in range(3):
         out_t, _ = dev.k2u(t_rand, 0, 2, 1)
         out_t.free()
-    n_r, ms_r, _ = dev.profile_read("probe")
+    n_r, ms_r, b_r = dev.profile_read("probe")
     keys_r = dev.profile_read("probe_keys")[2]
     dev.profile(False)
     t_rand.free()
@@ -1049,10 +1088,10 @@ def random_key_probe(dev, w, seed, line_peak):
     m2 = w.gstore.metas()[2]  # partition_sz, main [start, end), indirect [start, end), ...
     seg_bytes = int(m2[0] + (m2[4] - m2[3])) * 128
     seg_lines = dev.random_access_rate(max(seg_bytes, 1 << 20), 10)
-    return {"rows": n_rand, "keys_probed": keys_r / 3, "ms_per_launch": ms_r / max(n_r, 1),
-            "achieved": rand_rate, "frac_of_peak": rand_rate / line_peak,
-            "segment_bytes": seg_bytes, "random_lines_same_working_set": seg_lines,
-            "frac_of_random_lines_same_working_set": rand_rate / seg_lines,
+    gbs = b_r / (ms_r * 1e-3) / 1e9
+    return {"rows": n_rand, "keys_probed": keys_r / 3, "present": present, "ms_per_launch": ms_r / max(n_r, 1),
+            "alg_GBps": gbs, "frac_of_peak": gbs / HBM_PEAK_GBS, "keys_per_s": rand_rate,
+            "segment_bytes": seg_bytes, "tag_bytes": int(m2[0]) * 8, "random_lines_segment": seg_lines,
             "workload": "known_to_unknown over 64M uniformly random vertex ids, predicate 2 OUT"}
 
 
