@@ -104,18 +104,23 @@ STEP_KERNELS = ("probe", "probe_filter", "fanout_filter", "scan_tiles", "finaliz
                 "probe_one", "copy_list", "follow", "lineage")
 
 
+def _traffic(name):
+    """(HBM bytes per launch, source) of a committed rocprofv3 summary in profiles/, or (None, None)."""
+    path = os.path.join(ROOT, "profiles", name)
+    if not os.path.exists(path):
+        return None, None
+    with open(path) as f:
+        t = json.load(f)
+    return t["hbm_bytes_per_launch"], t["source"]
+
+
 def _expand_roofline(dev, n_queries, traffic_file, extra=None):
-    """HBM roofline of k_expand from HIP events over the profiled queries:
+    """HBM roofline of the expands from HIP events over the profiled queries:
     algorithmic bytes per launch / average launch time; traffic (PMC bytes
     per launch) from the committed rocprofv3 summary when there is one."""
     n_exp, ms_exp, b_exp = dev.profile_read("expand")
     achieved = b_exp / (ms_exp * 1e-3) / 1e9 if ms_exp > 0 else 0.0
-    traffic, src = None, None
-    tp = os.path.join(ROOT, "profiles", traffic_file)
-    if os.path.exists(tp):
-        with open(tp) as f:
-            t = json.load(f)
-        traffic, src = t["hbm_bytes_per_launch"], t["source"]
+    traffic, src = _traffic(traffic_file)
     r = {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
          "frac": achieved / HBM_PEAK_GBS, "traffic": traffic, "kernel": "expand (k_expand_hits and k_expand)",
          "launches_per_query": n_exp / max(n_queries, 1), "alg_bytes_per_launch": b_exp / max(n_exp, 1),
@@ -324,7 +329,7 @@ def run_config5(args, quick=False, nested=False):
     if msf > 0:
         ach = bf / (msf * 1e-3) / 1e9
         pairs = r.expanded  # (the fan-out's rows dominate the work count)
-        traffic, tsrc = None, None
+        traffic, tsrc = _traffic("fanout_cycle_2b.traffic.json")
         roof = {"bound": "hbm", "achieved": ach, "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": ach / HBM_PEAK_GBS,
                 "traffic": traffic, "traffic_source": tsrc,
                 "kernel": "fanout_filter (k_list_filter and k_list_long)",
