@@ -123,10 +123,10 @@ __device__ __forceinline__ uint32_t edge_at(const GraphView &g, uint64_t edge_st
   return g.edges[g.eframes[eframe_base + (local >> g.eshift)] + (local & mask)];
 }
 
-// Per-wave LDS scratch of wave_probe.
+// Per-wave LDS scratch of a probe.
 struct WaveProbeLds {
-  uint4 kb[kWave];   // pending bucket walks: (key lo, key hi, bucket, leader index)
-  uint2 res[kWave];  // run leaders' (degree, offset)
+  uint4 kb[kWave];   // pending bucket walks: (key lo, key hi, bucket, id: the leader's lane or row)
+  uint2 res[kWave];  // per lane: a walked leader's (degree, offset)
 };
 
 // Cluster-chaining probe of 64 consecutive rows, one per lane, all under one
@@ -145,8 +145,8 @@ struct WaveProbeLds {
 //  walk (without tags: every leader; with them: keys in chains and tag
 //  collisions, about one in fifteen) park (key, bucket, lane) in LDS as
 //  pending walks, taken 8 lanes per walk: each lane of a group loads one
-//  16-byte slot of the bucket (one coalesced 128-byte read, up to 8 bucket
-//  reads in flight per lane). The lane whose slot holds the key writes the
+//  16-byte slot of the bucket (one coalesced 128-byte read; 8 bucket reads in
+//  flight per lane without tags, 2 with them). The lane whose slot holds the key writes the
 //  leader's (degree, offset) to LDS; in a group with no match, lane 7 (the
 //  link slot) either records a miss or appends the walk, moved to the linked
 //  bucket, to the next hop's pending list. At last every lane takes its run
@@ -162,7 +162,8 @@ struct WaveProbeLds {
 // through the buckets, every key misses, present or not. 24M random keys, 36%
 // of them present: 512 us through the buckets (47 G keys/s), 300 us through
 // the tags (80 G keys/s); the executor's 512-query mix, mostly absent keys,
-// 730 -> 661 us a batch. Nontemporal slot reads leave the tag words their
+// 730 -> 661 us a batch. Where most keys are present the tag words are lines
+// on top of the slots': 12M rows, 74% of them present, 370 -> 404 us. Nontemporal slot reads leave the tag words their
 // place in the L2s (16.4M -> 13.2M misses) but measured slower (604 against
 // 517 us a step), as did nontemporal table reads and hit lists.
 struct ProbeCarry {
@@ -191,11 +192,6 @@ __device__ __forceinline__ uint2 gload(const uint2 *p) {
 }
 __device__ __forceinline__ uint4 gload(const uint4 *p) {
   const gu32x4 v = *(const WKG_GLOBAL gu32x4 *)p;
-  return make_uint4(v.x, v.y, v.z, v.w);
-}
-// A read that is not kept in the caches ahead of others (nontemporal).
-__device__ __forceinline__ uint4 gload_once(const uint4 *p) {
-  const gu32x4 v = __builtin_nontemporal_load((const WKG_GLOBAL gu32x4 *)p);
   return make_uint4(v.x, v.y, v.z, v.w);
 }
 __device__ __forceinline__ void gstore(uint2 *p, uint2 v) { *(WKG_GLOBAL gu32x2 *)p = gu32x2{v.x, v.y}; }

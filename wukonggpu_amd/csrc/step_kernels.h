@@ -111,7 +111,7 @@ __device__ __forceinline__ void group_scan(const GraphView &g, uint64_t estart, 
 // which this replaced, ran a group's 8 rows one after another (8
 // chains in flight, 8 times as long): a known_to_known step over
 // 3M rows, half of them walked edges, 401 -> 210 us; known_to_const over 12M
-// rows of one-entry lists 443 -> 370 us.
+// rows of one-entry lists 443 -> 370 us (before tag words: 404 with them).
 // Unsorted lists: the 8 lanes of a group scan the group's 8 lists in turn.
 template <bool SORTED, bool FRAMED>
 __device__ __forceinline__ void rows_member(const GraphView &g, uint64_t estart, uint64_t efb, uint32_t off,
@@ -288,7 +288,7 @@ __device__ __forceinline__ void probe_tile(const GraphView &g, const StepParams 
   }
   if (lane == 0) s_probed[wave] = probed;
   __syncthreads();
-  // thread t owns the tile's rows 8t .. 8t+7
+  // thread t owns the tile's rows [t * kRowsPerThread, (t + 1) * kRowsPerThread)
   uint64_t sum = 0, ex = 0;
   uint32_t nz = 0;
 #pragma unroll

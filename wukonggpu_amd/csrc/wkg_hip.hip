@@ -1651,6 +1651,10 @@ int wkg_ctx::step_filter_lists(int mode, const wkg_table *in, int pid, int dir, 
   return done(WKG_OK);
 }
 
+// Inputs of at most this many rows: too few for a fan-out to be fused with its
+// filter, or for a filter to be decided from lineage.
+constexpr uint64_t kTinyRows = 512;
+
 // known_to_unknown on column sc of `in` followed by a filter (fmode) whose
 // start column is the new column: when the filter can run on the fan-out's
 // lineage (step_filter_fanout), the fan-out is never written -- a table
@@ -1664,7 +1668,7 @@ int wkg_ctx::step_k2u_filter(const wkg_table *in, int sc, int pid, int dir, int 
                              uint64_t *ex_f) {
   *fused = 0;
   *ex_f = 0;
-  const bool fits = lineage && !framed && in && in->rows > 512 && in->cols >= 1 && sc >= 0 && sc < in->cols &&
+  const bool fits = lineage && !framed && in && in->rows > kTinyRows && in->cols >= 1 && sc >= 0 && sc < in->cols &&
                     !star_arm(in, sc) && in->cols + 1 <= kBlock &&
                     in->rows < (1ull << 32) && (in->owned || in->slice_of);
   if (!fits || check_pattern(fpid, fdir) != WKG_OK || (fmode == kModeK2K && (ec < 0 || ec >= in->cols)))
@@ -1744,7 +1748,7 @@ int wkg_ctx::step_known(int mode, const wkg_table *in, int sc, int pid, int dir,
   }
   const bool star = mode == kModeK2U && star_arm(in, sc);
   if (star && R >= kLineageRows) return step_k2u_lineage(in, sc, pid, dir, s, out, expanded);
-  const bool tiny = small_steps && R <= 512;  // (too few rows for the filters below to pay)
+  const bool tiny = small_steps && R <= kTinyRows;
   if (mode != kModeK2U && !tiny && lineage && !framed && in->glin_parent && sc == c - 1 &&
       (mode == kModeK2C || ec < in->glin_parent->cols) && R >= group_filter_rows && R >= 4 * in->glin_dtot)
     return step_filter_groups(mode, in, pid, dir, ec, cval, s, out, expanded);
