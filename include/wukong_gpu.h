@@ -127,7 +127,8 @@ int wkg_build_graph(wkg_ctx *ctx, const uint32_t *s, const uint32_t *p, const ui
 int wkg_graph_shape(const wkg_ctx *ctx, uint64_t *num_slots, uint64_t *num_edges, int *num_metas);
 int wkg_graph_download(wkg_ctx *ctx, uint64_t *slots, uint32_t *edges, wkg_pred_meta_abi *metas);
 
-/* Graph residency statistics: bytes resident, frame loads, evictions. */
+/* Graph residency statistics: bytes resident (the tag words of a resident
+ * image among them), frame loads, evictions. */
 int wkg_graph_stats(const wkg_ctx *ctx, uint64_t *resident_bytes,
                     uint64_t *segment_loads, uint64_t *segment_evictions);
 /* 1 when the loaded graph is framed (segments loaded on demand under a graph
@@ -175,8 +176,9 @@ int wkg_set_probe_tile_rows(wkg_ctx *ctx, int rows);
  * the same, row for row. On by default; 0 turns it off. No counterpart in the
  * reference, which probes every row (core/gpu_hash.cu:145-316). */
 int wkg_set_lineage(wkg_ctx *ctx, int on);
-/* With lineage on, the output of such a once-per-input-row step also keeps
- * its groups (an input row's list, joined to each of that row's children).
+/* With lineage on, the output of such a next arm (below 2^19 input rows: if
+ * it has at least `rows` rows) also keeps its groups (an input row's list,
+ * joined to each of that row's children).
  * A known_to_known / known_to_const step from that output's last column
  * (end column, if any, one of the input's) of at least `rows` rows (default
  * 2^22; 0: any size), and at least 4 per list entry of its groups, decides
@@ -186,12 +188,13 @@ int wkg_set_lineage(wkg_ctx *ctx, int on);
 int wkg_set_group_filter_rows(wkg_ctx *ctx, uint64_t rows);
 /* Such a filter over long lists shared by many parents (sorted lists) hashes
  * the targets of each list's parents and looks the neighbours of every
- * distinct list entry up among them; with more kept rows than that lists
- * (2^15), or unsorted lists, it runs a block of a list's entries against 64
- * of its parents per workgroup and lists the kept rows (at most kept_cap of
- * them, 0: 2^22; with more it reruns with one parent per workgroup). On by
- * default; 0 always runs one parent per workgroup. The output and work count
- * are the same either way. */
+ * distinct list entry up among them, listing the kept rows (at most 2^15, or
+ * kept_cap; with more it reruns with a bit per row). With unsorted lists, or
+ * more parents than 4096 + rows / 8192, it runs a block of a list's entries
+ * against 64 of its parents per workgroup and lists the kept rows (at most
+ * kept_cap of them, 0: 2^22; with more it reruns with one parent per
+ * workgroup). On by default; 0 always runs one parent per workgroup. The
+ * output and work count are the same either way. */
 int wkg_set_fanout_blocks(wkg_ctx *ctx, int on, uint64_t kept_cap);
 /* The calling thread's per-step calls on ctx (stream NULL) get a stream and
  * a pinned read-back block of their own until _end, so several threads can
@@ -203,7 +206,8 @@ int wkg_thread_context_end(wkg_ctx *ctx);
 /* A known-start step over at most 2^20 input rows (2048 probe tiles) runs as
  * two launches, the probe and one that scans, compacts and expands, while
  * its output fits a table guessed for it (twice the input's rows, at most 8 MB
- * and a 256th of the table budget), instead of three to five; its output is
+ * and a 256th of the table budget; tables hold at most another 256th of it
+ * beyond their rows, which does not count), instead of three to five; its output is
  * the same, row for row. On by default; 0 turns it off. A launch-count
  * optimisation with no counterpart in the reference. */
 int wkg_set_small_steps(wkg_ctx *ctx, int on);

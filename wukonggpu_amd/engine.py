@@ -159,8 +159,9 @@ class Device:
         self._check(N.hip_lib().wkg_thread_context_end(self._h))
 
     def set_fanout_blocks(self, on, kept_cap=0):
-        """Long shared lists: 64 parents per workgroup with a kept-row list of
-        kept_cap rows (0: 2^22); off: one parent per workgroup."""
+        """Long shared lists: through their parents' targets, or 64 parents per
+        workgroup, with a kept-row list of at most kept_cap rows (0: the
+        default); off: one parent per workgroup."""
         self._check(N.hip_lib().wkg_set_fanout_blocks(self._h, 1 if on else 0, int(kept_cap)))
 
     def set_group_filter_rows(self, rows):
