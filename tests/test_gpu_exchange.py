@@ -87,9 +87,11 @@ def test_split_many_tiles_property(dev_small):
     assert np.array_equal(got[np.argsort(got[:, 1])], t)
 
 
-@pytest.mark.parametrize("rows", [1, 1023, 1025, 8192 * 1024, 8192 * 1024 + 1, 5 * 2048 * 1024 - 1, 5 * 2048 * 1024 + 1])
+@pytest.mark.parametrize("rows", [1, 1023, 1025, 512 * 1024, 512 * 1024 + 1, 8192 * 1024,
+                                  8192 * 1024 + 1, 5 * 2048 * 1024 - 1, 5 * 2048 * 1024 + 1])
 def test_split_scan_edges(dev_small, rows):
-    # slabs of 1024 rows: a part's counts in one chunk up to 8192 of them, then in chunks of 2048
+    # slabs of 1024 rows: a part's counts in one wave up to 512 of them, one workgroup up to 8192, then in
+    # chunks of 2048
     t = np.stack([np.random.default_rng(rows).integers(1, 1 << 30, rows, dtype=np.int32),
                   np.arange(rows, dtype=np.int32)], axis=1)
     d = dev_small.table(t)

@@ -169,21 +169,24 @@ __global__ __launch_bounds__(kSplitBlock) void k_split_count(SplitArgs a) {
 // workgroup walking a part 8192 counts at a time took 38 and 147 and the
 // library's scan of the whole array 14 and 20.
 constexpr int kScanBlock = 1024;
+// Parts of at most 512 slabs are one wave's each (a thousand workgroups of
+// 1024 threads for a count or two each: 10 rows into 1000 parts 57 us, so 47,
+// with the library's scan 55).
 constexpr uint64_t kScanWhole = 8 * kScanBlock, kScanChunk = 2 * kScanBlock;
-template <int K>
-__global__ __launch_bounds__(kScanBlock) void k_split_scan(SplitArgs a, uint64_t nchunks, const uint64_t *sums) {
-  __shared__ uint64_t s_tmp[2 * kScanBlock / kWave];
+template <int K, int BS = kScanBlock>
+__global__ __launch_bounds__(BS) void k_split_scan(SplitArgs a, uint64_t nchunks, const uint64_t *sums) {
+  __shared__ uint64_t s_tmp[2 * BS / kWave];
   const uint64_t p = blockIdx.x / nchunks, chunk = blockIdx.x % nchunks;
   const uint32_t *cnt = a.cnt + p * a.nslabs;
   uint64_t *base = a.base + p * a.nslabs;
-  const uint64_t lo = (chunk * kScanBlock + threadIdx.x) * K;
+  const uint64_t lo = (chunk * BS + threadIdx.x) * K;
   uint64_t c[K], v[2] = {0, 0}, tot[2];  // this chunk's counts; the chunks before it
 #pragma unroll
   for (int k = 0; k < K; k++) c[k] = lo + k < a.nslabs ? cnt[lo + k] : 0;
-  for (uint64_t i = threadIdx.x; i < chunk; i += kScanBlock) v[1] += sums[p * nchunks + i];
+  for (uint64_t i = threadIdx.x; i < chunk; i += BS) v[1] += sums[p * nchunks + i];
 #pragma unroll
   for (int k = 0; k < K; k++) v[0] += c[k];
-  block_excl_scan_n<2, kScanBlock>(v, s_tmp, tot);
+  block_excl_scan_n<2, BS>(v, s_tmp, tot);
   uint64_t run = tot[1] + v[0];
 #pragma unroll
   for (int k = 0; k < K; k++)
@@ -542,7 +545,9 @@ int wkg_table_split(wkg_ctx *ctx, const wkg_table *in, int col, int nparts, void
       ProfScope ps(ctx, s, "split_scan", 12.0 * (double)ncnt);
       uint64_t *sums = (uint64_t *)(scr + b_cnt + b_base + b_total);
       const unsigned grid = (unsigned)(nchunks * (uint64_t)nparts);
-      if (nchunks == 1) {
+      if (a.nslabs <= 8 * (uint64_t)kWave) {
+        k_split_scan<8, kWave><<<grid, kWave, 0, s>>>(a, 1, nullptr);
+      } else if (nchunks == 1) {
         k_split_scan<8><<<grid, kScanBlock, 0, s>>>(a, 1, nullptr);
       } else {
         k_split_sums<<<grid, kScanBlock, 0, s>>>(a, nchunks, sums);
