@@ -167,11 +167,10 @@ __global__ __launch_bounds__(kSplitBlock) void k_split_count(SplitArgs a) {
 // 1M rows in 8 parts, 12 at 8M. Longer parts go in chunks of 2048 (K = 2),
 // two launches: 11 us at 33.5M rows in 8 parts, 15 at 134M, where one
 // workgroup walking a part 8192 counts at a time took 38 and 147 and the
-// library's scan of the whole array 14 and 20.
+// library's scan of the whole array 14 and 20. Parts of at most 512 slabs are
+// one wave's each (10 rows into 1000 parts: 57 us a call with workgroups of 1024
+// threads for a count or two each, 47 so, 55 with the library's scan).
 constexpr int kScanBlock = 1024;
-// Parts of at most 512 slabs are one wave's each (a thousand workgroups of
-// 1024 threads for a count or two each: 10 rows into 1000 parts 57 us, so 47,
-// with the library's scan 55).
 constexpr uint64_t kScanWhole = 8 * kScanBlock, kScanChunk = 2 * kScanBlock;
 template <int K, int BS = kScanBlock>
 __global__ __launch_bounds__(BS) void k_split_scan(SplitArgs a, uint64_t nchunks, const uint64_t *sums) {
