@@ -2456,9 +2456,13 @@ __device__ __forceinline__ bool list_keep(const ListFilter &f, uint32_t n, uint3
       if (shfl32(before, src + step) <= t) src += step;
     const uint32_t q = shfl32(first, src) + (t - shfl32(before, src)), kj = shfl32(j, src), ke = shfl32(e, src);
     if (t < all) {
-      const uint32_t p = f.order[q], row = (uint32_t)(f.excl[p] + kj);
-      if (BITS) atomicOr(&f.rbits[row >> 5], 1u << (row & 31));
-      else f.kept[base + t] = make_uint4(row, p, ke, 0u);
+      const uint32_t p = f.order[q];
+      const uint64_t row = f.excl[p] + kj;
+      if constexpr (BITS) {
+        if (row < f.R) atomicOr(&f.rbits[row >> 5], 1u << (row & 31));  // (always: lists at one offset are alike)
+      } else {
+        f.kept[base + t] = make_uint4((uint32_t)row, p, ke, 0u);
+      }
     }
   }
   return true;
